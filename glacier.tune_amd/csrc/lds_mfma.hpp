@@ -17,11 +17,14 @@ namespace glacier {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // Slot of piece p of row r: p ^ lds_sw(r) (16 pieces per row at D = 128, 8 at
-// D = 64, where two rows share one 256-byte line of the 64 banks).
+// D = 64 and 4 at D = 32, where two and four rows share one 256-byte line of
+// the 64 banks).
 template <int D>
 __device__ inline int lds_sw(int r) {
   if constexpr (D == 128)
     return ((r & 3) << 2) | ((r >> 2) & 3);
+  else if constexpr (D == 32)
+    return (r >> 2) & 3;
   else
     return (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
 }

@@ -1,603 +1,427 @@
-// proj_gemm.hip -- the projection's narrow base products on the matrix
-// cores (bf16 tensors): the k and v projections of a Qwen-style block have
-// 512 outputs against 3584 inputs, a shape a library GEMM covers with a few
-// dozen workgroups on a 256-CU chip.  Here every narrow projection of a call
-// goes through one launch per direction, tiled finely enough to fill the
-// chip:
-//   forward   Yf_p[s] = X W_p^T over the s-th slice of the inputs   (NT)
-//             64 outputs x 64 tokens per workgroup, the reduction split in
-//             S slices; lowrank_out adds the S partials in slice order
-//   backward  dXf2 = sum_p dY_p W_p over the narrow projections     (NN)
-//             64 inputs x 64 tokens per workgroup, the projections'
-//             reductions one after another; lowrank_out adds dXf2 to the
-//             library GEMM's dXf
+// proj_gemm.hip -- the projections' base products on the matrix cores, with
+// the LoRA delta, the bias and the output conversion in the same pass.
+//
 // GpuLoraEngine.ForwardQKV (GpuLoraEngine.Forward.cs:205-245) and
 // LoraAdapter.Backward (LoraAdapter.cs:190-247) compute the same products.
-//
-// Both kernels compute the transposed tile C^T = (feature rows) x (token
-// columns) with v_mfma_f32_16x16x32_bf16, so that a lane's four accumulators
-// are four consecutive outputs of one token: one 16-byte store.  Stages of 64
-// reduction elements go global -> registers -> LDS (rows of 144 bytes) with
-// four stages' loads in flight while one is multiplied (a stage is only 8
-// MFMAs per wave, far shorter than a load's round trip); one workgroup
-// barrier per stage, the LDS double-buffered.  Loads go through buffer resources whose range
-// ends at the last valid row, so rows past T or past a projection's outputs
-// read as zero.  Fixed reduction order everywhere: bitwise repeatable.
 #include "attn_common.hpp"
 #include "lds_mfma.hpp"
 #include "proj_launch.hpp"
+#include "split3.hpp"
 
 namespace glacier {
 namespace {
 
-constexpr int kGT = 64;       // tile rows (features) and columns (tokens)
-constexpr int kGK = 64;       // reduction elements per stage
-constexpr int kGS = kGK + 8;  // LDS row stride, elements (144 bytes)
-constexpr int kGThreads = 256;
-constexpr int kGTile = kGT * kGS;  // elements of one LDS operand tile
-constexpr int kGPf = 4;            // stages in flight (registers) ahead of the one multiplied
-
-// A row-major bf16 matrix seen from row `row0`: rows [row0, row0 + nrows)
-// readable, anything past them zero.
-struct RowSrc {
-  __amdgpu_buffer_rsrc_t rs;
-  int rowb;  // row stride in bytes
-};
-
-__device__ inline RowSrc row_src(const bf16* m, long ld, long row0, int nrows, int row_bytes) {
-  const int rowb = static_cast<int>(ld * (long)sizeof(bf16));
-  const int nrec = nrows <= 0 ? 0 : (nrows - 1) * rowb + row_bytes;
-  const bf16* base = m + row0 * ld;
-  const unsigned long long a = reinterpret_cast<unsigned long long>(base);
-  const unsigned long long au =
-      (static_cast<unsigned long long>(__builtin_amdgcn_readfirstlane(static_cast<int>(a >> 32))) << 32) |
-      static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(a & 0xffffffffu)));
-  RowSrc r;
-  r.rs = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(au), (short)0,
-                                           __builtin_amdgcn_readfirstlane(nrec), kBufferWord3);
-  r.rowb = __builtin_amdgcn_readfirstlane(rowb);
-  return r;
-}
-
-// One stage of one operand: 64 rows x 64 elements from column col0, two
-// 16-byte pieces per thread (piece tid + 256 i: row / 8, 8-element column).
-struct Stage {
-  i32x4 w[2];
-  __device__ inline void load(const RowSrc& s, int col0, int tid) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int idx = tid + kGThreads * i;
-      const int off = (idx >> 3) * s.rowb + (col0 + 8 * (idx & 7)) * (int)sizeof(bf16);
-      w[i] = __builtin_amdgcn_raw_buffer_load_b128(s.rs, off, 0, 0);
-    }
-  }
-  __device__ inline void store(bf16* tile, int tid) const {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int idx = tid + kGThreads * i;
-      *reinterpret_cast<i32x4*>(tile + (idx >> 3) * kGS + 8 * (idx & 7)) = w[i];
-    }
-  }
-};
-
 // The hardware deals workgroup ids to the 8 XCDs round-robin (id % 8), each
 // XCD with its own L2.  Renumbering so that consecutive logical indices run
-// on one XCD keeps the workgroups that share a weight tile (consecutive in
-// both kernels' tile orders) on one L2: each XCD then fetches only its own
-// share of the weights, instead of every XCD fetching all of them.
+// on one XCD keeps the workgroups that share operand tiles (tile_of) on one
+// L2: each XCD then fetches only its own share of the weights, instead of
+// every XCD fetching all of them.
 __device__ inline int xcd_logical(int id, int total) {
   constexpr int kXcds = 8;
   const int q = total / kXcds, r = total % kXcds, x = id % kXcds;
   return x * q + min(x, r) + id / kXcds;
 }
 
-__device__ inline f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-// Lane (g, c) of wave (wf, wt) holds C^T rows f0 + 32 wf + 16 fb + 4g + r
-// (features) of column t0 + 32 wt + 16 tb + c (token): C[token][f .. f + 3].
-__device__ inline void store_tile(const f32x4 (&acc)[2][2], float* c, long ldc, int f0, int t0,
-                                  int n_feat, int T, int wf, int wt, int lane) {
-  const int g = lane >> 4, cl = lane & 15;
-#pragma unroll
-  for (int tb = 0; tb < 2; ++tb) {
-    const int t = t0 + 32 * wt + 16 * tb + cl;
-    if (t >= T) continue;
-#pragma unroll
-    for (int fb = 0; fb < 2; ++fb) {
-      const int f = f0 + 32 * wf + 16 * fb + 4 * g;
-      if (f < n_feat) *reinterpret_cast<f32x4*>(c + (long)t * ldc + f) = acc[fb][tb];
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
-// Forward: workgroup b of job z is (split s, token tile, feature tile) with
-// s fastest; the reduction covers inputs [s kchunk, (s + 1) kchunk) n K.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kGThreads) void proj_gemm_nt_kernel(const NarrowFwd a) {
-  __shared__ __align__(16) bf16 lds[2][2][kGTile];  // [buffer][W, X]
-  const int id = xcd_logical((int)blockIdx.x, (int)gridDim.x);
-  int z = 0;
-  while (z + 1 < a.n && id >= a.j[z + 1].first) ++z;
-  const NarrowJob& job = a.j[z];
-  const int b = id - job.first;
-  const int s = b % a.nsplit, tile = b / a.nsplit;
-  const int ttiles = (a.T + kGT - 1) / kGT;
-  const int t0 = kGT * (tile % ttiles), f0 = kGT * (tile / ttiles);
-  const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
-  const int wf = w & 1, wt = w >> 1, g = lane >> 4, c = lane & 15;
-  const int k_begin = min(a.K, s * a.kchunk), k_end = min(a.K, k_begin + a.kchunk);
-  const int nst = (k_end - k_begin) / kGK;
-  const RowSrc ws = row_src(static_cast<const bf16*>(job.w), a.K, f0, job.n - f0, a.K * 2);
-  const RowSrc xs = row_src(static_cast<const bf16*>(a.x), a.K, t0, a.T - t0, a.K * 2);
-
-  f32x4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-  // kGPf stages in flight: stage st sits in register slot st % kGPf from
-  // its load until it is stored to LDS buffer st % 2, kGPf stages later.
-  // Every load is issued unconditionally (stages past the end read through a
-  // zero-length resource, i.e. zeros, and add nothing), so the loop body has
-  // no branch and the compiler waits only for the slot it stores.
-  const RowSrc zero = row_src(static_cast<const bf16*>(job.w), a.K, 0, 0, 0);
-  Stage pw[kGPf], px[kGPf];
-  auto issue = [&](Stage& w_, Stage& x_, int st) {
-    RowSrc w1 = zero, x1 = zero;
-    if (st < nst) {
-      w1 = ws;
-      x1 = xs;
-    }
-    w_.load(w1, k_begin + kGK * st, tid);
-    x_.load(x1, k_begin + kGK * st, tid);
-  };
-#pragma unroll
-  for (int j = 0; j < kGPf; ++j) {
-    issue(pw[j], px[j], j);
-    __builtin_amdgcn_sched_barrier(0);  // slot order = issue order
-  }
-  for (int st0 = 0; st0 < nst; st0 += kGPf) {
-#pragma unroll
-    for (int j = 0; j < kGPf; ++j) {
-      const int st = st0 + j;
-      bf16* wl = lds[j & 1][0];
-      bf16* xl = lds[j & 1][1];
-      pw[j].store(wl, tid);
-      px[j].store(xl, tid);
-      __syncthreads();
-      issue(pw[j], px[j], st + kGPf);
-      // keep the loads of slot j here, before the products: scheduled later
-      // they would be the newest loads when slot j is next stored, and that
-      // store would wait for every load in flight
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int kk = 0; kk < kGK / 32; ++kk) {
-        bf16x8 af[2], bf[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          af[i] = *reinterpret_cast<const bf16x8*>(wl + (32 * wf + 16 * i + c) * kGS + 32 * kk + 8 * g);
-          bf[i] = *reinterpret_cast<const bf16x8*>(xl + (32 * wt + 16 * i + c) * kGS + 32 * kk + 8 * g);
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int jj = 0; jj < 2; ++jj) acc[i][jj] = mfma_bf16(af[i], bf[jj], acc[i][jj]);
-      }
-    }
-  }
-  // partial s of this job: [T][n] at job.c + s T n (every split writes its
-  // slice, zeros for an empty one, so the sum over slices is complete)
-  store_tile(acc, job.c + (long)s * a.T * job.n, job.n, f0, t0, job.n, a.T, wf, wt, lane);
-}
-
-// ---------------------------------------------------------------------------
-// Backward: workgroup (input tile, token tile); the reduction runs over the
-// outputs of job 0, then job 1, ...  A operand W_p[k][f] read transposed from
-// its row-major LDS tile (permuted k-slots {4g + r} U {16 + 4g + r} of each
-// 32-step); B operand dY_p[t][k] read as the same slots, 8 bytes at a time.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kGThreads) void proj_gemm_nn_kernel(const NarrowBwd a) {
-  __shared__ __align__(16) bf16 lds[2][2][kGTile];  // [buffer][W, dY]
-  const int ttiles = (a.T + kGT - 1) / kGT;
-  const int id = xcd_logical((int)blockIdx.x, (int)gridDim.x);
-  const int t0 = kGT * (id % ttiles), f0 = kGT * (id / ttiles);
-  const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
-  const int wf = w & 1, wt = w >> 1, g = lane >> 4, c = lane & 15;
-
-  f32x4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-  // stage st belongs to job z with local reduction offset k0
-  int nst = 0;
-  for (int z = 0; z < a.n; ++z) nst += a.j[z].n / kGK;
-  auto src = [&](int st, RowSrc& ws, RowSrc& ys, int& k0) {
-    int z = 0, base = 0;
-    while (z + 1 < a.n && st >= base + a.j[z].n / kGK) base += a.j[z++].n / kGK;
-    const NarrowJob& job = a.j[z];
-    k0 = kGK * (st - base);
-    // W_p rows k0 .. k0 + 63 (of n), columns f0 ..; dY_p rows t0 .. (tokens)
-    ws = row_src(static_cast<const bf16*>(job.w), a.K, k0, job.n - k0, a.K * 2);
-    ys = row_src(static_cast<const bf16*>(job.dy), job.n, t0, a.T - t0, job.n * 2);
-  };
-  // as in the forward: loads unconditional, stages past the end zeros
-  const RowSrc zero = row_src(static_cast<const bf16*>(a.j[0].w), a.K, 0, 0, 0);
-  Stage pw[kGPf], py[kGPf];
-  auto issue = [&](Stage& w_, Stage& y_, int st) {
-    RowSrc ws = zero, ys = zero;
-    int k0 = 0;
-    if (st < nst) src(st, ws, ys, k0);
-    w_.load(ws, f0, tid);
-    y_.load(ys, k0, tid);
-  };
-#pragma unroll
-  for (int j = 0; j < kGPf; ++j) {
-    issue(pw[j], py[j], j);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  for (int st0 = 0; st0 < nst; st0 += kGPf) {
-#pragma unroll
-    for (int j = 0; j < kGPf; ++j) {
-      const int st = st0 + j;
-      bf16* wl = lds[j & 1][0];  // [k][f]
-      bf16* yl = lds[j & 1][1];  // [t][k]
-      pw[j].store(wl, tid);
-      py[j].store(yl, tid);
-      __syncthreads();
-      issue(pw[j], py[j], st + kGPf);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int kk = 0; kk < kGK / 32; ++kk) {
-        bf16x8 af[2], bf[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const bf16x4 lo = read_tr<kGS>(wl, 32 * kk, 32 * wf + 16 * i, lane);
-          const bf16x4 hi = read_tr<kGS>(wl, 32 * kk + 16, 32 * wf + 16 * i, lane);
-          const bf16* yr = yl + (32 * wt + 16 * i + c) * kGS + 32 * kk + 4 * g;
-          const bf16x4 ylo = *reinterpret_cast<const bf16x4*>(yr);
-          const bf16x4 yhi = *reinterpret_cast<const bf16x4*>(yr + 16);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            af[i][r] = lo[r];
-            af[i][4 + r] = hi[r];
-            bf[i][r] = ylo[r];
-            bf[i][4 + r] = yhi[r];
-          }
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int jj = 0; jj < 2; ++jj) acc[i][jj] = mfma_bf16(af[i], bf[jj], acc[i][jj]);
-      }
-    }
-  }
-  store_tile(acc, a.c, a.K, f0, t0, a.K, a.T, wf, wt, lane);
-}
-
-// ---------------------------------------------------------------------------
-// Wide projections (bf16 tensors; q of a Qwen-style block: 3584 x 3584): a
-// workgroup computes a 128-feature x 64-token tile of C^T on
-// v_mfma_f32_32x32x16_bf16, 4 waves of 64 features x 32 tokens each (two
-// 32 x 32 accumulator blocks per wave).  Stages of 64 reduction elements go
-// global -> LDS by DMA (buffer_load ... lds, 16 bytes a lane) into a 4-slot
-// ring, three stages ahead; one workgroup barrier per stage.  Rows are
-// unpadded with their 16-byte pieces XOR-swizzled (lds_sw), so the fragment
-// reads (16 rows x one piece per quarter-wave) and the transposing reads of
-// the backward (4 rows x 4 pieces per half-wave) are free of bank conflicts.
-//   forward  (NT) C^T[f][t] = sum_k W[f][k] X[t][k]: both operands are read
-//            as fragments, A from the [128][64] W tile, B from the [64][64]
-//            X tile;
-//   backward (NN) C^T[c][t] = sum_f W[f][c] dY[t][f]: A from the [64 f][128 c]
-//            W tile by ds_read_b64_tr_b16 (four f of one column per read,
-//            two reads per k-step), B from the [64][64] dY tile.
+// bf16 tensors.  One launch per direction takes every projection of the call:
+//   forward  (NT) Y_p[t][f] = sum_k X[t][k] W_p[f][k] + bias_p[f] + s_p (L_p B_p)[t][f]
+//   backward (NN) dX[t][c]  = sum_p sum_f dY_p[t][f] W_p[f][c] + s_p (dL_p A_p^T)[t][c]
+// with L_p = X A_p and dL_p = dY_p B_p^T in fp32 from lowrank_split.
+//
+// A workgroup of 8 waves computes a FT-feature x TT-token tile of the
+// transposed product C^T on v_mfma_f32_32x32x16_bf16: WF x WT waves of FB x
+// TB blocks of 32 x 32, times WK groups that share the k-steps of a stage
+// (their sums are added in group order through LDS at the end).  Stages of KT
+// reduction elements go global -> LDS by DMA (buffer_load ... lds, 16 bytes a
+// lane) into a ring of RING slots.  LDS rows are KT elements of a feature or
+// token (backward A: 64 features of one reduction row, FT / 64 such
+// sub-tiles), unpadded, their 16-byte pieces XOR-swizzled (lds_sw): fragment
+// reads and transposing reads (ds_read_b64_tr_b16) are free of bank conflicts.
+// Rows past T or past a projection's outputs, and the pieces past the
+// reduction's end, are outside the DMA's buffer range and arrive as zeros.
+//
+// The low-rank product is a further stretch of the same reduction: both fp32
+// operands are split in three bf16 terms (split3.hpp), laid out six times r
+// wide by lowrank_split so that one bf16 product sums the six term products.
+// A call that holds a non-finite value there (its marks, `odd`) takes fp32
+// MFMAs for it instead.  The bias starts the accumulators, and the bf16
+// conversion happens as the tile leaves through LDS in whole row pieces.  So
+// no fp32 product goes to memory and back.
 // MFMA layout (lane l, c = l % 32, h = l / 32): A[row c][k = 8h .. 8h + 7],
 // B[k = 8h ..][col c]; accumulator element e holds column c, row
-// 8 (e / 4) + 4h + e % 4, so each group of four is four consecutive
-// features of one token: one 16-byte store.
+// 8 (e / 4) + 4h + e % 4.
+//
+// What bounds it: large calls, the matrix cores at the clock the chip holds
+// under them (1.45-1.5 GHz with every CU on MFMAs of random data): 4096 x 4096
+// x 4096 forward 137 us (1.0 PFLOP/s), the products alone 117 us; 220 us before
+// (and 24 us of lowrank_out).  Small calls, the DMA: a 1 KB instruction takes
+// 16 clocks of the CU's vector-memory unit from L2 (24 with 64-byte rows, 24-28
+// when the chip's CUs share the fabric), and a stage's DMA is issued in a burst
+// behind its barrier.  512 x 3584 -> 3584/512/512: forward 33 us, backward 35
+// us, against 21.6 + 11.7 + 6.3 and 24.9 + 15.0 + 8.4 us in three launches.
 // ---------------------------------------------------------------------------
-constexpr int kWF = 128;                 // features per tile
-constexpr int kWT = 64;                  // tokens per tile
-constexpr int kWK = 64;                  // reduction elements per stage
-constexpr int kWA = kWF * kWK * 2;       // A tile bytes (16 KB)
-constexpr int kWB = kWT * kWK * 2;       // B tile bytes (8 KB)
-constexpr int kWStage = kWA + kWB;       // one ring slot
-constexpr int kWRing = 4;
-constexpr int kWThreads = 256;
-constexpr int kWDma = (kWA + kWB) / 1024 / 4;  // DMA instructions per wave per stage (6)
-
-static_assert(kWRing * kWStage <= 160 * 1024, "ring exceeds the LDS of a CU");
-static_assert(kWStage + 4096 * 3 < 65536, "read immediates fit their 16-bit field");
+constexpr int kGThreads = 512;  // 8 waves
+[[maybe_unused]] constexpr int kOob = 0x7ffffff0;  // a buffer offset past every range: reads as zero
 
 #if defined(__HIP_DEVICE_COMPILE__)
 __device__ inline f32x16 mma32(const bf16x8& a, const bf16x8& b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// Per-lane DMA offsets of 128-byte rows (8 pieces): instruction n covers
-// rows 8 n .. 8 n + 7; lane l writes slot l % 8 of row 8 n + l / 8 and
-// fetches the global piece slot ^ lds_sw<64>(row), which repeats every two
-// instructions.  256-byte rows (16 pieces): rows 4 n .. 4 n + 3, slot l % 16,
-// piece slot ^ lds_sw<128>(row), repeating every four instructions.
-__device__ inline int dma_off128(int lane, int n, int rowb) {
-  const int r = 8 * n + (lane >> 3), slot = lane & 7;
-  return (lane >> 3) * rowb + 16 * (slot ^ lds_sw<64>(r));
-}
-__device__ inline int dma_off256(int lane, int n, int rowb) {
-  const int r = 4 * n + (lane >> 4), slot = lane & 15;
-  return (lane >> 4) * rowb + 16 * (slot ^ lds_sw<128>(r));
-}
-
-// Byte offset, inside a tile of 128-byte rows, of this lane's fragment read
-// of k-step 0 for rows row0 + lane % 32 (row0 a multiple of 16); k-step s
-// reads at that offset ^ 32 s.
-__device__ inline unsigned frag_off128(int lane, int row0) {
+// Byte offset, inside a tile of rows of KT elements, of this lane's fragment
+// read of k-step 0 for rows row0 + lane % 32 (row0 a multiple of 16); k-step
+// s reads at that offset ^ 32 s, the 32 rows after at + 64 KT.
+template <int KT>
+__device__ inline unsigned frag_off(int lane, int row0) {
   const int r = row0 + (lane & 31), h = lane >> 5;
-  return static_cast<unsigned>(r * 128 + 16 * (h ^ lds_sw<64>(r)));
+  return static_cast<unsigned>(r * 2 * KT + 16 * (h ^ lds_sw<KT>(r)));
 }
-// Byte offset, inside a tile of 256-byte rows, of this lane's transposing
-// read j (0, 1) of k-step 0 for columns col0 + 16 (G & 1) + 4 (i & 3)
-// (quarter-wave G, lane i in it): rows 8 h + 4 j + i / 4; k-step s reads
-// 16 s rows further (+4096 s), the 32 columns after col0 at ^ 64.
-__device__ inline unsigned tr_off256(int lane, int col0, int j) {
+// Byte offset, inside a sub-tile of 64 reduction rows x 64 features, of this
+// lane's transposing read j (0, 1) of k-step 0 for features col0 + 16 (G & 1)
+// + 4 (i & 3) (quarter-wave G, lane i in it): rows 8 h + 4 j + i / 4; k-step
+// s reads 16 s rows further (+2048 s).
+__device__ inline unsigned tr_off128(int lane, int col0, int j) {
   const int G = lane >> 4, i = lane & 15, h = lane >> 5;
   const int r = 8 * h + 4 * j + (i >> 2);
   const int col = col0 + 16 * (G & 1) + 4 * (i & 3);
-  return static_cast<unsigned>(r * 256 + 16 * ((col >> 3) ^ lds_sw<128>(r)) + 2 * (col & 7));
-}
-
-// Stores this wave's two 32 x 32 blocks (features fw + 32 fb, tokens tw) of
-// C^T into C [T][ldc] (fp32), rows past T skipped.
-__device__ inline void store_wide(const f32x16 (&acc)[2], float* c, long ldc, int fw, int tw, int T,
-                                  int lane) {
-  const int t = tw + (lane & 31), h = lane >> 5;
-  if (t >= T) return;
-#pragma unroll
-  for (int fb = 0; fb < 2; ++fb)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int f = fw + 32 * fb + 8 * q + 4 * h;
-      *reinterpret_cast<f32x4*>(c + (long)t * ldc + f) =
-          f32x4{acc[fb][4 * q], acc[fb][4 * q + 1], acc[fb][4 * q + 2], acc[fb][4 * q + 3]};
-    }
+  return static_cast<unsigned>(r * 128 + 16 * ((col >> 3) ^ lds_sw<64>(r)) + 2 * (col & 7));
 }
 #endif
 
-// The stage loop shared by both directions: prologue of three stages, then
-// per stage: wait for this wave's DMA of the stage (the two later stages
-// stay in flight), barrier, DMA of the stage three ahead into the slot just
-// freed (every wave's reads of it completed before the barrier) (unconditional: past the end
-// it reads through an empty resource), then the stage's products.  The ring
-// slot of every read is an immediate offset: slots 0, 1 from the lane's
-// addresses as given, slots 2, 3 from the same + 2 kWStage.
-template <typename Issue, typename Compute>
-__device__ inline void wide_loop(int nst, Issue&& issue, Compute&& compute) {
-  issue(0, 0);
-  issue(1, 1);
-  issue(2, 2);
-  int st = 0;
-  auto one = [&](auto slot) {
-    constexpr int SL = decltype(slot)::value;
-    vmw<2 * kWDma>();
-    wg_barrier();
-    issue(st + 3, (SL + 3) & 3);
-    compute(slot);
-    ++st;
+// Tile id -> (feature tile, token tile): bands of 4 feature tiles, feature
+// fastest inside a band, so that the 32 workgroups an XCD runs at once cover
+// a block of about 4 x 8 tiles and share both operands through its L2.
+[[maybe_unused]] __device__ inline void tile_of(int id, int ftiles, int ttiles, int& f, int& t) {
+  const int band = id / (4 * ttiles), in = id - band * 4 * ttiles;
+  const int width = min(4, ftiles - 4 * band);
+  t = in / width;
+  f = 4 * band + in - t * width;
+}
+
+template <int FB, int TB, int WK>
+constexpr int block_owner(int fb, int tb) {
+  if constexpr (WK == 1)
+    return 0;
+  else if constexpr (FB % 2 == 0)
+    return fb / (FB / 2);
+  else if constexpr (TB % 2 == 0)
+    return tb / (TB / 2);
+  else
+    return 0;
+}
+
+template <bool NN, int KT, int FB, int TB, int WF, int WT, int WK, int G, int RING>
+__global__ __launch_bounds__(kGThreads) void proj_gemm_kernel(const GemmCall a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  static_assert(WF * WT * WK == 8 && (WK == 1 || WK == 2), "8 waves");
+  constexpr int FT = WF * FB * 32, TT = WT * TB * 32;
+  constexpr int RI = 1024 / (2 * KT);  // operand rows per DMA instruction
+  constexpr int NA = FT / (8 * RI), NB = TT / (8 * RI), ND = NA + NB;  // per wave and stage
+  constexpr int kA = FT * KT * 2, kStage = (FT + TT) * KT * 2;
+  static_assert(FT % (8 * RI) == 0 && TT % (8 * RI) == 0 && RING >= 2 && RING * kStage <= 160 * 1024, "tile");
+  constexpr int KS = KT / 16 / WK;  // k-steps of a stage per wave
+  constexpr int U = KS / G;         // units of a stage: G k-steps each
+  static_assert(KS % G == 0 && (U == 1 || U % 2 == 0), "fragment buffers alternate");
+  __shared__ __align__(1024) unsigned char lds[RING * kStage];
+  const int ttiles = (a.T + TT - 1) / TT;
+  const int id = xcd_logical((int)blockIdx.x, (int)gridDim.x);
+  int ft, tt;
+  tile_of(id, a.ftiles, ttiles, ft, tt);
+  int z = 0;  // forward: the tile's projection
+  if constexpr (!NN)
+    while (z + 1 < a.n && ft >= a.j[z + 1].first) ++z;
+  const int f0 = NN ? FT * ft : FT * (ft - a.j[z].first), t0 = TT * tt;
+  const int nf = NN ? a.K : a.j[z].n;  // features of the output
+  const int lane = threadIdx.x & 63, w = wave_id();
+  const int wf = w % WF, wt = w / WF % WT, wk = w / (WF * WT);
+  // a non-finite value among the low-rank operands: see below
+  bool slow = false;
+  for (int i = lane; i < a.n_odd; i += 64) slow |= a.odd[i] != 0;
+  slow = __any(slow);
+
+  // DMA: instruction i of this wave covers RI rows of an operand (backward A:
+  // 8 reduction rows of a sub-tile); a lane writes one 16-byte slot of a row
+  // and fetches the piece that belongs there.
+  constexpr int PR = KT / 8;  // pieces per row
+  const int row = RI * w + lane / PR;
+  const int piece = (lane % PR) ^ lds_sw<KT>(row);
+  int va[NA], vb[NB];
+  __amdgpu_buffer_rsrc_t ra, rb;
+  if constexpr (NN) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      const int n = w + 8 * i, r = 8 * (n % (KT / 8)) + (lane >> 3);
+      const int c = 64 * (n / (KT / 8)) + 8 * ((lane & 7) ^ lds_sw<64>(r));
+      va[i] = f0 + c < a.K ? r * a.K * 2 + 2 * c : kOob;
+    }
+  }
+  // the segments of the reduction: forward X W^T then L_p B_p, backward
+  // every dY_p W_p then every dL_p A_p^T (seg[kMaxProj + p], in split terms)
+  const int T = a.T, K = a.K, n_seg = a.n;
+  int nst = 0, sg = NN ? -1 : z - kMaxProj, kend = 0, kbase = 0, kcur = 0;
+  for (int y = NN ? 0 : z; y < (NN ? n_seg : z + 1); ++y)
+    nst += (a.seg[y].k + KT - 1) / KT + (slow ? 0 : (a.seg[kMaxProj + y].k + KT - 1) / KT);
+  // advance(st) (in order: 0, 1, ...) points the DMA at stage st; dma<i>(slot)
+  // issues its instruction i into ring slot `slot`
+  const bf16* wrow = nullptr;  // backward: A's rows from the segment's first, column f0
+  int k0 = 0;
+  bool past = false;  // this lane's piece lies past the segment's end
+  auto advance = [&](int st) {
+    while (st >= kend) {  // the next segment
+      sg = NN ? (sg + 1 == n_seg ? kMaxProj : sg + 1) : sg + kMaxProj;
+      kbase = kend;
+      kcur = a.seg[sg].k;
+      kend += (kcur + KT - 1) / KT;
+      const int rowb = kcur * 2;
+      rb = wave_rsrc(static_cast<const bf16*>(a.seg[sg].b) + (long)t0 * kcur, min(TT, T - t0) * rowb);
+#pragma unroll
+      for (int i = 0; i < NB; ++i) vb[i] = (8 * RI * i + row) * rowb + 16 * piece;
+      if constexpr (NN) {
+        wrow = static_cast<const bf16*>(a.seg[sg].a) + f0;
+      } else {
+        ra = wave_rsrc(static_cast<const bf16*>(a.seg[sg].a) + (long)f0 * kcur, min(FT, nf - f0) * rowb);
+#pragma unroll
+        for (int i = 0; i < NA; ++i) va[i] = (8 * RI * i + row) * rowb + 16 * piece;
+      }
+    }
+    k0 = (st - kbase) * KT;
+    if constexpr (NN)
+      ra = wave_rsrc(wrow + (long)k0 * K, (min(KT, kcur - k0) - 1) * K * 2 + (K - f0) * 2);
+    past = k0 + KT > kcur && k0 + 8 * piece >= kcur;
   };
+  auto dma = [&](auto ic, int slot) {
+    constexpr int I = decltype(ic)::value;
+    unsigned char* base = lds + slot * kStage + 1024 * w;
+    if constexpr (I < NA)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (GLACIER_LDS void*)(base + 8192 * I), 16,
+                                               NN ? va[I] : past ? kOob : va[I], NN ? 0 : 2 * k0, 0, 0);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (GLACIER_LDS void*)(base + kA + 8192 * (I - NA)), 16,
+                                               past ? kOob : vb[I - NA], 2 * k0, 0, 0);
+  };
+#pragma unroll
+  for (int i = 0; i < RING; ++i)
+    if (i < nst) {
+      advance(i);
+      static_for<ND>([&](auto ic) { dma(ic, i); });
+    }
+
+  // the accumulators start at the bias (in one group's)
+  f32x16 acc[FB][TB];
+  const int fw = f0 + 32 * FB * wf, tw = t0 + 32 * TB * wt;
+  const float* bias = NN || wk != 0 ? nullptr : a.j[z].bias;
+#pragma unroll
+  for (int fb = 0; fb < FB; ++fb)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int f = fw + 32 * fb + 8 * (e / 4) + 4 * (lane >> 5) + e % 4;
+      const float b = bias == nullptr ? 0.0f : bias[min(f, nf - 1)];
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb) acc[fb][tb][e] = b;
+    }
+  if (slow && wk == 0) {
+    // the low-rank products of a call with non-finite values, which have no
+    // split terms: sum over the terms of (s L [T][r]) V, V = B [r][n]
+    // (forward) or A^T with A [K][r], on fp32 MFMAs
+    for (int p = NN ? 0 : z; p < (NN ? a.n : z + 1); ++p) {
+      const GemmJob& job = a.j[p];
+      if (job.l == nullptr) continue;
 #pragma clang loop unroll(disable)
-  while (st + 3 < nst) {
-    one(std::integral_constant<int, 0>{});
-    one(std::integral_constant<int, 1>{});
-    one(std::integral_constant<int, 2>{});
-    one(std::integral_constant<int, 3>{});
-  }
-  if (st < nst) one(std::integral_constant<int, 0>{});
-  if (st < nst) one(std::integral_constant<int, 1>{});
-  if (st < nst) one(std::integral_constant<int, 2>{});
-  vmw<0>();  // the DMA issued past the end lands before the workgroup ends
-}
-
-__global__ __launch_bounds__(kWThreads) void proj_gemm_wide_nt_kernel(const WideFwd a) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  __shared__ __align__(1024) unsigned char lds[kWRing * kWStage];
-  const int ttiles = (a.T + kWT - 1) / kWT;
-  const int id = xcd_logical((int)blockIdx.x, (int)gridDim.x);
-  const int t0 = kWT * (id % ttiles), f0 = kWF * (id / ttiles);
-  const int lane = threadIdx.x & 63, w = wave_id();
-  const int wf = w & 1, wt = w >> 1;
-  const int rowb = a.K * 2;
-  // A: W rows f0 .., B: X rows t0 .. (rows past T read as zeros)
-  const __amdgpu_buffer_rsrc_t ra =
-      wave_rsrc(static_cast<const bf16*>(a.w) + (long)f0 * a.K, kWF * rowb);
-  const __amdgpu_buffer_rsrc_t rb = wave_rsrc(static_cast<const bf16*>(a.x) + (long)t0 * a.K,
-                                              max(0, min(kWT, a.T - t0)) * rowb);
-  const __amdgpu_buffer_rsrc_t rz = wave_rsrc(a.x, 0);
-  // this wave's DMA: A rows 32 w .. 32 w + 31 (4 instructions; every row
-  // valid, the row block in the scalar offset), B rows 16 w .. 16 w + 15 (2
-  // instructions; the row in the per-lane offset, which alone is checked
-  // against the resource's range, so rows past T read as zeros)
-  const int oa0 = dma_off128(lane, 0, rowb), oa1 = dma_off128(lane, 1, rowb);
-  const int ob0 = dma_off128(lane, 0, rowb) + 16 * w * rowb, ob1 = dma_off128(lane, 1, rowb) + (16 * w + 8) * rowb;
-  const unsigned sbase = static_cast<unsigned>(reinterpret_cast<uintptr_t>((GLACIER_LDS void*)lds));
-  auto issue = [&](int st, int slot) {
-    const bool live = st < a.K / kWK;
-    const __amdgpu_buffer_rsrc_t sa = live ? ra : rz, sb = live ? rb : rz;
-    unsigned char* base = lds + slot * kWStage;
-    const int k0 = st * kWK * 2;
+      for (int k0 = 0; k0 < a.rank; k0 += 2) {
+        const int kk = min(k0 + (lane >> 5), a.rank - 1);
+        const bool k_ok = k0 + (lane >> 5) < a.rank;
+        float lv[TB], vv[FB];
 #pragma unroll
-    for (int n = 0; n < 4; ++n)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(sa, (GLACIER_LDS void*)(base + (32 * w + 8 * n) * 128), 16,
-                                               (n & 1) ? oa1 : oa0, (32 * w + 8 * n) * rowb + k0, 0, 0);
+        for (int tb = 0; tb < TB; ++tb) {
+          const float v = job.l[(long)min(tw + 32 * tb + (lane & 31), a.T - 1) * a.rank + kk];
+          lv[tb] = k_ok ? job.s * v : 0.0f;
+        }
 #pragma unroll
-    for (int n = 0; n < 2; ++n)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(sb, (GLACIER_LDS void*)(base + kWA + (16 * w + 8 * n) * 128),
-                                               16, n ? ob1 : ob0, k0, 0, 0);
-  };
-  // read addresses: A rows 64 wf + 32 fb (fb at +4096), B rows 32 wt; k-step s
-  unsigned fa[2][4], fbb[2][4];
-  {
-    const unsigned oa = frag_off128(lane, 64 * wf), ob = frag_off128(lane, 32 * wt);
+        for (int fb = 0; fb < FB; ++fb) {
+          const int f = min(fw + 32 * fb + (lane & 31), nf - 1);
+          const float v = NN ? job.v[(long)f * a.rank + kk] : job.v[(long)kk * nf + f];
+          vv[fb] = k_ok ? v : 0.0f;
+        }
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      fa[0][s] = sbase + (oa ^ (32u * s));
-      fbb[0][s] = sbase + kWA + (ob ^ (32u * s));
-      fa[1][s] = fa[0][s] + 2 * kWStage;
-      fbb[1][s] = fbb[0][s] + 2 * kWStage;
+        for (int fb = 0; fb < FB; ++fb)
+#pragma unroll
+          for (int tb = 0; tb < TB; ++tb)
+            acc[fb][tb] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[fb], lv[tb], acc[fb][tb], 0, 0, 0);
+      }
     }
   }
-  f32x16 acc[2];
+
+  // read addresses of k-step s of slot 0: A (NT: fragments, blocks 32 rows
+  // apart; NN: transposing reads j of each block), B fragments
+  const unsigned sbase = static_cast<unsigned>(reinterpret_cast<uintptr_t>((GLACIER_LDS void*)lds));
+  unsigned oa[NN ? 2 * FB : KS], ob[KS];
+  {
+    const unsigned b = frag_off<KT>(lane, 32 * TB * wt);
 #pragma unroll
-  for (int fb = 0; fb < 2; ++fb)
+    for (int s = 0; s < KS; ++s) ob[s] = sbase + kA + (b ^ (32u * (KS * wk + s)));
+    if constexpr (NN) {
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[fb][e] = 0.0f;
-  auto compute = [&](auto slot) {
-    constexpr int SL = decltype(slot)::value, HS = SL >> 1, OFF = (SL & 1) * kWStage;
-    bf16x8 ra_[4][2], rb_[4];
-    auto rd = [&](auto sc) {
-      constexpr int S = decltype(sc)::value;
-      ra_[S][0] = rd128<OFF>(fa[HS][S]);
-      ra_[S][1] = rd128<OFF + 4096>(fa[HS][S]);
-      rb_[S] = rd128<OFF>(fbb[HS][S]);
-    };
-    rd(std::integral_constant<int, 0>{});
-    rd(std::integral_constant<int, 1>{});
-    static_for<4>([&](auto sc) {
-      constexpr int S = decltype(sc)::value;
-      if constexpr (S + 2 < 4) {
-        lgkm<3>();
-        rd(std::integral_constant<int, S + 2>{});
-        lgkm<6>();
-      } else if constexpr (S == 2) {
-        lgkm<3>();
-      } else {
-        lgkm<0>();
+      for (int fb = 0; fb < FB; ++fb) {
+        const int col = 32 * (FB * wf + fb);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          oa[2 * fb + j] = sbase + 128u * KT * (col / 64) + tr_off128(lane, col % 64, j) + 2048u * KS * wk;
       }
-      tie_v(ra_[S][0]);
-      tie_v(ra_[S][1]);
-      tie_v(rb_[S]);
-      acc[0] = mma32(ra_[S][0], rb_[S], acc[0]);
-      acc[1] = mma32(ra_[S][1], rb_[S], acc[1]);
+    } else {
+      const unsigned o = frag_off<KT>(lane, 32 * FB * wf);
+#pragma unroll
+      for (int s = 0; s < KS; ++s) oa[s] = sbase + (o ^ (32u * (KS * wk + s)));
+    }
+  }
+  // fragments in two buffers of one unit (G k-steps) each
+  constexpr int NRK = (NN ? 2 * FB : FB) + TB, NRD = G * NRK, NM = G * FB * TB;
+  bf16x8 fa[2][G][FB], fbk[2][G][TB];
+  bf16x4 ta[2][G][FB][2];
+  // read i of unit N of a stage into buffer P: the A blocks' first, then B's
+  auto rd = [&](auto pc, auto nc, auto ic, unsigned so) {
+    constexpr int P = decltype(pc)::value, I = decltype(ic)::value % NRK, g = decltype(ic)::value / NRK;
+    constexpr int S = decltype(nc)::value * G + g;
+    if constexpr (I >= NRK - TB)
+      fbk[P][g][I - (NRK - TB)] = rd128<64 * KT * (I - (NRK - TB))>(ob[S] + so);
+    else if constexpr (NN)
+      ta[P][g][I / 2][I & 1] = rdtr<2048 * S>(oa[I] + so);
+    else
+      fa[P][g][I] = rd128<64 * KT * I>(oa[S] + so);
+  };
+  // the reads into buffer P have arrived
+  auto arrive = [&](auto pc) {
+    constexpr int P = decltype(pc)::value;
+    lgkm<0>();
+    static_for<G>([&](auto gc) {
+      constexpr int g = decltype(gc)::value;
+      static_for<FB>([&](auto fc) {
+        constexpr int F = decltype(fc)::value;
+        if constexpr (NN) {
+          tie_v(ta[P][g][F][0]);
+          tie_v(ta[P][g][F][1]);
+          fa[P][g][F] = join8(ta[P][g][F][0], ta[P][g][F][1]);
+        } else {
+          tie_v(fa[P][g][F]);
+        }
+      });
+      static_for<TB>([&](auto tc) { tie_v(fbk[P][g][decltype(tc)::value]); });
     });
   };
-  wide_loop(a.K / kWK, issue, compute);
-  store_wide(acc, a.c, a.n, f0 + 64 * wf, t0 + 32 * wt, a.T, lane);
-#endif
-}
-
-__global__ __launch_bounds__(kWThreads) void proj_gemm_wide_nn_kernel(const WideBwd a) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  __shared__ __align__(1024) unsigned char lds[kWRing * kWStage];
-  const int ttiles = (a.T + kWT - 1) / kWT;
-  const int id = xcd_logical((int)blockIdx.x, (int)gridDim.x);
-  const int t0 = kWT * (id % ttiles), c0 = kWF * (id / ttiles);
-  const int lane = threadIdx.x & 63, w = wave_id();
-  const int wf = w & 1, wt = w >> 1;
-  const int rowbw = a.K * 2;
-  int nst = 0;
-  for (int z = 0; z < a.n; ++z) nst += a.j[z].n / kWK;
-  const __amdgpu_buffer_rsrc_t rz = wave_rsrc(a.j[0].w, 0);
-  const int ow[4] = {dma_off256(lane, 0, rowbw), dma_off256(lane, 1, rowbw), dma_off256(lane, 2, rowbw),
-                     dma_off256(lane, 3, rowbw)};
-  const unsigned sbase = static_cast<unsigned>(reinterpret_cast<uintptr_t>((GLACIER_LDS void*)lds));
-  // the job of the stages being issued (stages are issued in order): its
-  // resources over W_z (from column c0) and dY_z (from token t0), its first
-  // stage and the first stage of the next job
-  int z = -1, zbase = 0, zend = 0, rowby = 0, oy0 = 0, oy1 = 0;
-  __amdgpu_buffer_rsrc_t ra = rz, rb = rz;
-  auto issue = [&](int st, int slot) {
-    while (st >= zend && z + 1 < a.n) {
-      ++z;
-      zbase = zend;
-      zend += a.j[z].n / kWK;
-      const WideJob& job = a.j[z];
-      rowby = job.n * 2;
-      ra = wave_rsrc(static_cast<const bf16*>(job.w) + c0, (job.n - 1) * rowbw + kWF * 2);
-      rb = wave_rsrc(static_cast<const bf16*>(job.dy) + (long)t0 * job.n,
-                     max(0, min(kWT, a.T - t0)) * rowby);
-      // the row in the per-lane offset (checked against the range: rows
-      // past T read as zeros), the column f0 in the scalar one
-      oy0 = dma_off128(lane, 0, rowby) + 16 * w * rowby;
-      oy1 = dma_off128(lane, 1, rowby) + (16 * w + 8) * rowby;
-    }
-    const bool live = st < nst;
-    const __amdgpu_buffer_rsrc_t sa = live ? ra : rz, sb = live ? rb : rz;
-    const int f0 = (st - zbase) * kWK;  // the job's reduction rows f0 .. f0 + 63
-    unsigned char* base = lds + slot * kWStage;
-    // A: W_z[f0 + r][c0 ..] (256-byte rows); B: dY_z[t0 + r][f0 ..] (128 bytes)
-#pragma unroll
-    for (int n = 0; n < 4; ++n)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(sa, (GLACIER_LDS void*)(base + (16 * w + 4 * n) * 256), 16,
-                                               ow[n], (f0 + 16 * w + 4 * n) * rowbw, 0, 0);
-#pragma unroll
-    for (int n = 0; n < 2; ++n)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(sb, (GLACIER_LDS void*)(base + kWA + (16 * w + 8 * n) * 128),
-                                               16, n ? oy1 : oy0, 2 * f0, 0, 0);
-  };
-  // read addresses: A transposed, columns 64 wf + 32 fb (fb: ^ 64), reads j;
-  // B fragments rows 32 wt, k-step s
-  unsigned ta[2][2][2], fbb[2][4];
-  {
-    const unsigned o0 = tr_off256(lane, 64 * wf, 0), o1 = tr_off256(lane, 64 * wf, 1);
-    const unsigned ob = frag_off128(lane, 32 * wt);
-#pragma unroll
-    for (int hs = 0; hs < 2; ++hs) {
-#pragma unroll
-      for (int fb = 0; fb < 2; ++fb) {
-        ta[hs][fb][0] = sbase + 2u * kWStage * hs + (o0 ^ (64u * fb));
-        ta[hs][fb][1] = sbase + 2u * kWStage * hs + (o1 ^ (64u * fb));
+  // Between the MFMAs of a unit go the fragment reads of the next one, one
+  // at a time (eight waves' reads in a row fill the LDS queue and hold up the
+  // products behind them).  The one barrier of a stage stands before its last
+  // unit, whose fragments have then arrived: past it every wave is done with
+  // the stage's slot, so the DMA of the stage RING ahead goes into it, and the
+  // next stage has landed (each wave waited for its own DMA of it), so the
+  // next unit's fragments are read behind the last products as usual.
+  // Every read is waited for in the stage that issues it: the loop carries
+  // only values that have arrived.
+  vm_wait_v((min(nst, RING) - 1) * ND);
+  wg_barrier();
+  static_for<NRD>([&](auto ic) { rd(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, ic, 0u); });
+  arrive(std::integral_constant<int, 0>{});
+  int slot = 0;
+  auto stage = [&](int st, auto p0c) {
+    const int next = slot + 1 == RING ? 0 : slot + 1;
+    const unsigned so = static_cast<unsigned>(slot * kStage), sn = static_cast<unsigned>(next * kStage);
+    const bool more = st + RING < nst;
+    static_for<U>([&](auto uc) {
+      constexpr int UN = decltype(uc)::value, P = (decltype(p0c)::value + UN) & 1, N = (UN + 1) % U;
+      constexpr bool kLast = UN == U - 1;
+      constexpr int NI = NM > NRD ? NM : NRD;
+      if constexpr (kLast) {
+        if (more)
+          vmw<(RING - 2) * ND>();
+        else
+          vm_wait_v(max(nst - 2 - st, 0) * ND);
+        wg_barrier();
+        if (more) advance(st + RING);
       }
-#pragma unroll
-      for (int s = 0; s < 4; ++s) fbb[hs][s] = sbase + 2u * kWStage * hs + kWA + (ob ^ (32u * s));
-    }
-  }
-  f32x16 acc[2];
-#pragma unroll
-  for (int fb = 0; fb < 2; ++fb)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[fb][e] = 0.0f;
-  auto compute = [&](auto slot) {
-    constexpr int SL = decltype(slot)::value, HS = SL >> 1, OFF = (SL & 1) * kWStage;
-    bf16x4 rt[4][2][2];
-    bf16x8 rb_[4];
-    auto rd = [&](auto sc) {
-      constexpr int S = decltype(sc)::value;
-#pragma unroll
-      for (int fb = 0; fb < 2; ++fb) {
-        rt[S][fb][0] = rdtr<OFF + 4096 * S>(ta[HS][fb][0]);
-        rt[S][fb][1] = rdtr<OFF + 4096 * S>(ta[HS][fb][1]);
-      }
-      rb_[S] = rd128<OFF>(fbb[HS][S]);
-    };
-    rd(std::integral_constant<int, 0>{});
-    rd(std::integral_constant<int, 1>{});
-    static_for<4>([&](auto sc) {
-      constexpr int S = decltype(sc)::value;
-      if constexpr (S + 2 < 4) {
-        lgkm<5>();
-        rd(std::integral_constant<int, S + 2>{});
-        lgkm<10>();
-      } else if constexpr (S == 2) {
-        lgkm<5>();
-      } else {
-        lgkm<0>();
-      }
-#pragma unroll
-      for (int fb = 0; fb < 2; ++fb) {
-        tie_v(rt[S][fb][0]);
-        tie_v(rt[S][fb][1]);
-      }
-      tie_v(rb_[S]);
-      acc[0] = mma32(join8(rt[S][0][0], rt[S][0][1]), rb_[S], acc[0]);
-      acc[1] = mma32(join8(rt[S][1][0], rt[S][1][1]), rb_[S], acc[1]);
+      __builtin_amdgcn_sched_barrier(0);
+      static_for<(kLast && ND > NI ? ND : NI)>([&](auto ic) {
+        constexpr int I = decltype(ic)::value;
+        if constexpr (I < NM) {
+          constexpr int g = I / (FB * TB), fb = I % (FB * TB) / TB, tb = I % TB;
+          acc[fb][tb] = mma32(fa[P][g][fb], fbk[P][g][tb], acc[fb][tb]);
+        }
+        if constexpr (I < NRD)  // past the last stage: a slot's old rows, unused
+          rd(std::integral_constant<int, P ^ 1>{}, std::integral_constant<int, N>{}, ic, kLast ? sn : so);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kLast && I < ND) {
+          if (more) dma(ic, slot);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      });
+      arrive(std::integral_constant<int, P ^ 1>{});
     });
+    slot = next;
   };
-  wide_loop(nst, issue, compute);
-  store_wide(acc, a.c, a.K, c0 + 64 * wf, t0 + 32 * wt, a.T, lane);
+  for (int st = 0; st < nst; ++st) {
+    stage(st, std::integral_constant<int, 0>{});
+    if constexpr (U == 1)  // the buffers change roles
+      if (++st < nst) stage(st, std::integral_constant<int, 1>{});
+  }
+
+  // Epilogue.  WK == 2: each group hands the other the blocks that one
+  // finishes, and adds its own to what it receives (group 0's first).
+  __syncthreads();
+  if constexpr (WK == 2) {
+    f32x4* ex = reinterpret_cast<f32x4*>(lds) + (w % (WF * WT)) * (FB * TB * 256);
+#pragma unroll
+    for (int fb = 0; fb < FB; ++fb)
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb)
+        if (block_owner<FB, TB, WK>(fb, tb) != wk)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            ex[(fb * TB + tb) * 256 + q * 64 + lane] =
+                f32x4{acc[fb][tb][4 * q], acc[fb][tb][4 * q + 1], acc[fb][tb][4 * q + 2], acc[fb][tb][4 * q + 3]};
+    __syncthreads();
+#pragma unroll
+    for (int fb = 0; fb < FB; ++fb)
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb)
+        if (block_owner<FB, TB, WK>(fb, tb) == wk)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const f32x4 o = ex[(fb * TB + tb) * 256 + q * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[fb][tb][4 * q + e] += o[e];
+          }
+    __syncthreads();
+  }
+  // bias, bf16, and out through LDS: 32 tokens x 32 FB features per wave at a
+  // time, rows of kOutRow bytes (padded), then 16-byte row pieces
+  constexpr int kOutRow = 64 * FB + 16;
+  unsigned char* mine = lds + w * 32 * kOutRow;
+  static_assert(8 * 32 * kOutRow <= RING * kStage, "output staging fits the ring");
+  const int h = lane >> 5;
+  bf16* out = static_cast<bf16*>(NN ? a.dx : a.j[z].y);
+#pragma unroll
+  for (int tb = 0; tb < TB; ++tb) {
+#pragma unroll
+    for (int fb = 0; fb < FB; ++fb) {
+      if (block_owner<FB, TB, WK>(fb, tb) != wk) continue;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int fl = 32 * fb + 8 * q + 4 * h;
+        bf16x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = (bf16)acc[fb][tb][4 * q + e];
+        *reinterpret_cast<bf16x4*>(mine + (lane & 31) * kOutRow + 2 * fl) = v;
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+    constexpr int PC = 4 * FB;  // 16-byte pieces per row
+#pragma unroll
+    for (int i = 0; i < 32 * PC / 64; ++i) {
+      const int idx = 64 * i + lane, r = idx / PC, pc = idx % PC;
+      const int t = tw + 32 * tb + r, f = fw + 8 * pc;
+      if (block_owner<FB, TB, WK>(pc / 4, tb) == wk && t < a.T && f < nf)
+        *reinterpret_cast<i32x4*>(out + (long)t * nf + f) = *reinterpret_cast<const i32x4*>(mine + r * kOutRow + 16 * pc);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
 #endif
 }
 
@@ -748,16 +572,12 @@ __global__ __launch_bounds__(kFThreads) void proj_gemm_f32_kernel(const WideFwd 
     for (int i = 0; i < 2; ++i) {
       const int f = f0 + 32 * wf + 16 * i + 4 * g;
       float* d = cdst + (long)t * nout + f;
-      // backward after the wide kernel: add to what it wrote
-      const bool add = NN && ba.accumulate;
       if (f + 3 < nout && (nout & 3) == 0) {
-        f32x4 v = acc[i][j];
-        if (add) v += *reinterpret_cast<const f32x4*>(d);
-        *reinterpret_cast<f32x4*>(d) = v;
+        *reinterpret_cast<f32x4*>(d) = acc[i][j];
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (f + e < nout) d[e] = add ? d[e] + acc[i][j][e] : acc[i][j][e];
+          if (f + e < nout) d[e] = acc[i][j][e];
       }
     }
   }
@@ -765,51 +585,82 @@ __global__ __launch_bounds__(kFThreads) void proj_gemm_f32_kernel(const WideFwd 
 
 }  // namespace
 
-bool narrow_gemm_fits(int in_features, int out_features) {
-  return in_features % kGK == 0 && out_features % kGK == 0 && out_features <= kNarrowMaxOut;
+namespace {
+
+// Tile shapes (features x tokens), the times a stage of theirs was measured
+// to take, and their instances.  us per launch, forward / backward (rank 16):
+//   T, in -> outs                    256x256  128x128/2  128x128  128x64  64x64
+//   4096, 4096 -> 4096               137/138  162/174    182/193  219/237 278/295
+//   4096, 4096 -> 4096/1024/1024     225/202  228/244    259/272  314/339 406/418
+//   1290, 3584 -> 3584/512/512       82/108   59/69      67/88    76/94   97/103
+//   512, 3584 -> 3584/512/512        76/105   44/58      33/45    42/36   44/44
+//   201, 896 -> 896/128/128          24/31    11/15      12/16    9.5/12  7.9/9.9
+//   37, 3584 -> 3584/512/512         72/100   40/51      28/40    20/31   16/21
+struct GemmShape {
+  int slots;            // workgroups resident at once
+  float alone, loaded;  // us per 64 reduction elements: few workgroups, every slot taken
+  int kt;
+  int ft, tt;
+  void (*nt)(GemmCall);
+  void (*nn)(GemmCall);
+};
+#define GL_GEMM(SLOTS, ALONE, LOADED, KT, FB, TB, WF, WT, WK, G, RING)                                                       \
+  GemmShape { SLOTS, ALONE, LOADED, KT, 32 * FB * WF, 32 * TB * WT, proj_gemm_kernel<false, KT, FB, TB, WF, WT, WK, G, RING>,  \
+              proj_gemm_kernel<true, KT, FB, TB, WF, WT, WK, G, RING> }
+const GemmShape kShapes[] = {
+    GL_GEMM(256, 1.20f, 2.00f, 64, 4, 2, 2, 4, 1, 1, 2),   // 256 x 256
+    GL_GEMM(512, 0.68f, 1.20f, 64, 2, 2, 2, 2, 2, 1, 2),   // 128 x 128, two per CU
+    GL_GEMM(256, 0.50f, 0.66f, 64, 2, 2, 2, 2, 2, 2, 4),   // 128 x 128
+    GL_GEMM(256, 0.34f, 0.43f, 128, 2, 1, 2, 2, 2, 2, 3),  // 128 x 64
+    GL_GEMM(256, 0.23f, 0.27f, 128, 1, 1, 2, 2, 2, 4, 5),  // 64 x 64
+};
+#undef GL_GEMM
+
+int tiles_of(const GemmCall& a, bool nn, const GemmShape& s) {
+  int ftiles = 0;
+  if (nn)
+    ftiles = (a.K + s.ft - 1) / s.ft;
+  else
+    for (int z = 0; z < a.n; ++z) ftiles += (a.j[z].n + s.ft - 1) / s.ft;
+  return ftiles * ((a.T + s.tt - 1) / s.tt);
 }
 
-int narrow_fwd_splits(int T, int total_feature_tiles) {
-  const int tiles = ((T + kGT - 1) / kGT) * total_feature_tiles;
-  int s = 1;
-  while (s < 4 && tiles * s * 2 <= 256) s *= 2;  // at least one workgroup per CU if it takes <= 4
-  return s;
-}
-
-int narrow_feature_tiles(int out_features) { return (out_features + kGT - 1) / kGT; }
-
-hipError_t launch_narrow_fwd(NarrowFwd a, hipStream_t st) {
-  const int ttiles = (a.T + kGT - 1) / kGT;
-  int total = 0;
-  for (int z = 0; z < a.n; ++z) {
-    a.j[z].first = total;
-    total += ttiles * narrow_feature_tiles(a.j[z].n) * a.nsplit;
+// The shape with the least estimated time: rounds of the CUs times the time
+// of a stage, which grows with the share of the chip at work (the clock falls
+// under load).
+int gemm_shape(const GemmCall& a, bool nn) {
+  int best = 0;
+  float best_t = 0.0f;
+  for (int i = 0; i < (int)(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
+    const GemmShape& s = kShapes[i];
+    const int tiles = tiles_of(a, nn, s), full = tiles / s.slots, rest = tiles % s.slots;
+    const float t = full * s.loaded + (rest > 0 ? s.alone + (s.loaded - s.alone) * rest / s.slots : 0.0f);
+    if (i == 0 || t < best_t) best = i, best_t = t;
   }
-  if (total == 0) return hipSuccess;
-  hipLaunchKernelGGL(proj_gemm_nt_kernel, dim3(total), dim3(kGThreads), 0, st, a);
+  return best;
+}
+
+hipError_t launch_gemm_shape(GemmCall a, bool nn, int shape, hipStream_t st) {
+  const GemmShape& s = kShapes[shape];
+  a.ftiles = 0;
+  if (nn) {
+    a.ftiles = (a.K + s.ft - 1) / s.ft;
+  } else {
+    for (int z = 0; z < a.n; ++z) {
+      a.j[z].first = a.ftiles;
+      a.ftiles += (a.j[z].n + s.ft - 1) / s.ft;
+    }
+  }
+  const int ttiles = (a.T + s.tt - 1) / s.tt;
+  if (ttiles == 0 || a.ftiles == 0) return hipSuccess;
+  hipLaunchKernelGGL(nn ? s.nn : s.nt, dim3(a.ftiles * ttiles), dim3(kGThreads), 0, st, a);
   return hipGetLastError();
 }
 
-bool wide_gemm_fits(int in_features, int out_features) {
-  return in_features % kWF == 0 && out_features % kWF == 0;
-}
+}  // namespace
 
-hipError_t launch_wide_fwd(const WideFwd& a, hipStream_t st) {
-  const int ttiles = (a.T + kWT - 1) / kWT, ftiles = a.n / kWF;
-  if (ttiles == 0 || ftiles == 0) return hipSuccess;
-  if (a.K % kWK != 0 || a.n % kWF != 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(proj_gemm_wide_nt_kernel, dim3(ttiles * ftiles), dim3(kWThreads), 0, st, a);
-  return hipGetLastError();
-}
-
-hipError_t launch_wide_bwd(const WideBwd& a, hipStream_t st) {
-  const int ttiles = (a.T + kWT - 1) / kWT, ftiles = a.K / kWF;
-  if (ttiles == 0 || ftiles == 0 || a.n == 0) return hipSuccess;
-  if (a.K % kWF != 0) return hipErrorInvalidValue;
-  for (int z = 0; z < a.n; ++z)
-    if (a.j[z].n % kWK != 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(proj_gemm_wide_nn_kernel, dim3(ttiles * ftiles), dim3(kWThreads), 0, st, a);
-  return hipGetLastError();
+hipError_t launch_gemm(GemmCall a, bool nn, hipStream_t st) {
+  return launch_gemm_shape(a, nn, gemm_shape(a, nn), st);
 }
 
 hipError_t launch_generic_fwd(const WideFwd& a, bool io_bf16, hipStream_t st) {
@@ -825,13 +676,6 @@ hipError_t launch_generic_bwd(const WideBwd& a, bool io_bf16, hipStream_t st) {
   if (ttiles == 0 || ftiles == 0 || a.n == 0) return hipSuccess;
   auto fn = io_bf16 ? proj_gemm_f32_kernel<bf16, true> : proj_gemm_f32_kernel<float, true>;
   hipLaunchKernelGGL(fn, dim3(ttiles * ftiles), dim3(kFThreads), 0, st, WideFwd{}, a);
-  return hipGetLastError();
-}
-
-hipError_t launch_narrow_bwd(const NarrowBwd& a, hipStream_t st) {
-  const int ttiles = (a.T + kGT - 1) / kGT, ftiles = (a.K + kGT - 1) / kGT;
-  if (ttiles == 0 || ftiles == 0) return hipSuccess;
-  hipLaunchKernelGGL(proj_gemm_nn_kernel, dim3(ttiles * ftiles), dim3(kGThreads), 0, st, a);
   return hipGetLastError();
 }
 

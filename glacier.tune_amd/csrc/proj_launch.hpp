@@ -33,85 +33,73 @@ struct ProjLaunch {
   ProjSpec p[kMaxProj];
   const void* x;  // [T][in]
   void* dx;       // [T][in] (backward; overwritten)
-  // scratch (fp32), sized by proj_scratch_need
-  float* yf;       // forward: [T][out_p] base products, one after another
-                   // ([nsplit][T][out_p] for a narrow projection of bf16 tensors)
-  float* dxf;      // backward: [T][in] sum_p dY_p W_p over the library-GEMM
-                   // projections, then [T][in] over the narrow ones
+  // scratch, sized by proj_scratch_need
   float* lowrank;  // [slot][T][r] X A_p and dY_p B_p^T
-  float* part;     // split sums of those products
+  void* terms;     // fused calls: the split terms (bf16) of the adapters, then of s L
+  int* odd;        // fused calls: non-finite marks (SplitCall)
+  float* yf;       // other calls, forward: [T][out_p] base products, one after another
+  float* dxf;      // other calls, backward: [T][in] sum_p dY_p W_p
+  float* part;     // other calls: split sums of the low-rank products
 };
 
-// ---- the narrow base products on the library's own GEMM (proj_gemm.hip) ----
-// bf16 tensors, inputs a multiple of 64 and at most kNarrowMaxOut outputs,
-// also a multiple of 64 (the k and v projections of a GQA block).
-constexpr int kNarrowMaxOut = 1024;
-
-struct NarrowJob {
-  const void* w;   // W_p [n][in] (bf16)
-  const void* dy;  // backward: dY_p [T][n] (bf16)
-  float* c;        // forward: fp32 partials [nsplit][T][n]
-  int n;           // outputs of the projection
-  int first;       // forward: its first workgroup (set by launch_narrow_fwd)
+// ---- bf16 tensors: base products, low-rank delta, bias and conversion in ----
+// one launch per direction (proj_gemm.hip)
+struct GemmSeg {  // a stretch of the reduction: k elements
+  const void* a;  // forward [n][k], backward [k][K] (bf16)
+  const void* b;  // [T][k] (bf16)
+  int k;          // a multiple of 8
 };
-
-// Yf_p[s] = X W_p^T over input slice s (kchunk inputs) for each job.
-struct NarrowFwd {
-  const void* x;  // [T][K] (bf16)
-  int T, K, nsplit, kchunk, n;
-  NarrowJob j[kMaxProj];
+struct GemmJob {
+  void* y;            // forward: Y_p [T][n] (bf16)
+  const float* bias;  // forward: [n] or null
+  const float* l;     // L_p (forward) or dL_p (backward) [T][r]; null: no adapter
+  const float* v;     // B_p [r][n] (forward) or A_p [K][r] (backward)
+  float s;            // the adapter's scaling
+  int n;              // outputs of the projection
+  int first;          // forward: its first feature tile (set by launch_gemm)
 };
-
-// dXf2 [T][K] = sum over the jobs of dY_p W_p (K = the input features).
-struct NarrowBwd {
-  int T, K;
-  float* c;
-  int n;
-  NarrowJob j[kMaxProj];
+struct GemmCall {
+  void* dx;         // backward: dX [T][K] (bf16)
+  const int* odd;   // [n_odd] marks: the low-rank operands hold non-finite values
+  int n_odd;
+  int T, K, rank, n;
+  int ftiles;       // set by launch_gemm
+  GemmJob j[kMaxProj];
+  GemmSeg seg[2 * kMaxProj];  // p: W_p with X (forward) or dY_p; kMaxProj + p: the adapter's split terms
 };
+// Elements of a row of split terms: six stretches of r, in whole 16-byte pieces.
+__host__ __device__ constexpr int term_pitch(int rank) { return (6 * rank + 7) / 8 * 8; }
+hipError_t launch_gemm(GemmCall a, bool backward, hipStream_t st);
 
-bool narrow_gemm_fits(int in_features, int out_features);
-// Input slices of a forward launch: 1, 2 or 4, so that the launch has about
-// a workgroup per CU when the tiles alone are fewer.
-int narrow_fwd_splits(int T, int total_feature_tiles);
-int narrow_feature_tiles(int out_features);
-hipError_t launch_narrow_fwd(NarrowFwd a, hipStream_t st);
-hipError_t launch_narrow_bwd(const NarrowBwd& a, hipStream_t st);
-
-// ---- the wide base products on the library's own GEMM (proj_gemm.hip) ----
-// bf16 tensors, inputs and outputs multiples of 128 (the q projection).
+// ---- the base products alone, fp32 results, for every other call ----
 struct WideJob {
-  const void* w;   // W_z [n][K] (bf16)
-  const void* dy;  // dY_z [T][n] (bf16)
+  const void* w;   // W_z [n][K]
+  const void* dy;  // dY_z [T][n]
   int n;           // outputs of the projection
 };
 // c [T][n] = X W^T (fp32), one projection.
 struct WideFwd {
-  const void* x;  // [T][K] (bf16)
-  const void* w;  // [n][K] (bf16)
+  const void* x;  // [T][K]
+  const void* w;  // [n][K]
   float* c;
   int T, K, n;
 };
-// c [T][K] = sum over the jobs of dY_z W_z (fp32); accumulate (generic
-// kernel only): c += instead.
+// c [T][K] = sum over the jobs of dY_z W_z (fp32)
 struct WideBwd {
   float* c;
   int T, K, n;
   WideJob j[kMaxProj];
-  bool accumulate;
 };
-bool wide_gemm_fits(int in_features, int out_features);
-hipError_t launch_wide_fwd(const WideFwd& a, hipStream_t st);
-hipError_t launch_wide_bwd(const WideBwd& a, hipStream_t st);
 
-// ---- every other projection: the same two products on fp32 MFMAs, any ----
-// shape, fp32 or bf16 operands (io_bf16) converted to fp32 on load
+// fp32 MFMAs, any shape, fp32 or bf16 operands (io_bf16) converted on load
 hipError_t launch_generic_fwd(const WideFwd& a, bool io_bf16, hipStream_t st);
 hipError_t launch_generic_bwd(const WideBwd& a, bool io_bf16, hipStream_t st);
 
-// Floats of each ProjLaunch scratch buffer for a forward or backward call.
+// Floats (unless stated) of each ProjLaunch scratch buffer for a forward or backward call.
 struct ProjScratchNeed {
   long yf, dxf, lowrank, part;
+  long terms;  // bf16 elements
+  long odd;    // ints
 };
 ProjScratchNeed proj_scratch_need(const ProjLaunch& a, bool backward);
 

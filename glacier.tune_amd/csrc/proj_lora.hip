@@ -10,19 +10,21 @@
 //   backward  dX   = sum_p dY_p W_p + s_p (dY_p B_p^T) A_p^T
 //             dA_p += s_p X^T (dY_p B_p^T),  dB_p += s_p (X A_p)^T dY_p
 //
-// The base products X W_p^T and dY_p W_p are GEMMs with fp32 results, all on
-// the library's own kernels (proj_gemm.hip): for bf16 tensors the narrow
-// GEMM (the k and v projections of a GQA block) and the wide one (q), and
-// for fp32 tensors or shapes neither takes, a generic fp32-MFMA GEMM.
-// Everything low-rank is here, each kernel taking every projection of the
-// call in one launch:
-//   lowrank_rows    L = X A_p and dL = dY_p B_p^T (output r columns wide,
-//                   reduction over in / out): 16-row slabs, the reduction
-//                   split over workgroups and over their 8 waves, fp32 MFMAs
+// bf16 tensors (every width a multiple of 8, 16-byte aligned): three launches
+// forward, four backward.
+//   lowrank_split   L = X A_p and dL = dY_p B_p^T, and the split terms
+//                   (split3.hpp) of s L and of the adapters
+//   lowrank_cols    backward: grad_A += s X^T dL, grad_B += s L^T dY (reduction
+//                   over the tokens): 64-column slabs, tokens split over 8 waves
+//   proj_gemm       (proj_gemm.hip) Y_p = X W_p^T + bias_p + (s L_p) B_p for
+//                   every projection, or dX = sum_p dY_p W_p + (s dL_p) A_p^T
+// Other calls (fp32 tensors, widths that are multiples of 4 only):
+//   proj_gemm_f32   the base products, fp32 results, one launch per projection
+//   lowrank_rows    L and dL: 16-row slabs, the reduction split over workgroups
+//                   and over their 8 waves, fp32 MFMAs
 //   lowrank_reduce  adds the workgroups' split sums in split order
-//   lowrank_cols    grad_A += s X^T dL, grad_B += s L^T dY (reduction over
-//                   the tokens): 64-column slabs, tokens split over 8 waves
-//   lowrank_out     Y_p = io(Yf_p + bias_p + (s L) B_p) and dX = io(dXf +
+//   lowrank_cols    as above
+//   lowrank_out     Y_p = io(Yf_p + bias_p + (s L_p) B_p) and dX = io(dXf +
 //                   sum_p (s dL_p) A_p^T): 16 x 256 tiles, the rank-r
 //                   product on MFMAs, fused with the dtype conversion
 // The adapters, the low-rank activations and the gradients stay fp32, as in
@@ -30,7 +32,9 @@
 // operands and the outputs.  Every reduction has a fixed order, so every
 // result is bitwise repeatable.
 #include "attn_common.hpp"
+#include "lds_mfma.hpp"
 #include "proj_launch.hpp"
+#include "split3.hpp"
 
 namespace glacier {
 namespace {
@@ -202,6 +206,240 @@ __global__ __launch_bounds__(256) void lowrank_reduce_kernel(const float* __rest
   dense[idx] = sum;
 }
 
+// ---- bf16 tensors: the low-rank products and their split terms ----------
+// L [T][r] = U [T][K] V for each job (V as in RowsJob), with U in bf16: V goes
+// onto the bf16 MFMAs in its three terms (split3.hpp), so every product is
+// exact and the sums are fp32, at 3/8 of the fp32 MFMA's time.  The results
+// go out as L in fp32 (lowrank_cols) and, where the job has `terms`, as the
+// split terms of s L, the B operand of the GEMM's low-rank segment; the last
+// kTermBlocks workgroups write the adapters' own terms, its A operand.  A row
+// of terms holds six stretches of r: the products of the same stretch of the
+// two operands are h h, h m, m h, m m, h l, l h.
+// Bound by the vector-memory unit (V is read a column at a time, 64-byte
+// pieces): 11-15 us at 512 x 3584 -> 3584/512/512 and 23-39 us at 4096 x 4096
+// -> 4096/1024/1024, rank 16, where the fp32 form with its separate reduction
+// took 14 and 38 us without forming the terms.
+struct SplitJob {
+  const void* u;  // [T][K] (bf16)
+  const float* v;
+  float* l;       // [T][r]
+  void* terms;    // [T][P] (bf16) or null
+  float s;        // the terms are those of s L
+  int K;
+  int vt;
+};
+// terms [n][P] of V [r][n] (across 0), or terms [P][n] of V [n][r] (across 1)
+struct TermJob {
+  const float* v;
+  void* terms;
+  int n;
+};
+struct SplitCall {
+  SplitJob j[kMaxJobs];
+  TermJob v[kMaxProj];
+  int n, nv, across;
+  int slabs;   // row slabs of a job
+  int* odd;    // [kTermBlocks], then [n][slabs]: a non-finite value among what that workgroup wrote
+};
+
+__device__ inline bool not_finite(float x) { return (__float_as_uint(x) & 0x7f800000u) == 0x7f800000u; }
+
+// The six entries of a terms row for x: side 0 the adapters', side 1 (s L).
+template <typename Put>
+__device__ inline void put_terms(float x, int side, Put&& put) {
+  const bf16 h = (bf16)x;
+  const float r1 = x - (float)h;
+  const bf16 m = (bf16)r1, l = (bf16)(r1 - (float)m);
+  put(0, h);
+  put(1, side ? m : h);
+  put(2, side ? h : m);
+  put(3, m);
+  put(4, side ? l : h);
+  put(5, side ? h : l);
+}
+
+// x has a split: its terms are finite (false also for a finite x that rounds
+// to infinity).
+[[maybe_unused]] __device__ inline bool has_split(float x) { return !not_finite((float)(bf16)x); }
+
+constexpr int kTermBlocks = 64;
+// Waves of a lowrank_split workgroup
+constexpr int split_waves(int nt, int rb) { return rb == 1 && nt % 2 == 1 ? 16 : 8; }
+
+#if defined(__HIP_DEVICE_COMPILE__)
+// The k range [kb, ke) of one wave of lowrank_split_kernel, added into acc.
+// Steps of 32: lane (i, q) holds U[row i][k0 + 8q .. +7] and V[k0 + 8q ..
+// +7][16 jt + i].  K % 8 == 0, so a lane's 8 are all in or all out; out of
+// range V is zeroed, U clamped (and finite, or the step goes the fp32 way,
+// where U is zeroed as well).
+template <int NT, int RB, bool VT>
+__device__ inline void split_accumulate(const bf16* const (&u)[RB], const float* __restrict__ v0, int K,
+                                        int rank, int kb, int ke, f32x4 (&acc)[RB][NT]) {
+  const int lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
+  constexpr int CH = NT * RB <= 2 ? 4 : NT * RB <= 8 ? 2 : 1;  // steps whose loads are issued together
+  for (int k0 = kb; k0 < ke; k0 += 32 * CH) {
+    bf16x8 ur[CH][RB];
+    float vr[CH][NT][8];
+#pragma unroll
+    for (int s = 0; s < CH; ++s) {
+      const int kc = min(k0 + 32 * s + 8 * q, K - 8);
+#pragma unroll
+      for (int b = 0; b < RB; ++b) ur[s][b] = *reinterpret_cast<const bf16x8*>(u[b] + kc);
+#pragma unroll
+      for (int jt = 0; jt < NT; ++jt) {
+        const int jc = min(16 * jt + i, rank - 1);
+        if constexpr (VT) {
+          load8(v0 + (long)jc * K + kc, vr[s][jt]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) vr[s][jt][e] = v0[(long)(kc + e) * rank + jc];
+        }
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < CH; ++s) {
+      if (k0 + 32 * s >= ke) break;
+      const bool k_ok = k0 + 32 * s + 8 * q < ke;
+      float chk = 0.0f;  // NaN once an element of U is not finite
+#pragma unroll
+      for (int b = 0; b < RB; ++b)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) chk += 0.0f * (float)ur[s][b][e];
+#pragma unroll
+      for (int jt = 0; jt < NT; ++jt) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) vr[s][jt][e] = k_ok ? vr[s][jt][e] : 0.0f;
+        Split3 v;
+        const bool bad = v.set(vr[s][jt]) || chk != chk;
+        if (__any(bad)) {
+#pragma unroll
+          for (int b = 0; b < RB; ++b)
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              acc[b][jt] = mma_f32(k_ok ? (float)ur[s][b][e] : 0.0f, vr[s][jt][e], acc[b][jt]);
+        } else {
+#pragma unroll
+          for (int b = 0; b < RB; ++b) {
+            acc[b][jt] = Mfma<bf16>::mma(ur[s][b], v.l, acc[b][jt]);
+            acc[b][jt] = Mfma<bf16>::mma(ur[s][b], v.m, acc[b][jt]);
+            acc[b][jt] = Mfma<bf16>::mma(ur[s][b], v.h, acc[b][jt]);
+          }
+        }
+      }
+    }
+  }
+}
+#endif
+
+template <int NT, int RB>
+__global__ __launch_bounds__(64 * split_waves(NT, RB)) void lowrank_split_kernel(const SplitCall a, int T,
+                                                                             int rank) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int W = split_waves(NT, RB);  // waves, splitting K
+  constexpr int kRow = 16 * NT + 1;
+  __shared__ float red[W * 16 * RB * kRow];
+  const int P = term_pitch(rank);
+  bool odd = false;
+  const int rows_blocks = a.n * a.slabs;
+  if ((int)blockIdx.x >= rows_blocks) {
+    // the adapters' terms: four ranks of one feature a thread, its loads
+    // together (tied, so that none sinks under the bounds tests below),
+    // features consecutive over the threads
+    const int chunks = (rank + 3) / 4;
+    int total = 0;
+    for (int p = 0; p < a.nv; ++p) total += a.v[p].n * chunks;
+    for (int g = ((int)blockIdx.x - rows_blocks) * (64 * W) + (int)threadIdx.x; g < total;
+         g += kTermBlocks * 64 * W) {
+      int p = 0, idx = g;
+      while (idx >= a.v[p].n * chunks) idx -= a.v[p++].n * chunks;
+      const float* v = a.v[p].v;
+      bf16* out = static_cast<bf16*>(a.v[p].terms);
+      const int n = a.v[p].n, f = idx % n, j0 = 4 * (idx / n);
+      float x[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const int j = min(j0 + m, rank - 1);
+        x[m] = v[a.across ? (long)f * rank + j : (long)j * n + f];
+      }
+#pragma unroll
+      for (int m = 0; m < 4; ++m) tie_v(x[m]);
+      if (!a.across && rank % 4 == 0) {  // four entries of a row in one store
+        bf16x4 t4[6];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          odd |= !has_split(x[m]);
+          put_terms(x[m], 0, [&](int e, bf16 t) { t4[e][m] = t; });
+        }
+#pragma unroll
+        for (int e = 0; e < 6; ++e) *reinterpret_cast<bf16x4*>(out + (long)f * P + e * rank + j0) = t4[e];
+      } else {
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          if (j0 + m >= rank) break;
+          odd |= !has_split(x[m]);
+          put_terms(x[m], 0, [&](int e, bf16 t) {
+            const int q = e * rank + j0 + m;
+            out[a.across ? (long)q * n + f : (long)f * P + q] = t;
+          });
+        }
+      }
+      if (j0 == 0)
+        for (int q = 6 * rank; q < P; ++q) out[a.across ? (long)q * n + f : (long)f * P + q] = (bf16)0.0f;
+    }
+    odd = __syncthreads_or(odd);
+    if (threadIdx.x == 0) a.odd[(int)blockIdx.x - rows_blocks] = odd;
+    return;
+  }
+  const int z = (int)blockIdx.x / a.slabs, slab = (int)blockIdx.x % a.slabs;
+  const SplitJob& job = a.j[z];
+  const int K = job.K;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int i = lane & 15, q = lane >> 4;
+  const int t0 = slab * 16 * RB;
+  const bf16* u[RB];
+#pragma unroll
+  for (int b = 0; b < RB; ++b)
+    u[b] = static_cast<const bf16*>(job.u) + (long)min(t0 + 16 * b + i, T - 1) * K;
+  int kb, ke;
+  share(K, W, wave, 32, kb, ke);
+  f32x4 acc[RB][NT];
+#pragma unroll
+  for (int b = 0; b < RB; ++b)
+#pragma unroll
+    for (int jt = 0; jt < NT; ++jt) acc[b][jt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  if (job.vt)
+    split_accumulate<NT, RB, true>(u, job.v, K, rank, kb, ke, acc);
+  else
+    split_accumulate<NT, RB, false>(u, job.v, K, rank, kb, ke, acc);
+  // D of (b, jt): lane (i, q), register c holds row 16 b + 4q + c, column 16 jt + i
+#pragma unroll
+  for (int b = 0; b < RB; ++b)
+#pragma unroll
+    for (int jt = 0; jt < NT; ++jt)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        red[(wave * 16 * RB + 16 * b + 4 * q + c) * kRow + 16 * jt + i] = acc[b][jt][c];
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < 16 * RB * 16 * NT; idx += 64 * W) {
+    const int r = idx / (16 * NT), j = idx % (16 * NT), t = t0 + r;
+    if (t >= T || j >= rank) continue;
+    float sum = 0.0f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) sum += red[(w * 16 * RB + r) * kRow + j];
+    job.l[(long)t * rank + j] = sum;
+    if (job.terms == nullptr) continue;
+    bf16* row = static_cast<bf16*>(job.terms) + (long)t * P;
+    const float x = job.s * sum;
+    odd |= !has_split(x);
+    put_terms(x, 1, [&](int e, bf16 v) { row[e * rank + j] = v; });
+    if (j == 0)
+      for (int e = 6 * rank; e < P; ++e) row[e] = (bf16)0.0f;
+  }
+  odd = __syncthreads_or(odd);
+  if (threadIdx.x == 0) a.odd[kTermBlocks + (int)blockIdx.x] = odd;
+#endif
+}
+
 // One product Out (+)= alpha U^T W of lowrank_cols: U [T][cols] in the call's
 // dtype, W [T][r] fp32; Out [cols][r] or, transposed, [r][cols];
 // workgroups first .. first + ceil(cols / 64) - 1.
@@ -307,8 +545,6 @@ struct OutJob {
   const float* l[kMaxProj];
   const float* v[kMaxProj];
   float s[kMaxProj];
-  int nbase = 1;      // base products summed in order: base + i * stride, i < nbase
-  long stride = 0;
 };
 struct OutJobs {
   OutJob j[kMaxProj];
@@ -338,12 +574,6 @@ __global__ __launch_bounds__(kOutThreads) void lowrank_out_kernel(OutJobs jobs, 
 #pragma unroll
   for (int c = 0; c < 4; ++c)
     base[c] = *reinterpret_cast<const f32x4*>(job.base + (long)min(t0 + 4 * q + c, T - 1) * n + colc);
-  for (int i = 1; i < job.nbase; ++i) {  // split partials, in order
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      base[c] += *reinterpret_cast<const f32x4*>(job.base + i * job.stride +
-                                                 (long)min(t0 + 4 * q + c, T - 1) * n + colc);
-  }
   f32x4 acc[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) acc[e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -480,23 +710,93 @@ hipError_t run_out(const ProjLaunch& a, OutJobs& jobs, hipStream_t st) {
   return hipGetLastError();
 }
 
-const float* slot(const ProjLaunch& a, int z) { return a.lowrank + (long)z * a.T * a.rank; }
+float* slot(const ProjLaunch& a, int z) { return a.lowrank + (long)z * a.T * a.rank; }
 
-// Which projections of a call take the narrow GEMM, which the wide one; the
-// rest (fp32 tensors, shapes neither covers) take the generic one.
-bool is_narrow(const ProjLaunch& a, int p) {
-  return a.io_bf16 && narrow_gemm_fits(a.in, a.p[p].out);
-}
-bool is_wide(const ProjLaunch& a, int p) {
-  return a.io_bf16 && !is_narrow(a, p) && wide_gemm_fits(a.in, a.p[p].out);
+// Row blocks (of 16) per lowrank_split workgroup: V is read once per
+// workgroup, U once per job, so taller slabs save V's reads while the
+// launch still fills the CUs.
+int split_row_blocks(int T, int jobs, int nt) {
+  if (nt <= 2 && (T + 63) / 64 * jobs >= 128) return 4;
+  if ((T + 31) / 32 * jobs >= 128) return 2;
+  return 1;
 }
 
-// Input slices of the narrow forward launch (1 when there is none).
-int fwd_splits(const ProjLaunch& a) {
-  int tiles = 0;
+// Calls whose tensors the fused GEMM (proj_gemm.hip) takes: bf16, whole
+// 16-byte pieces in every row, 16-byte aligned tensors.  The others (fp32
+// tensors, widths that are multiples of 4 only) form the base products in
+// fp32 and add the rest in lowrank_out.
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+bool fused(const ProjLaunch& a, bool backward) {
+  if (!a.io_bf16 || a.in % 8 != 0 || !aligned16(a.x) || (backward && !aligned16(a.dx))) return false;
   for (int p = 0; p < a.n_proj; ++p)
-    if (is_narrow(a, p)) tiles += narrow_feature_tiles(a.p[p].out);
-  return tiles == 0 ? 1 : narrow_fwd_splits(a.T, tiles);
+    if (a.p[p].out % 8 != 0 || !aligned16(a.p[p].w) || !aligned16(backward ? a.p[p].dy : a.p[p].y)) return false;
+  return true;
+}
+
+hipError_t run_cols_any(const ProjLaunch& a, const RowsPlan& plan, hipStream_t st);
+
+// The fused form: the low-rank products and the split terms, then (backward)
+// the adapters' gradients, then one GEMM launch for everything else.
+hipError_t fused_impl(const ProjLaunch& a, bool backward, hipStream_t st) {
+  const RowsPlan plan = rows_plan(a, backward);
+  const int P = term_pitch(a.rank), nt = (a.rank + 15) / 16;
+  GemmCall g{};
+  g.dx = a.dx;
+  g.T = a.T;
+  g.K = a.in;
+  g.rank = a.rank;
+  g.n = a.n_proj;
+  bf16* vt = static_cast<bf16*>(a.terms);  // the adapters' terms, one after another
+  bf16* lt = vt;                           // then those of s L, [T][P] each
+  for (int p = 0; p < a.n_proj; ++p)
+    if (a.p[p].a != nullptr) lt += (long)P * (backward ? a.in : a.p[p].out);
+  SplitCall c{};
+  c.across = backward;
+  c.odd = a.odd;
+  for (int p = 0; p < a.n_proj; ++p) {
+    const ProjSpec& s = a.p[p];
+    g.j[p] = GemmJob{s.y, s.bias, nullptr, nullptr, s.scaling, s.out, 0};
+    g.seg[p] = GemmSeg{s.w, backward ? s.dy : a.x, backward ? s.out : a.in};
+    const int slot_l = backward ? plan.slot_dl[p] : plan.slot_l[p];
+    if (slot_l < 0) continue;
+    g.j[p].l = slot(a, slot_l);
+    g.j[p].v = backward ? s.a : s.b;
+    g.seg[kMaxProj + p] = GemmSeg{vt, lt, P};
+    const int n = backward ? a.in : s.out;
+    c.v[c.nv++] = TermJob{g.j[p].v, vt, n};
+    const RowsJob& r = plan.jobs.j[slot_l];
+    c.j[slot_l] = SplitJob{r.u, r.v, slot(a, slot_l), lt, s.scaling, r.K, r.vt};
+    vt += (long)P * n;
+    lt += (long)a.T * P;
+  }
+  if (backward)
+    for (int p = 0; p < a.n_proj; ++p)
+      if (const int z = plan.slot_l[p]; z >= 0) {
+        const RowsJob& r = plan.jobs.j[z];
+        c.j[z] = SplitJob{r.u, r.v, slot(a, z), nullptr, 0.0f, r.K, r.vt};
+      }
+  c.n = plan.n;
+  if (plan.n > 0) {
+    const int rb = split_row_blocks(a.T, plan.n, nt);
+    c.slabs = (a.T + 16 * rb - 1) / (16 * rb);
+    const dim3 grid(c.n * c.slabs + kTermBlocks), block(64 * split_waves(nt, rb));
+    switch (8 * rb + nt) {
+#define GL_SPLIT(RB, NT)                                                                                \
+  case 8 * RB + NT:                                                                                     \
+    hipLaunchKernelGGL((lowrank_split_kernel<NT, RB>), grid, block, 0, st, c, a.T, a.rank); \
+    break;
+      GL_SPLIT(1, 1) GL_SPLIT(1, 2) GL_SPLIT(1, 3) GL_SPLIT(1, 4)
+      GL_SPLIT(2, 1) GL_SPLIT(2, 2) GL_SPLIT(2, 3) GL_SPLIT(2, 4)
+      GL_SPLIT(4, 1) GL_SPLIT(4, 2)
+#undef GL_SPLIT
+      default: return hipErrorInvalidValue;
+    }
+    GL_CHECK(hipGetLastError());
+    g.odd = a.odd;
+    g.n_odd = kTermBlocks + c.n * c.slabs;
+  }
+  if (backward) GL_CHECK(run_cols_any(a, plan, st));
+  return launch_gemm(g, backward, st);
 }
 
 template <typename IO>
@@ -504,32 +804,13 @@ hipError_t forward_impl(const ProjLaunch& a, hipStream_t st) {
   long off = 0;
   OutJobs out{};
   out.n = a.n_proj;
-  NarrowFwd nf{};
-  nf.x = a.x;
-  nf.T = a.T;
-  nf.K = a.in;
-  nf.nsplit = fwd_splits(a);
-  nf.kchunk = (a.in + 64 * nf.nsplit - 1) / (64 * nf.nsplit) * 64;
   for (int p = 0; p < a.n_proj; ++p) {
     const ProjSpec& s = a.p[p];
     out.j[p] = OutJob{a.yf + off, s.bias, s.y, s.out, 0, 0, {}, {}, {}};
-    if (is_narrow(a, p)) {
-      // Yf_p[i] = X W_p^T over input slice i, summed by lowrank_out
-      nf.j[nf.n++] = NarrowJob{s.w, nullptr, a.yf + off, s.out, 0};
-      out.j[p].nbase = nf.nsplit;
-      out.j[p].stride = (long)a.T * s.out;
-      off += (long)nf.nsplit * a.T * s.out;
-    } else if (is_wide(a, p)) {
-      // Yf_p = X W_p^T on the library's own wide GEMM
-      GL_CHECK(launch_wide_fwd(WideFwd{a.x, s.w, a.yf + off, a.T, a.in, s.out}, st));
-      off += (long)a.T * s.out;
-    } else {
-      // Yf_p = X W_p^T on the generic GEMM
-      GL_CHECK(launch_generic_fwd(WideFwd{a.x, s.w, a.yf + off, a.T, a.in, s.out}, a.io_bf16, st));
-      off += (long)a.T * s.out;
-    }
+    // Yf_p = X W_p^T
+    GL_CHECK(launch_generic_fwd(WideFwd{a.x, s.w, a.yf + off, a.T, a.in, s.out}, a.io_bf16, st));
+    off += (long)a.T * s.out;
   }
-  if (nf.n > 0) GL_CHECK(launch_narrow_fwd(nf, st));
   const RowsPlan plan = rows_plan(a, false);
   GL_CHECK(run_rows<IO>(a, plan, st));  // L_p = X A_p
   for (int p = 0; p < a.n_proj; ++p) {
@@ -543,37 +824,9 @@ hipError_t forward_impl(const ProjLaunch& a, hipStream_t st) {
   return run_out<IO, false>(a, out, st);  // Y_p = io(Yf_p + bias_p + (s L_p) B_p)
 }
 
+// grad_A_p += s X^T dL_p;  grad_B_p += s L_p^T dY_p
 template <typename IO>
-hipError_t backward_impl(const ProjLaunch& a, hipStream_t st) {
-  // dXf = sum_p dY_p W_p: the wide projections (one launch over all of
-  // them), then the generic ones (one launch, adding to the wide sum) into
-  // dxf, the narrow ones into the buffer after it; lowrank_out adds the two
-  NarrowBwd nb{};
-  nb.T = a.T;
-  nb.K = a.in;
-  nb.c = a.dxf + (long)a.T * a.in;
-  WideBwd wb{}, gb{};
-  wb.c = gb.c = a.dxf;
-  wb.T = gb.T = a.T;
-  wb.K = gb.K = a.in;
-  for (int p = 0; p < a.n_proj; ++p) {
-    const ProjSpec& s = a.p[p];
-    if (is_narrow(a, p))
-      nb.j[nb.n++] = NarrowJob{s.w, s.dy, nullptr, s.out, 0};
-    else if (is_wide(a, p))
-      wb.j[wb.n++] = WideJob{s.w, s.dy, s.out};
-    else
-      gb.j[gb.n++] = WideJob{s.w, s.dy, s.out};
-  }
-  if (wb.n > 0) GL_CHECK(launch_wide_bwd(wb, st));
-  gb.accumulate = wb.n > 0;
-  if (gb.n > 0) GL_CHECK(launch_generic_bwd(gb, a.io_bf16, st));
-  const int wide = wb.n + gb.n;  // products written into dxf
-  if (nb.n > 0) GL_CHECK(launch_narrow_bwd(nb, st));
-  // dL_p = dY_p B_p^T, and L_p = X A_p where grad_B_p is wanted
-  const RowsPlan plan = rows_plan(a, true);
-  GL_CHECK(run_rows<IO>(a, plan, st));
-  // grad_A_p += s X^T dL_p;  grad_B_p += s L_p^T dY_p
+hipError_t run_cols(const ProjLaunch& a, const RowsPlan& plan, hipStream_t st) {
   ColsJobs cj{};
   int total = 0;
   for (int p = 0; p < a.n_proj; ++p) {
@@ -601,15 +854,31 @@ hipError_t backward_impl(const ProjLaunch& a, hipStream_t st) {
     }
     GL_CHECK(hipGetLastError());
   }
+  return hipSuccess;
+}
+
+hipError_t run_cols_any(const ProjLaunch& a, const RowsPlan& plan, hipStream_t st) {
+  return a.io_bf16 ? run_cols<bf16>(a, plan, st) : run_cols<float>(a, plan, st);
+}
+
+template <typename IO>
+hipError_t backward_impl(const ProjLaunch& a, hipStream_t st) {
+  // dXf = sum_p dY_p W_p in one launch
+  WideBwd gb{};
+  gb.c = a.dxf;
+  gb.T = a.T;
+  gb.K = a.in;
+  for (int p = 0; p < a.n_proj; ++p) gb.j[gb.n++] = WideJob{a.p[p].w, a.p[p].dy, a.p[p].out};
+  GL_CHECK(launch_generic_bwd(gb, a.io_bf16, st));
+  // dL_p = dY_p B_p^T, and L_p = X A_p where grad_B_p is wanted
+  const RowsPlan plan = rows_plan(a, true);
+  GL_CHECK(run_rows<IO>(a, plan, st));
+  GL_CHECK(run_cols<IO>(a, plan, st));
   // dX = io(dXf + sum_p (s dL_p) A_p^T)
   OutJobs out{};
   out.n = 1;
   OutJob& o = out.j[0];
-  o = OutJob{wide > 0 ? a.dxf : nb.c, nullptr, a.dx, a.in, 0, 0, {}, {}, {}};
-  if (wide > 0 && nb.n > 0) {
-    o.nbase = 2;
-    o.stride = (long)a.T * a.in;
-  }
+  o = OutJob{a.dxf, nullptr, a.dx, a.in, 0, 0, {}, {}, {}};
   for (int p = 0; p < a.n_proj; ++p) {
     if (plan.slot_dl[p] < 0) continue;
     o.l[o.n_terms] = slot(a, plan.slot_dl[p]);
@@ -624,29 +893,33 @@ hipError_t backward_impl(const ProjLaunch& a, hipStream_t st) {
 
 ProjScratchNeed proj_scratch_need(const ProjLaunch& a, bool backward) {
   ProjScratchNeed need{};
-  bool narrow = false;
-  for (int p = 0; p < a.n_proj; ++p) narrow = narrow || is_narrow(a, p);
-  if (backward) {
-    need.dxf = (long)a.T * a.in * (narrow ? 2 : 1);
-  } else {
-    const int splits = fwd_splits(a);
-    for (int p = 0; p < a.n_proj; ++p)
-      need.yf += (long)a.T * a.p[p].out * (is_narrow(a, p) ? splits : 1);
-  }
+  const bool f = fused(a, backward);
+  if (!f && backward) need.dxf = (long)a.T * a.in;
+  if (!f && !backward)
+    for (int p = 0; p < a.n_proj; ++p) need.yf += (long)a.T * a.p[p].out;
   const RowsPlan plan = rows_plan(a, backward);
   if (plan.n > 0) {
-    const long slabs = (a.T + 15) / 16, nt = (a.rank + 15) / 16;
     need.lowrank = (long)plan.n * a.T * a.rank;
-    need.part = (long)plan.n * rows_splits(a, plan) * slabs * 256 * nt;
+    if (f) {
+      need.odd = kTermBlocks + (long)plan.n * ((a.T + 15) / 16);
+      for (int p = 0; p < a.n_proj; ++p)
+        if (a.p[p].a != nullptr)
+          need.terms += (long)term_pitch(a.rank) * (a.T + (backward ? a.in : a.p[p].out));
+    } else {
+      const long slabs = (a.T + 15) / 16, nt = (a.rank + 15) / 16;
+      need.part = (long)plan.n * rows_splits(a, plan) * slabs * 256 * nt;
+    }
   }
   return need;
 }
 
 hipError_t launch_proj_forward(const ProjLaunch& a, hipStream_t st) {
+  if (fused(a, false)) return fused_impl(a, false, st);
   return a.io_bf16 ? forward_impl<bf16>(a, st) : forward_impl<float>(a, st);
 }
 
 hipError_t launch_proj_backward(const ProjLaunch& a, hipStream_t st) {
+  if (fused(a, true)) return fused_impl(a, true, st);
   return a.io_bf16 ? backward_impl<bf16>(a, st) : backward_impl<float>(a, st);
 }
 

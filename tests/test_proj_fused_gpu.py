@@ -1,0 +1,146 @@
+"""The projections' fused path for bf16 tensors (proj_gemm.hip,
+lowrank_split in proj_lora.hip) at the edges of its tiles, against float64
+products of the same bf16 operands on the GPU.
+
+Bound per element: the result's rounding to bf16 (8 significant bits with the
+implicit one: neighbours are 2^-7 apart relative to the lower power of two,
+so half of that, 2^-8 relative) plus fp32
+summation over n terms, n 2^-24 sum |terms| in the worst case; the sums
+round to both sides, so sqrt(n) 2^-22 sum |terms| holds with room, and the
+low-rank operands enter with all 24 bits (split3.hpp) within the same bound.
+"""
+import sys
+
+import pytest
+
+import glacier_attn as ga
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def engine():
+    assert torch.cuda.is_available(), "GPU tests need a ROCm GPU"
+    with ga.GpuAttentionEngine(0, ga.PREC_BF16) as e:
+        yield e
+
+
+def _problem(T, n_in, outs, rank, seed=3, w_shift=0):
+    """w_shift: elements by which each W misses its allocation's alignment."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    x = rnd(T, n_in).bfloat16()
+    projs = []
+    for i, o in enumerate(outs):
+        w = torch.empty(o * n_in + w_shift, device="cuda", dtype=torch.bfloat16)[w_shift:]
+        w = w.view(o, n_in).copy_(rnd(o, n_in) * n_in ** -0.5)
+        p = {"w": w, "bias": 0.1 * rnd(o), "dy": rnd(T, o).bfloat16(), "scaling": 2.0}
+        if i != 1:  # the second projection has no adapter
+            p.update(a=rnd(n_in, rank) * n_in ** -0.5, b=0.1 * rnd(rank, o))
+            p.update(grad_a=torch.zeros_like(p["a"]), grad_b=torch.zeros_like(p["b"]))
+        projs.append(p)
+    return x, projs
+
+
+def _reference(x, projs):
+    """(value, sum of |terms|) of each y and of dx, in float64."""
+    x = x.double()
+    ys, dx = [], [0.0, 0.0]
+    for p in projs:
+        w, dy = p["w"].double(), p["dy"].double()
+        y, bound = x @ w.t() + p["bias"].double(), x.abs() @ w.abs().t() + p["bias"].double().abs()
+        d, d_bound = dy @ w, dy.abs() @ w.abs()
+        if "a" in p:
+            a, b, s = p["a"].double(), p["b"].double(), p["scaling"]
+            y, bound = y + s * (x @ a) @ b, bound + s * (x.abs() @ a.abs()) @ b.abs()
+            d, d_bound = d + s * (dy @ b.t()) @ a.t(), d_bound + s * (dy.abs() @ b.abs().t()) @ a.abs().t()
+        ys.append((y, bound))
+        dx = [dx[0] + d, dx[1] + d_bound]
+    return ys, tuple(dx)
+
+
+def _check(got, want, terms, n, what):
+    err = (got.double() - want).abs()
+    bound = 2.0 ** -8 * want.abs() + n ** 0.5 * 2.0 ** -22 * terms
+    worst = float((err / bound).max())
+    print(f"  {what}: worst error {worst:.2f} of its bound", flush=True)
+    assert worst <= 1.0
+
+
+SHAPES = [  # T, in, outs, rank
+    (1, 8, (8,), 1),                       # one piece of one row
+    (37, 1000, (1000, 200, 200), 5),       # reduction tails, padded term rows
+    (65, 72, (264, 8), 64),                # a token past the tile, the largest rank
+    (129, 136, (128, 72, 136), 17),        # a second rank tile
+    (512, 3584, (3584, 512, 512), 16),
+    (640, 2056, (1032, 1032), 8),
+    (1290, 520, (2056, 136), 33),
+    (2051, 1024, (2048, 520, 264), 16),    # taller low-rank slabs
+    (4099, 256, (4104,), 12),              # the largest tiles, ragged in both directions
+]
+
+
+@pytest.mark.parametrize("T,n_in,outs,rank", SHAPES)
+def test_fused_projection_matches_float64(engine, T, n_in, outs, rank):
+    print(f"[fused proj] T={T} in={n_in} outs={outs} rank={rank}", flush=True)
+    sys.stdout.flush()
+    x, projs = _problem(T, n_in, outs, rank)
+    ys = engine.proj_forward(x, projs, rank)
+    dx = engine.proj_backward(x, projs, rank)
+    want, want_dx = _reference(x, projs)
+    for i, (y, (ref, terms)) in enumerate(zip(ys, want)):
+        _check(y, ref, terms, n_in, f"y{i}")
+    _check(dx, *want_dx, sum(outs), "dx")
+    xd = x.double()
+    for p in projs:
+        if "a" not in p:
+            continue
+        dl, l = p["dy"].double() @ p["b"].double().t(), xd @ p["a"].double()
+        for got, ref in ((p["grad_a"], 2.0 * xd.t() @ dl), (p["grad_b"], 2.0 * l.t() @ p["dy"].double())):
+            assert float((got.double() - ref).norm() / ref.norm()) <= 2e-6  # fp32 sums
+
+
+def test_unaligned_weights_take_the_general_path(engine):
+    """The DMA moves aligned 16-byte pieces; weights that are not stay with
+    the general kernels and give the same products."""
+    x, projs = _problem(70, 136, (72, 136), 8, w_shift=4)
+    assert projs[0]["w"].data_ptr() % 16 != 0
+    ys = engine.proj_forward(x, projs, 8)
+    dx = engine.proj_backward(x, projs, 8)
+    want, want_dx = _reference(x, projs)
+    for y, (ref, terms) in zip(ys, want):
+        _check(y, ref, terms, 136, "y")
+    _check(dx, *want_dx, 208, "dx")
+
+
+@pytest.mark.parametrize("where", ["x", "a", "b", "dy", "huge_b"])
+def test_non_finite_values_pass_through(engine, where):
+    """Infinities, NaN and values past bf16's range have no split terms: the
+    results hold inf and NaN exactly where float32 arithmetic does, and every
+    other element is unharmed."""
+    T, n_in, outs, rank = 70, 136, (72, 64), 8
+    x, projs = _problem(T, n_in, outs, rank)
+    p = projs[0]
+    if where == "x":
+        x[5, 7], x[9, 3] = float("inf"), float("nan")
+    elif where == "a":
+        p["a"][11, 2], p["a"][12, 3] = float("-inf"), float("nan")
+    elif where == "b":
+        p["b"][1, 20], p["b"][2, 21] = float("inf"), float("nan")
+    elif where == "dy":
+        p["dy"][6, 8] = float("inf")
+    else:
+        p["b"][1, 20] = 3.4e38  # rounds to infinity in bf16
+        for t in (x, p["dy"]):  # and whose products stay inside float32
+            t.mul_(1.0e-3)
+    ys = engine.proj_forward(x, projs, rank)
+    dx = engine.proj_backward(x, projs, rank)
+    want, want_dx = _reference(x, projs)
+    for got, (ref, terms) in zip([*ys, dx], [*want, want_dx]):
+        ref32 = ref.float().bfloat16()
+        assert torch.equal(torch.isnan(got), torch.isnan(ref32))
+        assert torch.equal(torch.isinf(got), torch.isinf(ref32))
+        ok = torch.isfinite(ref32) & torch.isfinite(terms)
+        if ok.any():
+            _check(got[ok], ref[ok], terms[ok], n_in, where)
