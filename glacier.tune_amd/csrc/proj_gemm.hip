@@ -16,7 +16,7 @@ namespace {
 // on one XCD keeps the workgroups that share operand tiles (tile_of) on one
 // L2: each XCD then fetches only its own share of the weights, instead of
 // every XCD fetching all of them.
-__device__ inline int xcd_logical(int id, int total) {
+[[maybe_unused]] __device__ inline int xcd_logical(int id, int total) {
   constexpr int kXcds = 8;
   const int q = total / kXcds, r = total % kXcds, x = id % kXcds;
   return x * q + min(x, r) + id / kXcds;
@@ -109,6 +109,40 @@ constexpr int block_owner(int fb, int tb) {
   else
     return 0;
 }
+
+#if defined(__HIP_DEVICE_COMPILE__)
+// WK == 2: each group hands the other the blocks that one finishes, and adds
+// its own to what it receives.  All of the workgroup is past its last use of
+// lds; barriers on both sides.
+template <int FB, int TB, int WK>
+__device__ inline void merge_groups(f32x16 (&acc)[FB][TB], unsigned char* lds, int place, int wk, int lane) {
+  if constexpr (WK == 2) {
+    f32x4* ex = reinterpret_cast<f32x4*>(lds) + place * (FB * TB * 256);
+#pragma unroll
+    for (int fb = 0; fb < FB; ++fb)
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb)
+        if (block_owner<FB, TB, WK>(fb, tb) != wk)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            ex[(fb * TB + tb) * 256 + q * 64 + lane] =
+                f32x4{acc[fb][tb][4 * q], acc[fb][tb][4 * q + 1], acc[fb][tb][4 * q + 2], acc[fb][tb][4 * q + 3]};
+    __syncthreads();
+#pragma unroll
+    for (int fb = 0; fb < FB; ++fb)
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb)
+        if (block_owner<FB, TB, WK>(fb, tb) == wk)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const f32x4 o = ex[(fb * TB + tb) * 256 + q * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[fb][tb][4 * q + e] += o[e];
+          }
+    __syncthreads();
+  }
+}
+#endif
 
 template <bool NN, int KT, int FB, int TB, int WF, int WT, int WK, int G, int RING>
 __global__ __launch_bounds__(kGThreads) void proj_gemm_kernel(const GemmCall a) {
@@ -362,35 +396,9 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_kernel(const GemmCall a) 
       if (++st < nst) stage(st, std::integral_constant<int, 1>{});
   }
 
-  // Epilogue.  WK == 2: each group hands the other the blocks that one
-  // finishes, and adds its own to what it receives (group 0's first).
   __syncthreads();
-  if constexpr (WK == 2) {
-    f32x4* ex = reinterpret_cast<f32x4*>(lds) + (w % (WF * WT)) * (FB * TB * 256);
-#pragma unroll
-    for (int fb = 0; fb < FB; ++fb)
-#pragma unroll
-      for (int tb = 0; tb < TB; ++tb)
-        if (block_owner<FB, TB, WK>(fb, tb) != wk)
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            ex[(fb * TB + tb) * 256 + q * 64 + lane] =
-                f32x4{acc[fb][tb][4 * q], acc[fb][tb][4 * q + 1], acc[fb][tb][4 * q + 2], acc[fb][tb][4 * q + 3]};
-    __syncthreads();
-#pragma unroll
-    for (int fb = 0; fb < FB; ++fb)
-#pragma unroll
-      for (int tb = 0; tb < TB; ++tb)
-        if (block_owner<FB, TB, WK>(fb, tb) == wk)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const f32x4 o = ex[(fb * TB + tb) * 256 + q * 64 + lane];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[fb][tb][4 * q + e] += o[e];
-          }
-    __syncthreads();
-  }
-  // bias, bf16, and out through LDS: 32 tokens x 32 FB features per wave at a
+  merge_groups<FB, TB, WK>(acc, lds, w % (WF * WT), wk, lane);
+  // bf16, and out through LDS: 32 tokens x 32 FB features per wave at a
   // time, rows of kOutRow bytes (padded), then 16-byte row pieces
   constexpr int kOutRow = 64 * FB + 16;
   unsigned char* mine = lds + w * 32 * kOutRow;
@@ -426,161 +434,398 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_kernel(const GemmCall a) 
 }
 
 // ---------------------------------------------------------------------------
-// Every other projection (fp32 tensors, the fp32-operand mode, or bf16
-// tensors of a shape neither kernel above takes): both directions on
-// v_mfma_f32_16x16x4f32, any shape, operands converted to fp32 on load.  A workgroup computes a 64-feature x
-// 64-token tile of C^T, 4 waves of 32 x 32 (2 x 2 blocks of 16 x 16).
-// Stages of 32 reduction elements go global -> registers -> LDS (two
-// buffers, one barrier per stage, the next stage's loads in flight during
-// the products); elements past any edge load as zero.
-//   forward  (NT) C^T[f][t] = sum_k W[f][k] X[t][k]   (A tile [f][k])
-//   backward (NN) C^T[c][t] = sum_z sum_f W_z[f][c] dY_z[t][f]   (A tile [f][c])
-// MFMA layout (lane l, c = l % 16, g = l / 16): A[row c][k = g],
-// B[k = g][col c]; accumulator i holds column c, row 4 g + i: four
-// consecutive features of one token.
+// Every other call (fp32 tensors, and bf16 tensors of other widths or
+// alignments): the same sums, with each operand element split in three bf16
+// terms (split3.hpp) on its way from global memory to LDS, and six
+// v_mfma_f32_32x32x16_bf16 per product of fragments.  The low-rank product is
+// again a stretch of the reduction, the adapters' ranks one after another, its
+// operands taken as they are (fp32, B and A read down their columns); it goes
+// first, while the base products' first stages are on their way.
+//
+// 8 waves: WF x WT waves of FB x TB blocks of 32 x 32, times WK groups that
+// share a stage's two k-steps.  Stages of 32 reduction elements go global ->
+// registers (PF stages ahead) -> three LDS planes of bf16 rows (layout as above:
+// 64-byte rows, backward A 64-feature sub-tiles), two buffers, one barrier a
+// stage.  Loads are unconditional at clamped addresses; elements past the
+// reduction are zeroed in A, rows past an edge reach no stored result.
+// A tile that meets an element without a split (not finite, or rounding to
+// infinity) is done over on fp32 MFMAs, straight from global memory.
+//
+// What bounds it: at one small tile per CU the chain of a stage (split, LDS,
+// six dependent products: 0.75 us); once the chip is full the six products
+// (6/16 of the fp32 MFMA's time) and the split's 11 vector instructions for each
+// 2 elements beside them.  201 x 896 -> 896/128/128: forward 24 us in one
+// launch (three of 35, and two low-rank passes, before), backward 31 us (46
+// and two).
 // ---------------------------------------------------------------------------
-constexpr int kFT = 64;       // features and tokens per tile
-constexpr int kFK = 32;       // reduction elements per stage
-constexpr int kFS = kFK + 4;  // row stride of [row][k] tiles (floats): conflict-free
-constexpr int kFC = kFT + 16; // row stride of the backward's [k][feature] tile
-constexpr int kFThreads = 256;
-
-// Four elements k .. k + 3 of a row (len elements valid) as fp32, zero past
-// the end; vec: the row allows one aligned vector load.
-template <typename IO>
-__device__ inline f32x4 load4_f32(const IO* row, int k, int len, bool vec) {
-  if (vec && k + 3 < len) {
-    if constexpr (sizeof(IO) == 4) {
-      return *reinterpret_cast<const f32x4*>(row + k);
-    } else {
-      const bf16x4 h = *reinterpret_cast<const bf16x4*>(row + k);
-      return f32x4{(float)h[0], (float)h[1], (float)h[2], (float)h[3]};
-    }
-  }
-  f32x4 v;
+// Ends a run of products where control flow joins: 16 wait states, so that the
+// copies of accumulators that the compiler may place there read what the last
+// MFMA wrote.  (It leaves too few of its own before copies in a loop's header:
+// one instance lost its sums that way.)
+template <int FB, int TB>
+__device__ inline void settle(f32x16 (&acc)[FB][TB]) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) v[i] = k + i < len ? (float)row[k + i] : 0.0f;
-  return v;
+  for (int fb = 0; fb < FB; ++fb)
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb) tie_v(acc[fb][tb]);
+  asm volatile("s_nop 15" : "+v"(acc[FB - 1][TB - 1]));
 }
 
-template <typename IO, bool NN>
-__global__ __launch_bounds__(kFThreads) void proj_gemm_f32_kernel(const WideFwd fa, const WideBwd ba) {
-  __shared__ __align__(16) float la[2][NN ? kFK * kFC : kFT * kFS];
-  __shared__ __align__(16) float lb[2][kFT * kFS];
-  const int T = NN ? ba.T : fa.T;
-  const int nout = NN ? ba.K : fa.n;  // C^T rows: features
-  const int ttiles = (T + kFT - 1) / kFT;
+template <typename E>
+__device__ inline void load4_any(const E* p, float (&x)[8], int at) {
+  typedef E E4 __attribute__((ext_vector_type(4)));
+  E4 v;
+  __builtin_memcpy(&v, p, sizeof(v));
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[at + e] = (float)v[e];
+}
+// A thread's 8 elements of a stage on their way to LDS, as loaded: the first
+// `valid` count, the rest are zeros.
+struct Piece {
+  float x[8];
+  int valid;
+};
+
+template <typename IO, bool NN, int FB, int TB, int WF, int WT, int WK, int PF>
+__global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCall a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  static_assert(WF * WT * WK == 8 && (WK == 1 || WK == 2), "8 waves");
+  constexpr int FT = WF * FB * 32, TT = WT * TB * 32, KT = 32, KS = 2 / WK;
+  constexpr int NA = FT * 4 / kGThreads, NB = TT * 4 / kGThreads;  // 8-element pieces per thread
+  constexpr int PA = FT * 4, PB = TT * 4;                          // pieces in all
+  constexpr int kPlaneA = FT * 64, kPlaneB = TT * 64, kBuf = 3 * (kPlaneA + kPlaneB);
+  static_assert((PA % kGThreads == 0 && PB % kGThreads == 0) || (NA == 0 && NB == 0 && PA + PB == kGThreads),
+                "pieces per thread");
+  constexpr bool kShared = NA == 0;  // half of the threads bring A, half B
+  constexpr int LA = kShared ? 1 : NA, LB = kShared ? 0 : NB;
+  __shared__ __align__(1024) unsigned char lds[2 * kBuf];
+  const int T = a.T, K = a.K, rank = a.rank;
+  const int ttiles = (T + TT - 1) / TT;
   const int id = xcd_logical((int)blockIdx.x, (int)gridDim.x);
-  const int t0 = kFT * (id % ttiles), f0 = kFT * (id / ttiles);
+  int ft, tt;
+  tile_of(id, a.ftiles, ttiles, ft, tt);
+  int z = 0;
+  if constexpr (!NN)
+    while (z + 1 < a.n && ft >= a.j[z + 1].first) ++z;
+  const int f0 = NN ? FT * ft : FT * (ft - a.j[z].first), t0 = TT * tt;
+  const int nf = NN ? K : a.j[z].n;
   const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
-  const int wf = w & 1, wt = w >> 1, c = lane & 15, g = lane >> 4;
-  // stages: forward over K; backward over every job's outputs in turn
-  int nst = 0;
-  if constexpr (NN) {
-    for (int z = 0; z < ba.n; ++z) nst += (ba.j[z].n + kFK - 1) / kFK;
-  } else {
-    nst = (fa.K + kFK - 1) / kFK;
+  const int wf = w % WF, wt = w / WF % WT, wk = w / (WF * WT);
+
+  // the base products: forward X W^T, backward every dY_p W_p
+  const int seg0 = NN ? 0 : z, seg1 = NN ? a.n : z + 1;
+  int nst = 0, terms = 0;
+  for (int y = seg0; y < seg1; ++y) {
+    nst += (a.seg[y].k + KT - 1) / KT;
+    terms += a.j[y].l != nullptr;
   }
-  f32x4 ra[2], rb[2];
-  auto load = [&](int st) {
-    const IO* wsrc;
-    const IO* bsrc;
-    int k0, klen, bstride;
+  // the terms in order: with element kk of the low-rank stretch in term kk / rank
+  const int n_low = terms * rank, low_st = (n_low + KT - 1) / KT;
+  auto job_of = [&](int term) {  // the term's projection
+    int y = seg0;
+    for (;; ++y)
+      if (a.j[y].l != nullptr && term-- == 0) break;
+    return y;
+  };
+
+  // Piece idx of a stage of the base products, reduction elements k0 .. of
+  // segment `cur`: A (forward: row f, 8 reduction elements; backward:
+  // reduction row, 8 features) and B (row t, 8 reduction elements).
+  int sg = seg0 - 1, kend = 0, kbase = 0, kcur = 0;
+  const IO *ca = nullptr, *cb = nullptr;
+  auto load_a = [&](int idx, int k0, Piece& p) {
     if constexpr (NN) {
-      int z = 0, base = 0;
-      while (z + 1 < ba.n && st >= base + (ba.j[z].n + kFK - 1) / kFK) base += (ba.j[z++].n + kFK - 1) / kFK;
-      k0 = kFK * (st - base);
-      klen = ba.j[z].n;
-      wsrc = static_cast<const IO*>(ba.j[z].w);
-      bsrc = static_cast<const IO*>(ba.j[z].dy);
-      bstride = klen;
+      const int k = k0 + (idx >> 3) % 32, f = f0 + 64 * (idx >> 8) + 8 * (idx & 7);
+      p.valid = k < kcur ? 8 : 0;
+      const IO* row = ca + (long)min(k, kcur - 1) * K;
+      load4_any(row + min(f, K - 4), p.x, 0);
+      load4_any(row + min(f + 4, K - 4), p.x, 4);
     } else {
-      k0 = kFK * st;
-      klen = fa.K;
-      wsrc = static_cast<const IO*>(fa.w);
-      bsrc = static_cast<const IO*>(fa.x);
-      bstride = fa.K;
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int idx = tid + kFThreads * i;
-      if constexpr (NN) {
-        // A: W_z rows k0 + idx / 16 (of klen), columns f0 + 4 (idx % 16)
-        const int kr = k0 + (idx >> 4), cc = f0 + 4 * (idx & 15);
-        ra[i] = kr < klen ? load4_f32(wsrc + (long)kr * ba.K, cc, nout, (ba.K & 3) == 0) : f32x4{0, 0, 0, 0};
-      } else {
-        // A: W rows f0 + idx / 8, columns k0 + 4 (idx % 8)
-        const int fr = f0 + (idx >> 3), kc = k0 + 4 * (idx & 7);
-        ra[i] = fr < nout ? load4_f32(wsrc + (long)fr * fa.K, kc, klen, (fa.K & 3) == 0) : f32x4{0, 0, 0, 0};
-      }
-      // B: rows t0 + idx / 8 (tokens), columns k0 + 4 (idx % 8)
-      const int tr = t0 + (idx >> 3), kc = k0 + 4 * (idx & 7);
-      rb[i] = tr < T ? load4_f32(bsrc + (long)tr * bstride, kc, klen, (bstride & 3) == 0) : f32x4{0, 0, 0, 0};
+      const int f = min(f0 + (idx >> 2), nf - 1), k = k0 + 8 * (idx & 3);
+      p.valid = kcur - k;
+      const IO* row = ca + (long)f * kcur;
+      load4_any(row + min(k, kcur - 4), p.x, 0);
+      load4_any(row + min(k + 4, kcur - 4), p.x, 4);
     }
   };
-  auto store = [&](int buf) {
+  auto load_b = [&](int idx, int k0, Piece& p) {
+    const int t = min(t0 + (idx >> 2), T - 1), k = k0 + 8 * (idx & 3);
+    p.valid = 8;
+    const IO* row = cb + (long)t * kcur;
+    load4_any(row + min(k, kcur - 4), p.x, 0);
+    load4_any(row + min(k + 4, kcur - 4), p.x, 4);
+  };
+  // the same of the low-rank stretch, its elements kk0 ..
+  auto low_a = [&](int idx, int kk0, Piece& p) {
+    const int kk = NN ? kk0 + (idx >> 3) % 32 : kk0 + 8 * (idx & 3);
+    const int f = NN ? f0 + 64 * (idx >> 8) + 8 * (idx & 7) : min(f0 + (idx >> 2), nf - 1);
+    p.valid = NN ? (kk < n_low ? 8 : 0) : n_low - kk;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int idx = tid + kFThreads * i;
-      if constexpr (NN)
-        *reinterpret_cast<f32x4*>(&la[buf][(idx >> 4) * kFC + 4 * (idx & 15)]) = ra[i];
+    for (int e = 0; e < 8; ++e) {
+      const int q = min(NN ? kk : kk + e, n_low - 1), term = q / rank, j = q - term * rank;
+      const float* v = a.j[job_of(term)].v;
+      p.x[e] = NN ? v[(long)min(f + e, K - 1) * rank + j] : v[(long)j * nf + f];
+    }
+  };
+  auto low_b = [&](int idx, int kk0, Piece& p) {
+    const int t = min(t0 + (idx >> 2), T - 1), kk = kk0 + 8 * (idx & 3);
+    p.valid = 8;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int q = min(kk + e, n_low - 1), term = q / rank, j = q - term * rank;
+      const GemmJob& job = a.j[job_of(term)];
+      p.x[e] = job.s * job.l[(long)t * rank + j];
+    }
+  };
+  struct Pieces {
+    Piece a[LA], b[LB > 0 ? LB : 1];
+  };
+  auto load = [&](int st, Pieces& p) {
+    while (st >= kend && sg + 1 < seg1) {
+      ++sg;
+      kbase = kend;
+      kcur = a.seg[sg].k;
+      kend += (kcur + KT - 1) / KT;
+      ca = static_cast<const IO*>(a.seg[sg].a);
+      cb = static_cast<const IO*>(a.seg[sg].b);
+    }
+    const int k0 = (st - kbase) * KT;
+    if constexpr (kShared) {
+      if (w < PA / 64)
+        load_a(tid, k0, p.a[0]);
       else
+        load_b(tid - PA, k0, p.a[0]);
+    } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) la[buf][(idx >> 3) * kFS + 4 * (idx & 7) + e] = ra[i][e];
+      for (int i = 0; i < LA; ++i) load_a(tid + kGThreads * i, k0, p.a[i]);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) lb[buf][(idx >> 3) * kFS + 4 * (idx & 7) + e] = rb[i][e];
+      for (int i = 0; i < LB; ++i) load_b(tid + kGThreads * i, k0, p.b[i]);
     }
   };
-  f32x4 acc[2][2];
+  auto load_low = [&](int st, Pieces& p) {
+    if constexpr (kShared) {
+      if (w < PA / 64)
+        low_a(tid, st * KT, p.a[0]);
+      else
+        low_b(tid - PA, st * KT, p.a[0]);
+    } else {
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < LA; ++i) low_a(tid + kGThreads * i, st * KT, p.a[i]);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  if (nst > 0) {
-    load(0);
-    store(0);
-  }
-  __syncthreads();
-  for (int st = 0; st < nst; ++st) {
-    const int buf = st & 1;
-    if (st + 1 < nst) load(st + 1);
+      for (int i = 0; i < LB; ++i) low_b(tid + kGThreads * i, st * KT, p.b[i]);
+    }
+  };
+  bool bad = false;
+  // piece idx of operand `b` (0: A, 1: B) into the three planes of a buffer
+  auto put = [&](unsigned char* base, int idx, bool b, Piece& q) {
 #pragma unroll
-    for (int kk = 0; kk < kFK / 4; ++kk) {
-      float av[2], bv[2];
+    for (int e = 0; e < 8; ++e) {
+      tie_v(q.x[e]);  // the load stays unconditional
+      q.x[e] = e < q.valid ? q.x[e] : 0.0f;
+    }
+    Split3 s;
+    bad |= s.set(q.x);
+    int off;
+    if (NN && !b) {
+      const int r = (idx >> 3) % 32;
+      off = 4096 * (idx >> 8) + 128 * r + 16 * ((idx & 7) ^ lds_sw<64>(r));
+    } else {
+      const int r = idx >> 2;
+      off = 64 * r + 16 * ((idx & 3) ^ lds_sw<32>(r));
+    }
+    unsigned char* p = base + (b ? 3 * kPlaneA : 0) + off;
+    const int plane = b ? kPlaneB : kPlaneA;
+    *reinterpret_cast<bf16x8*>(p) = s.h;
+    *reinterpret_cast<bf16x8*>(p + plane) = s.m;
+    *reinterpret_cast<bf16x8*>(p + 2 * plane) = s.l;
+  };
+  auto put_all = [&](unsigned char* base, Pieces& p) {
+    if constexpr (kShared) {
+      put(base, w < PA / 64 ? tid : tid - PA, w >= PA / 64, p.a[0]);
+    } else {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int fr = 32 * wf + 16 * i + c, tr = 32 * wt + 16 * i + c, k = 4 * kk + g;
-        av[i] = NN ? la[buf][k * kFC + fr] : la[buf][fr * kFS + k];
-        bv[i] = lb[buf][tr * kFS + k];
+      for (int i = 0; i < LA; ++i) put(base, tid + kGThreads * i, false, p.a[i]);
+#pragma unroll
+      for (int i = 0; i < LB; ++i) put(base, tid + kGThreads * i, true, p.b[i]);
+    }
+  };
+
+  const int fw = f0 + 32 * FB * wf, tw = t0 + 32 * TB * wt;
+  const float* bias = NN || wk != 0 ? nullptr : a.j[z].bias;
+  f32x16 acc[FB][TB];
+  auto clear = [&] {
+#pragma unroll
+    for (int fb = 0; fb < FB; ++fb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int f = fw + 32 * fb + 8 * (e / 4) + 4 * (lane >> 5) + e % 4;
+        const float b = bias == nullptr ? 0.0f : bias[min(f, nf - 1)];
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) acc[fb][tb][e] = b;
       }
+  };
+  clear();
+
+  // LDS offsets of the fragments of k-step s of this wave
+  unsigned oa[NN ? 2 * FB : KS], ob[KS];
+  {
+    const unsigned b = frag_off<32>(lane, 32 * TB * wt);
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+    for (int s = 0; s < KS; ++s) ob[s] = 3 * kPlaneA + (b ^ (32u * (KS * wk + s)));
+    if constexpr (NN) {
+#pragma unroll
+      for (int fb = 0; fb < FB; ++fb) {
+        const int col = 32 * (FB * wf + fb);
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+          oa[2 * fb + j] = 4096u * (col / 64) + tr_off128(lane, col % 64, j) + 2048u * KS * wk;
+      }
+    } else {
+      const unsigned o = frag_off<32>(lane, 32 * FB * wf);
+#pragma unroll
+      for (int s = 0; s < KS; ++s) oa[s] = o ^ (32u * (KS * wk + s));
     }
-    if (st + 1 < nst) store(buf ^ 1);
-    __syncthreads();
   }
-  // C [T][nout]: token t0 + 32 wt + 16 j + c, features f0 + 32 wf + 16 i + 4 g ..
-  float* cdst = NN ? ba.c : fa.c;
+  bf16x8 fa[KS][FB][3], fbk[KS][TB][3];
+  auto fragments = [&](const unsigned char* base) {
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int t = t0 + 32 * wt + 16 * j + c;
-    if (t >= T) continue;
+    for (int s = 0; s < KS; ++s)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int f = f0 + 32 * wf + 16 * i + 4 * g;
-      float* d = cdst + (long)t * nout + f;
-      if (f + 3 < nout && (nout & 3) == 0) {
-        *reinterpret_cast<f32x4*>(d) = acc[i][j];
-      } else {
+      for (int p = 0; p < 3; ++p) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (f + e < nout) d[e] = acc[i][j][e];
+        for (int fb = 0; fb < FB; ++fb) {
+          if constexpr (NN) {
+            auto tr = [&](int j) {
+              return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((bf16x4 GLACIER_LDS*)const_cast<unsigned char*>(
+                  base + oa[2 * fb + j] + kPlaneA * p + 2048 * s));
+            };
+            fa[s][fb][p] = join8(tr(0), tr(1));
+          } else {
+            fa[s][fb][p] = *reinterpret_cast<const bf16x8*>(base + oa[s] + kPlaneA * p + 2048 * fb);
+          }
+        }
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb)
+          fbk[s][tb][p] = *reinterpret_cast<const bf16x8*>(base + ob[s] + kPlaneB * p + 2048 * tb);
+      }
+  };
+  auto products = [&] {
+    // the small products first
+    constexpr int kPa[6] = {2, 0, 1, 1, 0, 0}, kPb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+#pragma unroll
+        for (int fb = 0; fb < FB; ++fb)
+#pragma unroll
+          for (int tb = 0; tb < TB; ++tb)
+            acc[fb][tb] = mma32(fa[s][fb][kPa[q]], fbk[s][tb][kPb[q]], acc[fb][tb]);
+  };
+  // Stage n in buffer n % 2: its fragments are read, the next stage's pieces
+  // split and written to the other buffer (every wave is past its reads of it)
+  // behind those reads, then come the products, then the barrier that makes
+  // the next stage's rows visible.
+  int n = 0;
+  auto turn = [&](auto&& next) {
+    fragments(lds + (n & 1) * kBuf);
+    ++n;
+    next(lds + (n & 1) * kBuf);
+    products();
+    lgkm<0>();
+    wg_barrier();
+  };
+  Pieces ring[PF];
+  {
+    Pieces low;
+    if (low_st > 0) load_low(0, low);
+    static_for<PF>([&](auto jc) { load(decltype(jc)::value, ring[decltype(jc)::value]); });
+    if (low_st > 0) {
+      put_all(lds, low);
+      if (low_st > 1) load_low(1, low);
+      lgkm<0>();
+      wg_barrier();
+      for (int st = 1; st < low_st; ++st)
+        turn([&](unsigned char* base) {
+          put_all(base, low);
+          if (st + 1 < low_st) load_low(st + 1, low);
+        });
+      turn([&](unsigned char* base) { put_all(base, ring[0]); });
+    } else {
+      put_all(lds, ring[0]);
+      lgkm<0>();
+      wg_barrier();
+    }
+    load(PF, ring[0]);
+  }
+  settle(acc);
+  for (int st0 = 0; st0 < nst; st0 += PF) {
+    static_for<PF>([&](auto jc) {
+      // stages past the end hold zeros (no valid element), and add nothing
+      constexpr int J = (decltype(jc)::value + 1) % PF;
+      turn([&](unsigned char* base) {
+        put_all(base, ring[J]);
+        load(st0 + decltype(jc)::value + 1 + PF, ring[J]);
+      });
+    });
+    settle(acc);
+  }
+  if (__syncthreads_or(bad)) {
+    // the same sums on fp32 MFMAs: lane l supplies A[row l % 32][k + l / 32]
+    // and B's column likewise; group 0 sums everything
+    clear();
+    if (wk == 0) {
+      for (int i = 2 * seg0; i < 2 * seg1; ++i) {
+        const int y = i / 2;
+        const bool low = i & 1;
+        const GemmJob& job = a.j[y];
+        const int len = !low ? a.seg[y].k : job.l == nullptr ? 0 : rank;
+#pragma clang loop unroll(disable)
+        for (int k0 = 0; k0 < len; k0 += 2) {
+          const int k = min(k0 + (lane >> 5), len - 1);
+          const bool ok = k0 + (lane >> 5) < len;
+          float va[FB], vb[TB];
+#pragma unroll
+          for (int fb = 0; fb < FB; ++fb) {
+            const int f = min(fw + 32 * fb + (lane & 31), nf - 1);
+            const float v = low ? (NN ? job.v[(long)f * rank + k] : job.v[(long)k * nf + f])
+                                : (float)static_cast<const IO*>(a.seg[y].a)[NN ? (long)k * K + f : (long)f * len + k];
+            va[fb] = ok ? v : 0.0f;
+          }
+#pragma unroll
+          for (int tb = 0; tb < TB; ++tb) {
+            const long at = (long)min(tw + 32 * tb + (lane & 31), T - 1) * len + k;
+            const float v = low ? job.s * job.l[at] : (float)static_cast<const IO*>(a.seg[y].b)[at];
+            vb[tb] = ok ? v : 0.0f;
+          }
+#pragma unroll
+          for (int fb = 0; fb < FB; ++fb)
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb)
+              acc[fb][tb] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[fb], vb[tb], acc[fb][tb], 0, 0, 0);
+        }
       }
     }
   }
+  merge_groups<FB, TB, WK>(acc, lds, w % (WF * WT), wk, lane);
+  IO* out = static_cast<IO*>(NN ? a.dx : a.j[z].y);
+#pragma unroll
+  for (int tb = 0; tb < TB; ++tb) {
+    const int t = tw + 32 * tb + (lane & 31);
+    if (t >= T) continue;
+#pragma unroll
+    for (int fb = 0; fb < FB; ++fb) {
+      if (block_owner<FB, TB, WK>(fb, tb) != wk) continue;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int f = fw + 32 * fb + 8 * q + 4 * (lane >> 5);
+        if (f < nf)  // nf % 4 == 0
+          store4(out + (long)t * nf + f,
+                 f32x4{acc[fb][tb][4 * q], acc[fb][tb][4 * q + 1], acc[fb][tb][4 * q + 2], acc[fb][tb][4 * q + 3]});
+      }
+    }
+  }
+#endif
 }
 
 }  // namespace
@@ -615,6 +860,8 @@ const GemmShape kShapes[] = {
     GL_GEMM(256, 0.23f, 0.27f, 128, 1, 1, 2, 2, 2, 4, 5),  // 64 x 64
 };
 #undef GL_GEMM
+
+constexpr int kBigSplitTiles = 128;
 
 int tiles_of(const GemmCall& a, bool nn, const GemmShape& s) {
   int ftiles = 0;
@@ -659,24 +906,40 @@ hipError_t launch_gemm_shape(GemmCall a, bool nn, int shape, hipStream_t st) {
 
 }  // namespace
 
+namespace {
+
+template <typename IO, bool NN>
+hipError_t launch_split(GemmCall a, hipStream_t st) {
+  // 128 x 128 tiles once they fill most of the CUs (their waves do twice the
+  // products per LDS byte), else 64 x 64
+  auto tiles = [&](int ft) {
+    a.ftiles = 0;
+    for (int z = 0; z < (NN ? 1 : a.n); ++z) {
+      a.j[z].first = a.ftiles;
+      a.ftiles += ((NN ? a.K : a.j[z].n) + ft - 1) / ft;
+    }
+    return a.ftiles * ((a.T + ft - 1) / ft);
+  };
+  int n = tiles(128);
+  const bool big = n >= kBigSplitTiles;
+  if (!big) n = tiles(64);
+  if (n == 0) return hipSuccess;
+  if (big)
+    hipLaunchKernelGGL((proj_gemm_split_kernel<IO, NN, 2, 1, 2, 4, 1, 2>), dim3(n), dim3(kGThreads), 0, st, a);
+  else
+    hipLaunchKernelGGL((proj_gemm_split_kernel<IO, NN, 1, 1, 2, 2, 2, 4>), dim3(n), dim3(kGThreads), 0, st, a);
+  return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_gemm(GemmCall a, bool nn, hipStream_t st) {
   return launch_gemm_shape(a, nn, gemm_shape(a, nn), st);
 }
 
-hipError_t launch_generic_fwd(const WideFwd& a, bool io_bf16, hipStream_t st) {
-  const int ttiles = (a.T + kFT - 1) / kFT, ftiles = (a.n + kFT - 1) / kFT;
-  if (ttiles == 0 || ftiles == 0) return hipSuccess;
-  auto fn = io_bf16 ? proj_gemm_f32_kernel<bf16, false> : proj_gemm_f32_kernel<float, false>;
-  hipLaunchKernelGGL(fn, dim3(ttiles * ftiles), dim3(kFThreads), 0, st, a, WideBwd{});
-  return hipGetLastError();
-}
-
-hipError_t launch_generic_bwd(const WideBwd& a, bool io_bf16, hipStream_t st) {
-  const int ttiles = (a.T + kFT - 1) / kFT, ftiles = (a.K + kFT - 1) / kFT;
-  if (ttiles == 0 || ftiles == 0 || a.n == 0) return hipSuccess;
-  auto fn = io_bf16 ? proj_gemm_f32_kernel<bf16, true> : proj_gemm_f32_kernel<float, true>;
-  hipLaunchKernelGGL(fn, dim3(ttiles * ftiles), dim3(kFThreads), 0, st, WideFwd{}, a);
-  return hipGetLastError();
+hipError_t launch_gemm_split(const GemmCall& a, bool nn, bool io_bf16, hipStream_t st) {
+  if (io_bf16) return nn ? launch_split<bf16, true>(a, st) : launch_split<bf16, false>(a, st);
+  return nn ? launch_split<float, true>(a, st) : launch_split<float, false>(a, st);
 }
 
 }  // namespace glacier

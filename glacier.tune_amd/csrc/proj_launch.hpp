@@ -37,9 +37,6 @@ struct ProjLaunch {
   float* lowrank;  // [slot][T][r] X A_p and dY_p B_p^T
   void* terms;     // fused calls: the split terms (bf16) of the adapters, then of s L
   int* odd;        // fused calls: non-finite marks (SplitCall)
-  float* yf;       // other calls, forward: [T][out_p] base products, one after another
-  float* dxf;      // other calls, backward: [T][in] sum_p dY_p W_p
-  float* part;     // other calls: split sums of the low-rank products
 };
 
 // ---- bf16 tensors: base products, low-rank delta, bias and conversion in ----
@@ -71,35 +68,15 @@ struct GemmCall {
 __host__ __device__ constexpr int term_pitch(int rank) { return (6 * rank + 7) / 8 * 8; }
 hipError_t launch_gemm(GemmCall a, bool backward, hipStream_t st);
 
-// ---- the base products alone, fp32 results, for every other call ----
-struct WideJob {
-  const void* w;   // W_z [n][K]
-  const void* dy;  // dY_z [T][n]
-  int n;           // outputs of the projection
-};
-// c [T][n] = X W^T (fp32), one projection.
-struct WideFwd {
-  const void* x;  // [T][K]
-  const void* w;  // [n][K]
-  float* c;
-  int T, K, n;
-};
-// c [T][K] = sum over the jobs of dY_z W_z (fp32)
-struct WideBwd {
-  float* c;
-  int T, K, n;
-  WideJob j[kMaxProj];
-};
+// Every other call (fp32 tensors; bf16 ones of other widths or alignments),
+// the operands split as they are loaded; the adapter's terms are not used.
+hipError_t launch_gemm_split(const GemmCall& a, bool backward, bool io_bf16, hipStream_t st);
 
-// fp32 MFMAs, any shape, fp32 or bf16 operands (io_bf16) converted on load
-hipError_t launch_generic_fwd(const WideFwd& a, bool io_bf16, hipStream_t st);
-hipError_t launch_generic_bwd(const WideBwd& a, bool io_bf16, hipStream_t st);
-
-// Floats (unless stated) of each ProjLaunch scratch buffer for a forward or backward call.
+// Elements of each ProjLaunch scratch buffer for a forward or backward call.
 struct ProjScratchNeed {
-  long yf, dxf, lowrank, part;
-  long terms;  // bf16 elements
-  long odd;    // ints
+  long lowrank;  // floats
+  long terms;    // bf16
+  long odd;      // ints
 };
 ProjScratchNeed proj_scratch_need(const ProjLaunch& a, bool backward);
 

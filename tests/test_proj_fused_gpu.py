@@ -1,6 +1,6 @@
-"""The projections' fused path for bf16 tensors (proj_gemm.hip,
-lowrank_split in proj_lora.hip) at the edges of its tiles, against float64
-products of the same bf16 operands on the GPU.
+"""The projections' GEMMs (proj_gemm.hip: bf16 by DMA, and split operands for
+fp32 tensors and other widths) and lowrank_split (proj_lora.hip) at the edges
+of their tiles, against float64 products of the same operands on the GPU.
 
 Bound per element: the result's rounding to bf16 (8 significant bits with the
 implicit one: neighbours are 2^-7 apart relative to the lower power of two,
@@ -8,6 +8,7 @@ so half of that, 2^-8 relative) plus fp32
 summation over n terms, n 2^-24 sum |terms| in the worst case; the sums
 round to both sides, so sqrt(n) 2^-22 sum |terms| holds with room, and the
 low-rank operands enter with all 24 bits (split3.hpp) within the same bound.
+fp32 results have 2^-24 in the place of 2^-8.
 """
 import sys
 
@@ -20,22 +21,30 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.fixture(scope="module")
-def engine():
+def engines():
     assert torch.cuda.is_available(), "GPU tests need a ROCm GPU"
-    with ga.GpuAttentionEngine(0, ga.PREC_BF16) as e:
-        yield e
+    made = {torch.bfloat16: ga.GpuAttentionEngine(0, ga.PREC_BF16),
+            torch.float32: ga.GpuAttentionEngine(0, ga.PREC_FP32)}
+    yield made
+    for e in made.values():
+        e.close()
 
 
-def _problem(T, n_in, outs, rank, seed=3, w_shift=0):
+@pytest.fixture(scope="module")
+def engine(engines):
+    return engines[torch.bfloat16]
+
+
+def _problem(T, n_in, outs, rank, seed=3, w_shift=0, dtype=torch.bfloat16):
     """w_shift: elements by which each W misses its allocation's alignment."""
     g = torch.Generator(device="cuda").manual_seed(seed)
     rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
-    x = rnd(T, n_in).bfloat16()
+    x = rnd(T, n_in).to(dtype)
     projs = []
     for i, o in enumerate(outs):
-        w = torch.empty(o * n_in + w_shift, device="cuda", dtype=torch.bfloat16)[w_shift:]
+        w = torch.empty(o * n_in + w_shift, device="cuda", dtype=dtype)[w_shift:]
         w = w.view(o, n_in).copy_(rnd(o, n_in) * n_in ** -0.5)
-        p = {"w": w, "bias": 0.1 * rnd(o), "dy": rnd(T, o).bfloat16(), "scaling": 2.0}
+        p = {"w": w, "bias": 0.1 * rnd(o), "dy": rnd(T, o).to(dtype), "scaling": 2.0}
         if i != 1:  # the second projection has no adapter
             p.update(a=rnd(n_in, rank) * n_in ** -0.5, b=0.1 * rnd(rank, o))
             p.update(grad_a=torch.zeros_like(p["a"]), grad_b=torch.zeros_like(p["b"]))
@@ -62,7 +71,7 @@ def _reference(x, projs):
 
 def _check(got, want, terms, n, what):
     err = (got.double() - want).abs()
-    bound = 2.0 ** -8 * want.abs() + n ** 0.5 * 2.0 ** -22 * terms
+    bound = 2.0 ** (-8 if got.dtype == torch.bfloat16 else -24) * want.abs() + n ** 0.5 * 2.0 ** -22 * terms
     worst = float((err / bound).max())
     print(f"  {what}: worst error {worst:.2f} of its bound", flush=True)
     assert worst <= 1.0
@@ -81,17 +90,26 @@ SHAPES = [  # T, in, outs, rank
 ]
 
 
-@pytest.mark.parametrize("T,n_in,outs,rank", SHAPES)
-def test_fused_projection_matches_float64(engine, T, n_in, outs, rank):
-    print(f"[fused proj] T={T} in={n_in} outs={outs} rank={rank}", flush=True)
-    sys.stdout.flush()
-    x, projs = _problem(T, n_in, outs, rank)
-    ys = engine.proj_forward(x, projs, rank)
-    dx = engine.proj_backward(x, projs, rank)
+OTHER_SHAPES = [  # the split-operand GEMM
+    (torch.float32, 1, 4, (4,), 1),
+    (torch.float32, 37, 100, (36, 72), 3),
+    (torch.float32, 65, 1000, (1000, 200, 200), 20),
+    (torch.float32, 130, 264, (516, 4), 64),
+    (torch.float32, 512, 3584, (3584, 512, 512), 16),  # the larger tiles
+    (torch.float32, 1025, 520, (2052,), 8),
+    (torch.bfloat16, 37, 100, (36, 72), 3),            # rows of half 16-byte pieces
+    (torch.bfloat16, 700, 1004, (3004, 12), 17),
+]
+
+
+def _run_and_check(eng, x, projs, rank):
+    n_in = x.shape[1]
+    ys = eng.proj_forward(x, projs, rank)
+    dx = eng.proj_backward(x, projs, rank)
     want, want_dx = _reference(x, projs)
     for i, (y, (ref, terms)) in enumerate(zip(ys, want)):
         _check(y, ref, terms, n_in, f"y{i}")
-    _check(dx, *want_dx, sum(outs), "dx")
+    _check(dx, *want_dx, sum(p["w"].shape[0] for p in projs), "dx")
     xd = x.double()
     for p in projs:
         if "a" not in p:
@@ -99,6 +117,20 @@ def test_fused_projection_matches_float64(engine, T, n_in, outs, rank):
         dl, l = p["dy"].double() @ p["b"].double().t(), xd @ p["a"].double()
         for got, ref in ((p["grad_a"], 2.0 * xd.t() @ dl), (p["grad_b"], 2.0 * l.t() @ p["dy"].double())):
             assert float((got.double() - ref).norm() / ref.norm()) <= 2e-6  # fp32 sums
+
+
+@pytest.mark.parametrize("T,n_in,outs,rank", SHAPES)
+def test_fused_projection_matches_float64(engine, T, n_in, outs, rank):
+    print(f"[fused proj] T={T} in={n_in} outs={outs} rank={rank}", flush=True)
+    sys.stdout.flush()
+    _run_and_check(engine, *_problem(T, n_in, outs, rank), rank)
+
+
+@pytest.mark.parametrize("dtype,T,n_in,outs,rank", OTHER_SHAPES)
+def test_split_projection_matches_float64(engines, dtype, T, n_in, outs, rank):
+    print(f"[split proj] {dtype} T={T} in={n_in} outs={outs} rank={rank}", flush=True)
+    sys.stdout.flush()
+    _run_and_check(engines[dtype], *_problem(T, n_in, outs, rank, dtype=dtype), rank)
 
 
 def test_unaligned_weights_take_the_general_path(engine):
@@ -115,12 +147,14 @@ def test_unaligned_weights_take_the_general_path(engine):
 
 
 @pytest.mark.parametrize("where", ["x", "a", "b", "dy", "huge_b"])
-def test_non_finite_values_pass_through(engine, where):
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_non_finite_values_pass_through(engines, dtype, where):
     """Infinities, NaN and values past bf16's range have no split terms: the
     results hold inf and NaN exactly where float32 arithmetic does, and every
     other element is unharmed."""
     T, n_in, outs, rank = 70, 136, (72, 64), 8
-    x, projs = _problem(T, n_in, outs, rank)
+    engine = engines[dtype]
+    x, projs = _problem(T, n_in, outs, rank, dtype=dtype)
     p = projs[0]
     if where == "x":
         x[5, 7], x[9, 3] = float("inf"), float("nan")
@@ -138,7 +172,7 @@ def test_non_finite_values_pass_through(engine, where):
     dx = engine.proj_backward(x, projs, rank)
     want, want_dx = _reference(x, projs)
     for got, (ref, terms) in zip([*ys, dx], [*want, want_dx]):
-        ref32 = ref.float().bfloat16()
+        ref32 = ref.float().to(dtype)
         assert torch.equal(torch.isnan(got), torch.isnan(ref32))
         assert torch.equal(torch.isinf(got), torch.isinf(ref32))
         ok = torch.isfinite(ref32) & torch.isfinite(terms)
