@@ -138,6 +138,27 @@ class LoraProj(ctypes.Structure):
 
 
 _lib = None
+_torch_mod = None
+
+
+def _torch():
+    """torch, imported on the first device call (the host entry points need
+    none of it); a call costs no import statement after that."""
+    global _torch_mod
+    if _torch_mod is None:
+        import torch
+
+        _torch_mod = torch
+    return _torch_mod
+
+
+
+def _current_stream() -> int:
+    """The handle of torch's current stream on the current device (without
+    building a Stream object, where this torch has the call for it)."""
+    cuda = _torch().cuda
+    raw = getattr(_torch_mod._C, "_cuda_getCurrentRawStream", None)
+    return cuda.current_stream().cuda_stream if raw is None else raw(cuda.current_device())
 
 
 def header_functions() -> list[str]:
@@ -232,40 +253,46 @@ def kernel_names() -> list[str]:
     return [L.glacier_attn_kernel_name(i).decode() for i in range(L.glacier_attn_kernel_count())]
 
 
+def _label(name):
+    """An argument's name: text, or (i, key) of projection i, put together only
+    when a message needs it."""
+    return name if isinstance(name, str) else f"proj[{name[0]}].{name[1]}"
+
+
 def _need(t, name, shape, dtype=None, like=None):
     """Checks a device tensor against what the descriptor promises the kernels
     (shape, dtype, contiguity, device) before its pointer crosses the ABI: a
     mismatched tensor would otherwise become an out-of-bounds device access.
     `like` gives the dtype and device of a reference tensor."""
     if t is None:
-        raise TypeError(f"{name} is required")
-    if tuple(t.shape) != tuple(shape):
-        raise TypeError(f"{name} must have shape {tuple(shape)}, got {tuple(t.shape)}")
+        raise TypeError(f"{_label(name)} is required")
+    if t.shape != shape:  # torch.Size compares as a tuple
+        raise TypeError(f"{_label(name)} must have shape {tuple(shape)}, got {tuple(t.shape)}")
     want = like.dtype if like is not None else dtype
     if want is not None and t.dtype != want:
-        raise TypeError(f"{name} must be {want}, got {t.dtype}")
+        raise TypeError(f"{_label(name)} must be {want}, got {t.dtype}")
     if not t.is_contiguous():
-        raise TypeError(f"{name} must be contiguous")
+        raise TypeError(f"{_label(name)} must be contiguous")
 
 
 def _on_gpu(*named):
     """Every given (name, tensor) on the GPU, on the first one's device."""
-    dev = None
+    index = first = None
     for name, t in named:
         if t is None:
             continue
         if not t.is_cuda:
-            raise TypeError(f"{name} must be a GPU tensor")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise TypeError(f"{name} must be on {dev}, got {t.device}")
+            raise TypeError(f"{_label(name)} must be a GPU tensor")
+        if first is None:
+            index, first = t.get_device(), t
+        elif t.get_device() != index:
+            raise TypeError(f"{_label(name)} must be on {first.device}, got {t.device}")
 
 
 def check_forward_args(q, k, v, out=None, lse=None, q_rot=None, k_rot=None):
     """The forward's tensors: q [T,Hq,D], k and v [T,Hkv,D] of q's dtype;
     out and q_rot like q, k_rot like k, lse float32 [Hq,T]."""
-    import torch
+    torch = _torch()
 
     if q.dim() != 3 or k.dim() != 3:
         raise TypeError("q must be [T, Hq, D] and k [T, Hkv, D]")
@@ -287,7 +314,7 @@ def check_forward_args(q, k, v, out=None, lse=None, q_rot=None, k_rot=None):
 def check_backward_args(d_out, q_rot, k_rot, v, out, lse, dq=None, dk=None, dv=None):
     """The backward's tensors: d_out, q_rot, out, dq [T,Hq,D]; k_rot, v, dk,
     dv [T,Hkv,D], all of q_rot's dtype; lse float32 [Hq,T]."""
-    import torch
+    torch = _torch()
 
     if q_rot.dim() != 3 or k_rot.dim() != 3:
         raise TypeError("q_rot must be [T, Hq, D] and k_rot [T, Hkv, D]")
@@ -308,33 +335,38 @@ def check_proj_args(x, projs, rank, backward):
     """x [T, in]; per projection w [out, in] of x's dtype, float32 bias
     [out], lora a [in, rank], b [rank, out], grad_a/grad_b like a/b, and y
     (forward) or dy (backward) [T, out] of x's dtype."""
-    import torch
+    torch = _torch()
 
     if x.dim() != 2:
         raise TypeError("x must be [T, in]")
     T, n_in = x.shape
     _need(x, "x", (T, n_in), dtype=x.dtype)
+    f32 = torch.float32
+    io = "dy" if backward else "y"
+    on_gpu = [("x", x)]
     for i, pr in enumerate(projs):
-        w = pr.get("w")
+        get = pr.get
+        w = get("w")
         if w is None or w.dim() != 2:
             raise TypeError(f"proj[{i}].w must be a [out, in] tensor")
         n_out = w.shape[0]
-        _need(w, f"proj[{i}].w", (n_out, n_in), like=x)
-        f32 = {"bias": (n_out,), "a": (n_in, rank), "b": (rank, n_out),
-               "grad_a": (n_in, rank), "grad_b": (rank, n_out)}
-        for key, shape in f32.items():
-            if pr.get(key) is not None:
-                _need(pr[key], f"proj[{i}].{key}", shape, dtype=torch.float32)
-        io = "dy" if backward else "y"
-        if backward or pr.get(io) is not None:
-            _need(pr.get(io), f"proj[{i}].{io}", (T, n_out), like=x)
-    _on_gpu(("x", x), *[(f"proj[{i}].{key}", pr.get(key)) for i, pr in enumerate(projs)
-                        for key in ("w", "bias", "a", "b", "grad_a", "grad_b", "y", "dy")])
+        _need(w, (i, "w"), (n_out, n_in), like=x)
+        for key, shape in (("bias", (n_out,)), ("a", (n_in, rank)), ("b", (rank, n_out)),
+                           ("grad_a", (n_in, rank)), ("grad_b", (rank, n_out))):
+            t = get(key)
+            if t is not None:
+                _need(t, (i, key), shape, dtype=f32)
+        t = get(io)
+        if backward or t is not None:
+            _need(t, (i, io), (T, n_out), like=x)
+        for key in ("w", "bias", "a", "b", "grad_a", "grad_b", "y", "dy"):
+            on_gpu.append(((i, key), get(key)))
+    _on_gpu(*on_gpu)
 
 
 def check_norm_args(x, weight, d_weight=None):
     """weight (and d_weight) float32 [n] for x [rows, n]."""
-    import torch
+    torch = _torch()
 
     n = x.shape[1]
     _need(weight, "weight", (n,), dtype=torch.float32)
@@ -418,19 +450,18 @@ class GpuAttentionEngine:
         return desc, keep
 
     def _bind_stream(self):
-        import torch
-
-        _check(load().glacier_attn_set_stream(self._h, ctypes.c_void_p(
-            torch.cuda.current_stream().cuda_stream)))
+        rc = load().glacier_attn_set_stream(self._h, _current_stream())
+        if rc != OK:
+            _check(rc)
 
     @staticmethod
     def _ptr(t):
-        return None if t is None else ctypes.c_void_p(t.data_ptr())
+        """The argument of a void* parameter: an address, or None for NULL."""
+        return None if t is None else t.data_ptr()
 
     @staticmethod
     def _io_of(t):
-        import torch
-
+        torch = _torch()
         if t.dtype == torch.float32:
             return IO_F32
         if t.dtype == torch.bfloat16:
@@ -441,7 +472,7 @@ class GpuAttentionEngine:
                 out=None, lse=None, q_rot=None, k_rot=None):
         """q [T,Hq,D], k/v [T,Hkv,D] (pre-RoPE, on the GPU, float32 or bfloat16).
         Returns (out, lse, q_rot, k_rot); the last three are None unless save."""
-        import torch
+        torch = _torch()
 
         prec = self.precision if precision is None else precision
         check_forward_args(q, k, v, out, lse if save else None, q_rot if save else None,
@@ -466,7 +497,7 @@ class GpuAttentionEngine:
     def backward(self, d_out, q_rot, k_rot, v, out, lse, rope_freq_base, precision=None,
                  cu_seqlens=None, dq=None, dk=None, dv=None):
         """Returns (dq, dk, dv); dq/dk w.r.t. the pre-RoPE q/k."""
-        import torch
+        torch = _torch()
 
         prec = self.precision if precision is None else precision
         check_backward_args(d_out, q_rot, k_rot, v, out, lse, dq, dk, dv)
@@ -575,40 +606,21 @@ class GpuAttentionEngine:
         p = GpuAttentionEngine._ptr
         for i, pr in enumerate(projs):
             w = pr["w"]
-            if not (w.is_cuda and w.is_contiguous() and w.dtype == x.dtype and w.dim() == 2
-                    and w.shape[1] == x.shape[1]):
-                raise TypeError("w must be a contiguous [out, in] GPU tensor of x's dtype")
-            for key in ("bias", "a", "b", "grad_a", "grad_b"):
-                t = pr.get(key)
-                if t is not None and not (t.is_cuda and t.is_contiguous() and t.dtype.is_floating_point
-                                          and t.element_size() == 4):
-                    raise TypeError(f"{key} must be a contiguous float32 GPU tensor")
-            e = arr[i]
-            e.w = p(w).value
-            e.bias = None if pr.get("bias") is None else p(pr["bias"]).value
-            e.lora_a = None if pr.get("a") is None else p(pr["a"]).value
-            e.lora_b = None if pr.get("b") is None else p(pr["b"]).value
-            e.scaling = float(pr.get("scaling", 0.0))
-            e.out_features = int(w.shape[0])
-            e.y = None if pr.get("y") is None else p(pr["y"]).value
-            e.dy = None if pr.get("dy") is None else p(pr["dy"]).value
-            e.grad_a = None if pr.get("grad_a") is None else p(pr["grad_a"]).value
-            e.grad_b = None if pr.get("grad_b") is None else p(pr["grad_b"]).value
+            get = pr.get
+            arr[i] = (p(w), p(get("bias")), p(get("a")), p(get("b")), float(get("scaling", 0.0)),
+                      int(w.shape[0]), p(get("y")), p(get("dy")), p(get("grad_a")), p(get("grad_b")))
         return arr
 
     def _proj_desc(self, x, rank, precision):
-        desc = ProjDesc()
-        desc.total_tokens, desc.in_features = int(x.shape[0]), int(x.shape[1])
-        desc.rank = int(rank)
-        desc.precision = int(self.precision if precision is None else precision)
-        desc.io_dtype = self._io_of(x)
-        return desc
+        T, n_in = x.shape
+        return ProjDesc(T, n_in, int(rank), int(self.precision if precision is None else precision),
+                        self._io_of(x))
 
     def proj_forward(self, x, projs, rank=0, precision=None):
         """x [T, in] (GPU, float32 or bfloat16).  projs: dicts with w [out, in]
         (x's dtype), optional bias [out], a [in, rank], b [rank, out] (float32),
         scaling, and optionally y [T, out] to write.  Returns the list of y."""
-        import torch
+        torch = _torch()
 
         if not (x.is_cuda and x.is_contiguous() and x.dim() == 2):
             raise TypeError("x must be a contiguous [T, in] GPU tensor")
@@ -626,7 +638,7 @@ class GpuAttentionEngine:
         """projs as for proj_forward with dy [T, out] (x's dtype) and optional
         float32 grad_a [in, rank] / grad_b [rank, out] accumulators (added to).
         Returns dx [T, in] (overwritten)."""
-        import torch
+        torch = _torch()
 
         if not (x.is_cuda and x.is_contiguous() and x.dim() == 2):
             raise TypeError("x must be a contiguous [T, in] GPU tensor")
@@ -646,11 +658,8 @@ class GpuAttentionEngine:
     def _norm_desc(self, x, eps):
         if not (x.is_cuda and x.is_contiguous() and x.dim() == 2):
             raise TypeError("x must be a contiguous [rows, n] GPU tensor")
-        desc = NormDesc()
-        desc.rows, desc.n = int(x.shape[0]), int(x.shape[1])
-        desc.io_dtype = self._io_of(x)
-        desc.eps = float(eps)
-        return desc
+        rows, n = x.shape
+        return NormDesc(rows, n, self._io_of(x), eps)
 
     @staticmethod
     def _like(t, ref, name):
@@ -662,7 +671,7 @@ class GpuAttentionEngine:
         """x1 = x + delta, y = RMSNorm(x1) weight (delta None: y = RMSNorm(x)
         weight and x1 is None).  x, delta [rows, n] float32 or bfloat16, weight
         [n] float32.  Returns (x1, y)."""
-        import torch
+        torch = _torch()
 
         desc = self._norm_desc(x, eps)
         check_norm_args(x, weight)
@@ -681,7 +690,7 @@ class GpuAttentionEngine:
     def rmsnorm_backward(self, dy, x, weight, eps, d_residual=None, dx=None, d_weight=None):
         """dx = RMSNormBackward(dy; x, weight) + d_residual; d_weight (float32
         [n], optional) is accumulated.  Returns dx."""
-        import torch
+        torch = _torch()
 
         desc = self._norm_desc(x, eps)
         check_norm_args(x, weight, d_weight)
@@ -735,7 +744,7 @@ class GpuAttentionEngine:
     def lmhead_loss_and_grad(self, hidden, targets, weight, d_hidden=None, precision=None):
         """As lmhead_loss, plus d_hidden [T, hidden] (overwritten).  Returns
         (loss, n_valid, d_hidden)."""
-        import torch
+        torch = _torch()
 
         d_hidden = torch.empty_like(hidden) if d_hidden is None else d_hidden
         loss, nv = self._lmhead(hidden, targets, weight, d_hidden, True, precision)
