@@ -91,12 +91,22 @@ __device__ inline void write_acc_block(unsigned addr, const f32x4 (&o)[NDB][QB],
 // arrive preloaded in SGPRs (-amdgpu-kernarg-preload-count, build.py), so the
 // K/V and Q loads issue without waiting for the kernarg segment.  The sine
 // table starts sin_off floats after the cosine table.
-template <typename IO, int D, bool VARLEN, int QB>
+//
+// RK (bf16 tensors, sequences of at most kFwdWaves * kChunk tokens): kc is the
+// caller's K before the rotation.  Each wave then has one chunk at most and
+// turns it in its own LDS ring, as rope_k would have (the same fp32 rotation of
+// the same values, rounded once), and the workgroup of a sequence's last rows
+// and of the group's first head writes k_rot.  That is the rotation done again
+// by every workgroup of a KV head, about 0.5 us of a short call, against
+// rope_k's launch of 2-2.5 us; with more than one chunk per wave it grows with
+// the sequence (2.9 us at 512 tokens) and the separate kernel stays.
+template <typename IO, int D, bool VARLEN, int QB, bool RK>
 __global__ __launch_bounds__(kFwdWaves * 64) void attn_fwd_kernel_ks(
     int total_tokens, int n_heads_kv, int group, int sin_off, const bf16* __restrict__ kc,
     const bf16* __restrict__ v, const TileDesc* __restrict__ tiles, const IO* __restrict__ q,
     const float* __restrict__ cos_t, IO* __restrict__ out, float* __restrict__ lse,
-    IO* __restrict__ q_rot, float scale_log2) {
+    IO* __restrict__ q_rot, float scale_log2, bf16* __restrict__ k_rot) {
+  static_assert(!RK || std::is_same_v<IO, bf16>, "the chunks are the caller's K as it is");
   using M = Mfma<bf16>;
   using F = FwdLayout<D>;
   using Frag = M::Frag;
@@ -432,6 +442,46 @@ __global__ __launch_bounds__(kFwdWaves * 64) void attn_fwd_kernel_ks(
       else
         wait_vmcnt<NDMA / 2>();
       GL_STAMP(kKernFwd, 18);
+      if constexpr (RK) {
+        // lane pieces: row n / PPR, rotation pairs 8 (n % PPR) ..; rows past
+        // the sequence's end repeat its last row and are masked below
+        constexpr int KI = kChunk * PPR / 64;
+        bf16x8 x0[KI], x1[KI];
+        float kc_[KI][8], ks_[KI][8];
+        bool write[KI];
+        bf16* at[KI][2];
+        const bool last = k_rot != nullptr && blockIdx.x == 0 && q0 + nq == td.len;
+#pragma unroll
+        for (int n = 0; n < KI; ++n) {
+          const int idx = lane + 64 * n, r = idx / PPR, j = idx % PPR;
+          const int pos = kChunk * w + r, sw = swz<D>(r);
+          write[n] = last && pos < td.len;
+          at[n][0] = kring + r * D + 8 * (j ^ sw);
+          at[n][1] = kring + r * D + 8 * ((PPR + j) ^ sw);
+          x0[n] = *reinterpret_cast<const bf16x8*>(at[n][0]);
+          x1[n] = *reinterpret_cast<const bf16x8*>(at[n][1]);
+          const long ti = (long)min(pos, td.len - 1) * H + 8 * j;
+          load8(cos_t + ti, kc_[n]);
+          load8(sin_t + ti, ks_[n]);
+        }
+#pragma unroll
+        for (int n = 0; n < KI; ++n) {
+          float y0[8], y1[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) rope_fwd((float)x0[n][e], (float)x1[n][e], kc_[n][e], ks_[n][e], y0[e], y1[e]);
+          store8(at[n][0], y0);
+          store8(at[n][1], y1);
+          if (write[n]) {
+            const int idx = lane + 64 * n;
+            bf16* dst = k_rot + ((long)(td.tok0 + kChunk * w + idx / PPR) * n_heads_kv + kvh) * D + 8 * (idx % PPR);
+            store8(dst, y0);
+            store8(dst + H, y1);
+          }
+        }
+        // the rotated rows are in LDS before the fragment reads below, which
+        // the compiler does not see
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
       bf16x8 kf[NKD][2];
 #pragma unroll
       for (int kk = 0; kk < NKD; ++kk) {
@@ -601,13 +651,29 @@ __global__ __launch_bounds__(kFwdWaves * 64) void attn_fwd_kernel_ks(
 
 }  // namespace
 
+bool fwd_rotates_k(const FwdLaunch& a, int max_len) {
+  // two arrays, not one turned in place: other workgroups still read K
+  return a.io_bf16 && (a.head_dim == 64 || a.head_dim == 128) && a.tile_rows != 64 &&
+         max_len <= kFwdWaves * kChunk && a.k_rot != a.k;
+}
+
 template <typename IO, int D>
 hipError_t launch_fwd_bf16(const FwdLaunch& a, hipStream_t st, KernelTimer* tm) {
   // 32-query workgroups (two per table entry) when the launch is short of CUs
   const int nsub = a.tile_rows == 16 ? 4 : a.tile_rows == 32 ? 2 : 1;  // workgroups per 64-row tile
-  auto fn = a.single_seq ? attn_fwd_kernel_ks<IO, D, false, 4> : attn_fwd_kernel_ks<IO, D, true, 4>;
-  if (nsub == 2) fn = a.single_seq ? attn_fwd_kernel_ks<IO, D, false, 2> : attn_fwd_kernel_ks<IO, D, true, 2>;
-  if (nsub == 4) fn = a.single_seq ? attn_fwd_kernel_ks<IO, D, false, 1> : attn_fwd_kernel_ks<IO, D, true, 1>;
+  auto pick = [&](auto qb, auto rk) {
+    constexpr int QB = decltype(qb)::value;
+    constexpr bool RK = decltype(rk)::value;
+    return a.single_seq ? attn_fwd_kernel_ks<IO, D, false, QB, RK> : attn_fwd_kernel_ks<IO, D, true, QB, RK>;
+  };
+  using std::integral_constant;
+  auto fn = pick(integral_constant<int, 4>{}, std::false_type{});
+  if (nsub == 2) fn = pick(integral_constant<int, 2>{}, std::false_type{});
+  if (nsub == 4) fn = pick(integral_constant<int, 1>{}, std::false_type{});
+  if constexpr (std::is_same_v<IO, bf16>) {
+    if (a.rotate_k) fn = nsub == 4 ? pick(integral_constant<int, 1>{}, std::true_type{})
+                                   : pick(integral_constant<int, 2>{}, std::true_type{});
+  }
   constexpr size_t lds = FwdLayout<D>::BYTES;
   GL_CHECK(allow_lds(fn, lds));
   // the tables are one allocation: the sine table's offset in floats
@@ -617,10 +683,11 @@ hipError_t launch_fwd_bf16(const FwdLaunch& a, hipStream_t st, KernelTimer* tm) 
   LaunchTiming t(tm, kKernFwd);
   GL_LAUNCH(t, fn, dim3(group, a.n_heads_kv, a.n_tiles * nsub), dim3(kFwdWaves * 64), lds,
                         st, a.total_tokens, a.n_heads_kv, group, static_cast<int>(sin_off),
-                        static_cast<const bf16*>(a.kc),
+                        static_cast<const bf16*>(a.rotate_k ? a.k : a.kc),
                         static_cast<const bf16*>(a.vc != nullptr ? a.vc : a.v), a.tiles_fwd,
                         static_cast<const IO*>(a.q), a.cos_t, static_cast<IO*>(a.out), a.lse,
-                        static_cast<IO*>(a.q_rot), a.scale_log2);
+                        static_cast<IO*>(a.q_rot), a.scale_log2,
+                        a.rotate_k ? static_cast<bf16*>(a.k_rot) : nullptr);
   GL_CHECK(hipGetLastError());
   t.launched();
   return hipSuccess;

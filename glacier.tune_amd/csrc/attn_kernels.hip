@@ -1059,7 +1059,7 @@ template <typename IO, typename T, int D>
 hipError_t forward_impl(const FwdLaunch& a, hipStream_t st, KernelTimer* tm) {
   const dim3 blk(kThreads);
   T* kc = static_cast<T*>(a.kc);
-  {
+  if (!a.rotate_k) {
     const long n = (long)a.total_tokens * (D / 16);
     const dim3 grid(static_cast<unsigned>((n + kThreads - 1) / kThreads), a.n_heads_kv);
     IO* k_rot = static_cast<IO*>(a.k_rot);

@@ -145,6 +145,7 @@ struct FwdLaunch {
   // query rows per workgroup of the bf16 forward: 64, or 32 or 16 (two or
   // four workgroups per tile) for launches that would otherwise leave CUs idle
   int tile_rows;
+  bool rotate_k;                 // the bf16 forward turns K itself (no rope_k launch)
   float scale_log2;
   const void *q, *k, *v;
   void *out, *q_rot, *k_rot;
@@ -155,6 +156,9 @@ struct FwdLaunch {
   const int32_t* pos_of;         // position of each token inside its sequence
   const float *cos_t, *sin_t;    // [max len][D/2]
 };
+// Whether the bf16 forward (attn_fwd.hip) takes the launch with rotate_k, for
+// sequences of at most max_len tokens; everything but kc is filled in.
+bool fwd_rotates_k(const FwdLaunch& a, int max_len);
 
 // Backward kernel choice for bf16 tensors.  kBwdAuto takes the 32x32x16-MFMA
 // kernel (attn_bwd3.hip) once the call's work, query heads times causal pairs

@@ -571,9 +571,13 @@ class GpuAttentionEngine {
     a.scale_log2 = kLog2e / std::sqrt(static_cast<float>(dreal));
     a.q = q; a.k = k; a.v = v;
     a.out = out; a.lse = lse; a.q_rot = q_rot; a.k_rot = k_rot;
+    a.rotate_k = fwd_rotates_k(a, ts.max_len);
     // The attention kernel reads rotated K in the compute dtype: the caller's
-    // k_rot when it is that dtype, else library scratch.
-    if (k_rot != nullptr && esz == io_esz)
+    // k_rot when it is that dtype, else library scratch; none when it turns K
+    // itself.
+    if (a.rotate_k)
+      a.kc = nullptr;
+    else if (k_rot != nullptr && esz == io_esz)
       a.kc = k_rot;
     else
       a.kc = kc_.ensure((size_t)s.total_tokens * s.n_heads_kv * s.head_dim * esz, "K scratch");
