@@ -267,10 +267,18 @@ hipError_t launch_bwd3(const BwdLaunch& a, hipStream_t st, KernelTimer* tm);
 // elements padded to dp (a built size) with the rotation halves kept apart
 // (columns 0 .. d/2 - 1 and dp/2 .. dp/2 + d/2 - 1, an odd d's last element
 // at d/2, zeros elsewhere), and back; rows: tokens x heads; bf16 or float.
-hipError_t launch_pad_rows(bool io_bf16, const void* src, void* dst, long rows, int d, int dp,
-                           hipStream_t st);
-hipError_t launch_unpad_rows(bool io_bf16, const void* src, void* dst, long rows, int d, int dp,
-                             hipStream_t st);
+struct PadJob {
+  const void* src;
+  void* dst;
+  long rows;
+};
+struct PadCall {  // the tensors of one direction
+  PadJob j[5];
+  int n;
+  void add(const void* src, void* dst, long rows) { j[n++] = PadJob{src, dst, rows}; }
+};
+hipError_t launch_pad_rows(bool io_bf16, const PadCall& a, int d, int dp, hipStream_t st);
+hipError_t launch_unpad_rows(bool io_bf16, const PadCall& a, int d, int dp, hipStream_t st);
 
 // Kernels whose dynamic LDS exceeds 64 KB must say so before their launch.
 template <typename F>

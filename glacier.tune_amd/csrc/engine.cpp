@@ -541,16 +541,20 @@ class GpuAttentionEngine {
       void* op = pad_o_.ensure(rq * dp * esz, "padded out");
       void* qrp = q_rot != nullptr ? pad_qr_.ensure(rq * dp * esz, "padded q_rot") : nullptr;
       void* krp = k_rot != nullptr ? pad_kr_.ensure(rk * dp * esz, "padded k_rot") : nullptr;
-      check_hip(launch_pad_rows(bf, q, qp, rq, d, dp, stream()), "pad q");
-      check_hip(launch_pad_rows(bf, k, kp, rk, d, dp, stream()), "pad k");
-      check_hip(launch_pad_rows(bf, v, vp, rk, d, dp, stream()), "pad v");
+      PadCall pad{};
+      pad.add(q, qp, rq);
+      pad.add(k, kp, rk);
+      pad.add(v, vp, rk);
+      check_hip(launch_pad_rows(bf, pad, d, dp, stream()), "pad rows");
       Shape sp = s;
       sp.head_dim = dp;
       sp.real_dim = d;
       LaunchAttnTrainFwd(sp, qp, kp, vp, op, lse, qrp, krp);
-      check_hip(launch_unpad_rows(bf, op, out, rq, d, dp, stream()), "unpad out");
-      if (q_rot != nullptr) check_hip(launch_unpad_rows(bf, qrp, q_rot, rq, d, dp, stream()), "unpad q_rot");
-      if (k_rot != nullptr) check_hip(launch_unpad_rows(bf, krp, k_rot, rk, d, dp, stream()), "unpad k_rot");
+      PadCall back{};
+      back.add(op, out, rq);
+      if (q_rot != nullptr) back.add(qrp, q_rot, rq);
+      if (k_rot != nullptr) back.add(krp, k_rot, rk);
+      check_hip(launch_unpad_rows(bf, back, d, dp, stream()), "unpad rows");
       return;
     }
     const int dreal = s.real_dim > 0 ? s.real_dim : s.head_dim;
@@ -667,18 +671,22 @@ class GpuAttentionEngine {
       void* dqp = pad_dq_.ensure(rq * dp * esz, "padded dq");
       void* dkp = pad_dk_.ensure(rk * dp * esz, "padded dk");
       void* dvp = pad_dv_.ensure(rk * dp * esz, "padded dv");
-      check_hip(launch_pad_rows(bf, d_out, dop, rq, d, dp, stream()), "pad d_out");
-      check_hip(launch_pad_rows(bf, q_rot, qrp, rq, d, dp, stream()), "pad q_rot");
-      check_hip(launch_pad_rows(bf, k_rot, krp, rk, d, dp, stream()), "pad k_rot");
-      check_hip(launch_pad_rows(bf, v, vp, rk, d, dp, stream()), "pad v");
-      check_hip(launch_pad_rows(bf, out, op, rq, d, dp, stream()), "pad out");
+      PadCall pad{};
+      pad.add(d_out, dop, rq);
+      pad.add(q_rot, qrp, rq);
+      pad.add(k_rot, krp, rk);
+      pad.add(v, vp, rk);
+      pad.add(out, op, rq);
+      check_hip(launch_pad_rows(bf, pad, d, dp, stream()), "pad rows");
       Shape sp = s;
       sp.head_dim = dp;
       sp.real_dim = d;
       LaunchAttnTrainBwd(sp, dop, qrp, krp, vp, op, lse, dqp, dkp, dvp);
-      check_hip(launch_unpad_rows(bf, dqp, dq, rq, d, dp, stream()), "unpad dq");
-      check_hip(launch_unpad_rows(bf, dkp, dk, rk, d, dp, stream()), "unpad dk");
-      check_hip(launch_unpad_rows(bf, dvp, dv, rk, d, dp, stream()), "unpad dv");
+      PadCall back{};
+      back.add(dqp, dq, rq);
+      back.add(dkp, dk, rk);
+      back.add(dvp, dv, rk);
+      check_hip(launch_unpad_rows(bf, back, d, dp, stream()), "unpad rows");
       return;
     }
     const int dreal = s.real_dim > 0 ? s.real_dim : s.head_dim;
