@@ -918,11 +918,16 @@ __global__ __launch_bounds__((kThreads * bwd_groups<T, D>())) void attn_bwd_kern
 // (token, kv head) row, so a workgroup covers kRedThreads / (D / 8) rows.
 constexpr int kRedThreads = 128;
 
-// 4 consecutive partial elements (the tensors' dtype) as fp32.
-__device__ inline f32x4 load_partial4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
-__device__ inline f32x4 load_partial4(const bf16* p) {
-  const bf16x4 v = *reinterpret_cast<const bf16x4*>(p);
+// 4 consecutive partial elements, in the tensors' dtype (Raw4) and as fp32.
+template <typename IO>
+using Raw4 = IO __attribute__((ext_vector_type(4)));
+__device__ inline f32x4 as_f32(Raw4<float> v) { return v; }
+__device__ inline f32x4 as_f32(Raw4<bf16> v) {
   return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+}
+template <typename IO>
+__device__ inline Raw4<IO> load_partial4(const IO* p) {
+  return *reinterpret_cast<const Raw4<IO>*>(p);
 }
 
 // SPLIT: the call split dK/dV tiles (bf16 partials), so rows below
@@ -958,28 +963,33 @@ __global__ __launch_bounds__(kRedThreads) void attn_bwd_reduce_kernel(
   const IO* wkr2 = wk2 + ((long)tok * n_heads_q + (long)j * ratio) * D + p0;
   const IO* wvr2 = wv2 + ((long)tok * n_heads_q + (long)j * ratio) * D + p0;
   f32x4 k0 = {0.0f, 0.0f, 0.0f, 0.0f}, k1 = k0, v0 = k0, v1 = k0;
-  constexpr int RMAX = 8;
-  constexpr int RMAX2 = SPLIT ? RMAX : 1;
   const int nparts = (ratio + hstep - 1) / hstep;  // partials per row, at heads 0, hstep, ..
-  if (nparts <= RMAX) {
-    // Every head's partial in flight at once (a load per head that the sum
-    // waits on would cost one memory round trip per head), then the sum in
-    // ascending head order; heads past the group add nothing.
-    f32x4 pk0[RMAX], pk1[RMAX], pv0[RMAX], pv1[RMAX];
-    f32x4 qk0[RMAX2], qk1[RMAX2], qv0[RMAX2], qv1[RMAX2];
+  // Bound by the latency of the partials: those of up to eight heads are in
+  // flight at once, then summed in ascending head order; heads past the group
+  // add nothing.  The loaded registers stay in the tensors' dtype until the tie
+  // behind the last load: left to itself the compiler converts each load as it
+  // arrives at head sizes that are no power of two, one round trip per load
+  // (28 heads over 4, 100 tokens, head size 96: 14.6 us, 4.7 so).  A group of more
+  // than eight took one trip per head (32 heads over 2, 500 tokens, 64: 9.9 us,
+  // 4.8 so); a smaller one loads no more than it has (28 over 4 in pairs, 4096
+  // tokens, 128: 9.5 us with eight loads for its four, 7.8 so).
+  const auto sum_heads = [&](auto width, int h0) {
+    constexpr int R = decltype(width)::value, R2 = SPLIT ? R : 1;
+    Raw4<IO> pk0[R], pk1[R], pv0[R], pv1[R], qk0[R2], qk1[R2], qv0[R2], qv1[R2];
+    const int n = nparts - h0;
 #pragma unroll
-    for (int hh = 0; hh < RMAX; ++hh) {
-      const long o = (long)(hh < nparts ? hh * hstep : 0) * D;
+    for (int hh = 0; hh < R; ++hh) {
+      const long o = (long)(h0 + (hh < n ? hh : 0)) * hstep * D;
       pk0[hh] = load_partial4(wkr + o);
       pk1[hh] = load_partial4(wkr + o + H);
       pv0[hh] = load_partial4(wvr + o);
       pv1[hh] = load_partial4(wvr + o + H);
     }
-    if constexpr (RMAX2 == RMAX) {
+    if constexpr (SPLIT) {
       if (two) {
 #pragma unroll
-        for (int hh = 0; hh < RMAX; ++hh) {
-          const long o = (long)(hh < ratio ? hh : 0) * D;
+        for (int hh = 0; hh < R; ++hh) {
+          const long o = (long)(h0 + (hh < n ? hh : 0)) * hstep * D;
           qk0[hh] = load_partial4(wkr2 + o);
           qk1[hh] = load_partial4(wkr2 + o + H);
           qv0[hh] = load_partial4(wvr2 + o);
@@ -988,36 +998,32 @@ __global__ __launch_bounds__(kRedThreads) void attn_bwd_reduce_kernel(
       }
     }
 #pragma unroll
-    for (int hh = 0; hh < RMAX; ++hh) {
-      if (hh < nparts) {
-        k0 += pk0[hh];
-        k1 += pk1[hh];
-        v0 += pv0[hh];
-        v1 += pv1[hh];
-        if constexpr (RMAX2 == RMAX) {
+    for (int hh = 0; hh < R; ++hh)
+      asm volatile("" : "+v"(pk0[hh]), "+v"(pk1[hh]), "+v"(pv0[hh]), "+v"(pv1[hh]));
+#pragma unroll
+    for (int hh = 0; hh < R; ++hh) {
+      if (hh < n) {
+        k0 += as_f32(pk0[hh]);
+        k1 += as_f32(pk1[hh]);
+        v0 += as_f32(pv0[hh]);
+        v1 += as_f32(pv1[hh]);
+        if constexpr (SPLIT) {
           if (two) {
-            k0 += qk0[hh];
-            k1 += qk1[hh];
-            v0 += qv0[hh];
-            v1 += qv1[hh];
+            k0 += as_f32(qk0[hh]);
+            k1 += as_f32(qk1[hh]);
+            v0 += as_f32(qv0[hh]);
+            v1 += as_f32(qv1[hh]);
           }
         }
       }
     }
-  } else {
-    for (int hh = 0; hh < ratio; hh += hstep) {
-      k0 += load_partial4(wkr + (long)hh * D);
-      k1 += load_partial4(wkr + (long)hh * D + H);
-      v0 += load_partial4(wvr + (long)hh * D);
-      v1 += load_partial4(wvr + (long)hh * D + H);
-      if (two) {
-        k0 += load_partial4(wkr2 + (long)hh * D);
-        k1 += load_partial4(wkr2 + (long)hh * D + H);
-        v0 += load_partial4(wvr2 + (long)hh * D);
-        v1 += load_partial4(wvr2 + (long)hh * D + H);
-      }
-    }
-  }
+  };
+  if (nparts <= 2)
+    sum_heads(std::integral_constant<int, 2>{}, 0);
+  else if (nparts <= 4)
+    sum_heads(std::integral_constant<int, 4>{}, 0);
+  else
+    for (int h0 = 0; h0 < nparts; h0 += 8) sum_heads(std::integral_constant<int, 8>{}, h0);
   f32x4 y0, y1;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
