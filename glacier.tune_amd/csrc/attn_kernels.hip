@@ -963,23 +963,28 @@ __global__ __launch_bounds__(kRedThreads) void attn_bwd_reduce_kernel(
   const IO* wkr2 = wk2 + ((long)tok * n_heads_q + (long)j * ratio) * D + p0;
   const IO* wvr2 = wv2 + ((long)tok * n_heads_q + (long)j * ratio) * D + p0;
   f32x4 k0 = {0.0f, 0.0f, 0.0f, 0.0f}, k1 = k0, v0 = k0, v1 = k0;
-  const int nparts = (ratio + hstep - 1) / hstep;  // partials per row, at heads 0, hstep, ..
+  // partials per row, at heads 0, hstep, .. (hstep 1 or 2: no division before the loads)
+  const int nparts = (ratio + hstep - 1) >> (hstep - 1);
   // Bound by the latency of the partials: those of up to eight heads are in
   // flight at once, then summed in ascending head order; heads past the group
   // add nothing.  The loaded registers stay in the tensors' dtype until the tie
   // behind the last load: left to itself the compiler converts each load as it
   // arrives at head sizes that are no power of two, one round trip per load
-  // (28 heads over 4, 100 tokens, head size 96: 14.6 us, 4.7 so).  A group of more
+  // (28 heads over 4, 100 tokens, head size 96: 14.6 us, 4.6 so).  A group of more
   // than eight took one trip per head (32 heads over 2, 500 tokens, 64: 9.9 us,
-  // 4.8 so); a smaller one loads no more than it has (28 over 4 in pairs, 4096
-  // tokens, 128: 9.5 us with eight loads for its four, 7.8 so).
+  // 4.1 so); a smaller one loads no more than it has (28 over 4 in pairs, 4096
+  // tokens, 128: 9.5 us with eight loads for its four, 8 so).  Five to eight come
+  // first and straight through: at this length a jump over the other widths and a
+  // loop's 64-bit offsets showed (0.3 us of a 36 us step).
+  const int step = hstep * D;  // elements from partial to partial
   const auto sum_heads = [&](auto width, int h0) {
     constexpr int R = decltype(width)::value, R2 = SPLIT ? R : 1;
     Raw4<IO> pk0[R], pk1[R], pv0[R], pv1[R], qk0[R2], qk1[R2], qv0[R2], qv1[R2];
     const int n = nparts - h0;
+    const long base = (long)h0 * step;
 #pragma unroll
     for (int hh = 0; hh < R; ++hh) {
-      const long o = (long)(h0 + (hh < n ? hh : 0)) * hstep * D;
+      const long o = base + (hh < n ? hh * step : 0);
       pk0[hh] = load_partial4(wkr + o);
       pk1[hh] = load_partial4(wkr + o + H);
       pv0[hh] = load_partial4(wvr + o);
@@ -989,7 +994,7 @@ __global__ __launch_bounds__(kRedThreads) void attn_bwd_reduce_kernel(
       if (two) {
 #pragma unroll
         for (int hh = 0; hh < R; ++hh) {
-          const long o = (long)(h0 + (hh < n ? hh : 0)) * hstep * D;
+          const long o = base + (hh < n ? hh * step : 0);
           qk0[hh] = load_partial4(wkr2 + o);
           qk1[hh] = load_partial4(wkr2 + o + H);
           qv0[hh] = load_partial4(wvr2 + o);
@@ -1018,12 +1023,15 @@ __global__ __launch_bounds__(kRedThreads) void attn_bwd_reduce_kernel(
       }
     }
   };
-  if (nparts <= 2)
-    sum_heads(std::integral_constant<int, 2>{}, 0);
-  else if (nparts <= 4)
+  if (nparts > 4) [[likely]] {
+    sum_heads(std::integral_constant<int, 8>{}, 0);
+    for (int h0 = 8; h0 < nparts; h0 += 8) [[unlikely]]
+      sum_heads(std::integral_constant<int, 8>{}, h0);
+  } else if (nparts > 2) {
     sum_heads(std::integral_constant<int, 4>{}, 0);
-  else
-    for (int h0 = 0; h0 < nparts; h0 += 8) sum_heads(std::integral_constant<int, 8>{}, h0);
+  } else {
+    sum_heads(std::integral_constant<int, 2>{}, 0);
+  }
   f32x4 y0, y1;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
