@@ -43,7 +43,7 @@ namespace {
 // The low-rank product is a further stretch of the same reduction: both fp32
 // operands are split in three bf16 terms (split3.hpp), laid out six times r
 // wide by lowrank_split so that one bf16 product sums the six term products.
-// A call that holds a non-finite value there (its marks, `odd`) takes fp32
+// A call that holds a value without a split there (its marks, `odd`) takes fp32
 // MFMAs for it instead.  The bias starts the accumulators, and the bf16
 // conversion happens as the tile leaves through LDS in whole row pieces.  So
 // no fp32 product goes to memory and back.
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_kernel(const GemmCall a) 
   const int nf = NN ? a.K : a.j[z].n;  // features of the output
   const int lane = threadIdx.x & 63, w = wave_id();
   const int wf = w % WF, wt = w / WF % WT, wk = w / (WF * WT);
-  // a non-finite value among the low-rank operands: see below
+  // a value without a split among the low-rank operands: see below
   bool slow = false;
   for (int i = lane; i < a.n_odd; i += 64) slow |= a.odd[i] != 0;
   slow = __any(slow);
@@ -254,8 +254,8 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_kernel(const GemmCall a) 
       for (int tb = 0; tb < TB; ++tb) acc[fb][tb][e] = b;
     }
   if (slow && wk == 0) {
-    // the low-rank products of a call with non-finite values, which have no
-    // split terms: sum over the terms of (s L [T][r]) V, V = B [r][n]
+    // the low-rank products of a call with values that have no split terms:
+    // sum over the terms of (s L [T][r]) V, V = B [r][n]
     // (forward) or A^T with A [K][r], on fp32 MFMAs
     for (int p = NN ? 0 : z; p < (NN ? a.n : z + 1); ++p) {
       const GemmJob& job = a.j[p];
@@ -448,8 +448,7 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_kernel(const GemmCall a) 
 // 64-byte rows, backward A 64-feature sub-tiles), two buffers, one barrier a
 // stage.  Loads are unconditional at clamped addresses; elements past the
 // reduction are zeroed in A, rows past an edge reach no stored result.
-// A tile that meets an element without a split (not finite, or rounding to
-// infinity) is done over on fp32 MFMAs, straight from global memory.
+// A tile that meets an element without a split is done over on fp32 MFMAs, straight from global memory.
 //
 // What bounds it: at one small tile per CU the chain of a stage (split, LDS,
 // six dependent products: 0.75 us); once the chip is full the six products
@@ -615,7 +614,7 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
       for (int i = 0; i < LB; ++i) low_b(tid + kGThreads * i, st * KT, p.b[i]);
     }
   };
-  bool bad = false;
+  SplitMarks mark;
   // piece idx of operand `b` (0: A, 1: B) into the three planes of a buffer
   auto put = [&](unsigned char* base, int idx, bool b, Piece& q) {
 #pragma unroll
@@ -624,7 +623,7 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
       q.x[e] = e < q.valid ? q.x[e] : 0.0f;
     }
     Split3 s;
-    bad |= s.set(q.x);
+    s.set(q.x, mark);
     int off;
     if (NN && !b) {
       const int r = (idx >> 3) % 32;
@@ -770,7 +769,7 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
     });
     settle(acc);
   }
-  if (__syncthreads_or(bad)) {
+  if (__syncthreads_or(mark.bad())) {
     // the same sums on fp32 MFMAs: lane l supplies A[row l % 32][k + l / 32]
     // and B's column likewise; group 0 sums everything
     clear();

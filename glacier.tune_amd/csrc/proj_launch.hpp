@@ -36,7 +36,7 @@ struct ProjLaunch {
   // scratch, sized by proj_scratch_need
   float* lowrank;  // [slot][T][r] X A_p and dY_p B_p^T
   void* terms;     // fused calls: the split terms (bf16) of the adapters, then of s L
-  int* odd;        // fused calls: non-finite marks (SplitCall)
+  int* odd;        // fused calls: marks of values without a split (SplitCall)
 };
 
 // ---- bf16 tensors: base products, low-rank delta, bias and conversion in ----
@@ -57,7 +57,7 @@ struct GemmJob {
 };
 struct GemmCall {
   void* dx;         // backward: dX [T][K] (bf16)
-  const int* odd;   // [n_odd] marks: the low-rank operands hold non-finite values
+  const int* odd;   // [n_odd] marks: the low-rank operands hold values without a split
   int n_odd;
   int T, K, rank, n;
   int ftiles;       // set by launch_gemm

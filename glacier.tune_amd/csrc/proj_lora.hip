@@ -127,28 +127,27 @@ struct SplitCall {
   TermJob v[kMaxProj];
   int n, nv, across;
   int slabs;   // row slabs of a job
-  int* odd;    // [kTermBlocks], then [n][slabs]: a non-finite value among what that workgroup wrote
+  int* odd;    // [kTermBlocks], then [n][slabs]: a value without split terms among what that workgroup wrote
 };
 
-__device__ inline bool not_finite(float x) { return (__float_as_uint(x) & 0x7f800000u) == 0x7f800000u; }
-
 // The six entries of a terms row for x: side 0 the adapters', side 1 (s L).
+// True if x has no split (split3.hpp): the entries are then meaningless.
 template <typename Put>
-__device__ inline void put_terms(float x, int side, Put&& put) {
+__device__ inline bool put_terms(float x, int side, Put&& put) {
   const bf16 h = (bf16)x;
   const float r1 = x - (float)h;
-  const bf16 m = (bf16)r1, l = (bf16)(r1 - (float)m);
+  const bf16 m = (bf16)r1;
+  const float r2 = r1 - (float)m;
+  const bf16 l = (bf16)r2;
   put(0, h);
   put(1, side ? m : h);
   put(2, side ? h : m);
   put(3, m);
   put(4, side ? l : h);
   put(5, side ? h : l);
+  const unsigned left = __float_as_uint(r2);
+  return (left & 0xffffu) != 0 || (left & 0x7f800000u) == 0x7f800000u;
 }
-
-// x has a split: its terms are finite (false also for a finite x that rounds
-// to infinity).
-[[maybe_unused]] __device__ inline bool has_split(float x) { return !not_finite((float)(bf16)x); }
 
 constexpr int kTermBlocks = 64;
 // Waves of a lowrank_split workgroup
@@ -204,26 +203,26 @@ __device__ inline void split_accumulate(const IO* const (&u)[RB], const float* _
       bool odd_u = false;
 #pragma unroll
       for (int b = 0; b < RB; ++b) {
-        float chk = 0.0f;  // NaN once an element of U is not finite
+        SplitMarks mark;  // bf16: NaN once an element is not finite
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           x[b][e] = (float)raw_at(ur[s][b][e / 4], e % 4);
           if constexpr (!kF32) {
             ub[b][e] = (bf16)x[b][e];
-            chk += 0.0f * x[b][e];
+            mark.sum += 0.0f * x[b][e];
           }
         }
-        if constexpr (kF32)
-          odd_u |= us[b].set(x[b]);
-        else
-          odd_u |= chk != chk;
+        if constexpr (kF32) us[b].set(x[b], mark);
+        odd_u |= mark.bad();
       }
 #pragma unroll
       for (int jt = 0; jt < NT; ++jt) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) vr[s][jt][e] = ok[e / 4] ? vr[s][jt][e] : 0.0f;
         Split3 v;
-        if (__any(v.set(vr[s][jt]) || odd_u)) {
+        SplitMarks mark;
+        v.set(vr[s][jt], mark);
+        if (__any(mark.bad() || odd_u)) {
 #pragma unroll
           for (int b = 0; b < RB; ++b)
 #pragma unroll
@@ -287,18 +286,14 @@ __global__ __launch_bounds__(64 * split_waves(NT, RB)) void lowrank_split_kernel
       if (!a.across && rank % 4 == 0) {  // four entries of a row in one store
         bf16x4 t4[6];
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-          odd |= !has_split(x[m]);
-          put_terms(x[m], 0, [&](int e, bf16 t) { t4[e][m] = t; });
-        }
+        for (int m = 0; m < 4; ++m) odd |= put_terms(x[m], 0, [&](int e, bf16 t) { t4[e][m] = t; });
 #pragma unroll
         for (int e = 0; e < 6; ++e) *reinterpret_cast<bf16x4*>(out + (long)f * P + e * rank + j0) = t4[e];
       } else {
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
           if (j0 + m >= rank) break;
-          odd |= !has_split(x[m]);
-          put_terms(x[m], 0, [&](int e, bf16 t) {
+          odd |= put_terms(x[m], 0, [&](int e, bf16 t) {
             const int q = e * rank + j0 + m;
             out[a.across ? (long)q * n + f : (long)f * P + q] = t;
           });
@@ -350,9 +345,7 @@ __global__ __launch_bounds__(64 * split_waves(NT, RB)) void lowrank_split_kernel
     job.l[(long)t * rank + j] = sum;
     if (job.terms == nullptr) continue;
     bf16* row = static_cast<bf16*>(job.terms) + (long)t * P;
-    const float x = job.s * sum;
-    odd |= !has_split(x);
-    put_terms(x, 1, [&](int e, bf16 v) { row[e * rank + j] = v; });
+    odd |= put_terms(job.s * sum, 1, [&](int e, bf16 v) { row[e * rank + j] = v; });
     if (j == 0)
       for (int e = 6 * rank; e < P; ++e) row[e] = (bf16)0.0f;
   }

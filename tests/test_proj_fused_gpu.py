@@ -178,3 +178,46 @@ def test_non_finite_values_pass_through(engines, dtype, where):
         ok = torch.isfinite(ref32) & torch.isfinite(terms)
         if ok.any():
             _check(got[ok], ref[ok], terms[ok], n_in, where)
+
+
+@pytest.mark.parametrize("T,n_in,outs,rank", [(201, 896, (896, 128), 8), (1100, 1024, (2048, 520), 16)])
+@pytest.mark.parametrize("where", ["x", "w", "a"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_small_values_keep_their_bits(engines, dtype, where, T, n_in, outs, rank):
+    """Operands down to 2^-118, whose last bits three bf16 terms do not reach
+    (split3.hpp): fp32 results stay within 2e-6 of float64 in the 2-norm (fp32
+    sums, the gate of the adapters' gradients), bf16 ones within 2^-8.  With
+    "a" only the low-rank product is left, on activations of about 2^-120 in
+    fp32 and, to show in bf16 results, 2^-130 in bf16 (19 bits in themselves)."""
+    print(f"[small values] {dtype} {where} T={T} in={n_in} outs={outs} rank={rank}", flush=True)
+    x, projs = _problem(T, n_in, outs, rank, dtype=dtype)
+    for p in projs:
+        p["bias"] = None
+    if where == "a":
+        x.mul_(2.0 ** -60)
+        for p in projs:
+            p["w"].zero_()
+        projs[0]["a"].mul_(2.0 ** (-60 if dtype == torch.float32 else -70))
+        projs[0]["b"].mul_(2.0 ** 30)
+    else:
+        for t in [x, *[p["dy"] for p in projs]] if where == "x" else [p["w"] for p in projs]:
+            t.mul_(2.0 ** -118)
+    if where == "w":
+        projs[0]["a"].mul_(2.0 ** -118)
+    p = projs[0]
+    ys = engines[dtype].proj_forward(x, projs, rank)
+    dx = engines[dtype].proj_backward(x, projs, rank)
+    xd, dy = x.double(), p["dy"].double()
+    low = xd @ p["a"].double()
+    y = xd @ p["w"].double().t() + 2.0 * low @ p["b"].double()
+    want_dx = sum(q["dy"].double() @ q["w"].double() for q in projs)
+    want_dx = want_dx + 2.0 * (dy @ p["b"].double().t()) @ p["a"].double().t()
+    gate = 2e-6 if dtype == torch.float32 else 2.0 ** -8
+    for got, want, within in ((ys[0], y, gate), (dx, want_dx, gate),
+                              (p["grad_b"], 2.0 * low.t() @ dy, gate if where == "a" else 2e-6)):
+        if float(want.abs().max()) < 2.0 ** -118:
+            continue  # results of few bits themselves
+        scale = 2.0 ** 100  # squares inside float64 either way; norms of small numbers stay normal
+        err = float(((got.double() - want) * scale).norm() / (want * scale).norm())
+        print(f"  {err:.2e} of {within:.2e}", flush=True)
+        assert err <= within
