@@ -652,9 +652,11 @@ __global__ __launch_bounds__(kFwdWaves * 64) void attn_fwd_kernel_ks(
 }  // namespace
 
 bool fwd_rotates_k(const FwdLaunch& a, int max_len) {
-  // two arrays, not one turned in place: other workgroups still read K
+  // two arrays, not one turned in place: other workgroups still read K; and K in
+  // whole 16-byte pieces, as the DMA moves it (rope_k's loads need no alignment)
   return a.io_bf16 && (a.head_dim == 64 || a.head_dim == 128) && a.tile_rows != 64 &&
-         max_len <= kFwdWaves * kChunk && a.k_rot != a.k;
+         max_len <= kFwdWaves * kChunk && a.k_rot != a.k &&
+         (reinterpret_cast<uintptr_t>(a.k) & 15) == 0;
 }
 
 template <typename IO, int D>

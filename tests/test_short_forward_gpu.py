@@ -55,3 +55,18 @@ def test_forward_turning_k_matches_rope_k(engines, hq, hkv, d, lengths):
         for a, b in zip(got, want):
             assert torch.equal(a, b)
         assert torch.equal(plain, want[0])
+
+
+@pytest.mark.parametrize("off", [2, 4])
+@pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (28, 4, 128)])
+def test_unaligned_k_stays_with_rope_k(engines, hq, hkv, d, off):
+    """K in a view off 16 bytes is not for the DMA: rope_k turns it, and the
+    results are those of an aligned K."""
+    print(f"[short forward] K off by {2 * off} bytes heads={hq}/{hkv} d={d}", flush=True)
+    T = 97
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    q, k, v = (torch.randn(T, h, d, device="cuda", generator=gen).bfloat16() for h in (hq, hkv, hkv))
+    moved = torch.empty(k.numel() + off, device="cuda", dtype=k.dtype)[off:].view(k.shape).copy_(k)
+    assert moved.data_ptr() % 16 == 2 * off
+    for a, b in zip(engines["auto"].forward(q, moved, v, 1.0e6), engines["auto"].forward(q, k, v, 1.0e6)):
+        assert torch.equal(a, b)
