@@ -652,11 +652,20 @@ __global__ __launch_bounds__(kFwdWaves * 64) void attn_fwd_kernel_ks(
 }  // namespace
 
 bool fwd_rotates_k(const FwdLaunch& a, int max_len) {
-  // two arrays, not one turned in place: other workgroups still read K; and K in
-  // whole 16-byte pieces, as the DMA moves it (rope_k's loads need no alignment)
+  // K in whole 16-byte pieces, as the DMA moves it (rope_k's loads need no
+  // alignment), and apart from what the launch writes: its workgroups read K
+  // while others store their rows (rope_k is done with it before)
+  const size_t rows = static_cast<size_t>(a.total_tokens);
+  const size_t q_bytes = rows * a.n_heads_q * a.head_dim * 2, k_bytes = rows * a.n_heads_kv * a.head_dim * 2;
+  const uintptr_t k = reinterpret_cast<uintptr_t>(a.k);
+  auto apart = [&](const void* p, size_t bytes) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(p);
+    return p == nullptr || at + bytes <= k || k + k_bytes <= at;
+  };
   return a.io_bf16 && (a.head_dim == 64 || a.head_dim == 128) && a.tile_rows != 64 &&
-         max_len <= kFwdWaves * kChunk && a.k_rot != a.k &&
-         (reinterpret_cast<uintptr_t>(a.k) & 15) == 0;
+         max_len <= kFwdWaves * kChunk && (k & 15) == 0 && apart(a.out, q_bytes) &&
+         apart(a.q_rot, q_bytes) && apart(a.k_rot, k_bytes) &&
+         apart(a.lse, rows * a.n_heads_q * sizeof(float));
 }
 
 template <typename IO, int D>

@@ -70,3 +70,17 @@ def test_unaligned_k_stays_with_rope_k(engines, hq, hkv, d, off):
     assert moved.data_ptr() % 16 == 2 * off
     for a, b in zip(engines["auto"].forward(q, moved, v, 1.0e6), engines["auto"].forward(q, k, v, 1.0e6)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("name", ["out", "q_rot", "k_rot"])
+@pytest.mark.parametrize("d", [64, 128])
+def test_output_in_the_place_of_k(engines, name, d):
+    """K is read before anything is written over it: the results of an output
+    in K's memory are those of one beside it."""
+    print(f"[short forward] {name} in K's place d={d}", flush=True)
+    T, h = 97, 3
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    q, k, v = (torch.randn(T, h, d, device="cuda", generator=gen).bfloat16() for _ in range(3))
+    want = engines["auto"].forward(q, k, v, 1.0e6)
+    for a, b in zip(engines["auto"].forward(q, k, v, 1.0e6, **{name: k}), want):
+        assert torch.equal(a, b)
