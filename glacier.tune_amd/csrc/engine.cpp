@@ -1080,6 +1080,7 @@ class GpuAttentionEngine {
     a.lowrank = get(lowrank_, need.lowrank, "low-rank scratch");
     a.terms = need.terms > 0 ? terms_.ensure(need.terms * 2, "low-rank split terms") : nullptr;
     a.odd = need.odd > 0 ? static_cast<int*>(odd_.ensure(need.odd * sizeof(int), "low-rank marks")) : nullptr;
+    a.shadow = need.shadow > 0 ? shadow_.ensure(need.shadow, "projection output") : nullptr;
   }
 
   int device_;
@@ -1105,7 +1106,7 @@ class GpuAttentionEngine {
   int fwd_rows_ = 0;      // bf16 forward rows per workgroup (GLACIER_ATTN_FWD_ROWS; 0: auto)
   int bwd_pairs_mode_ = -1;  // wide backward over head pairs: 1 on, 0 off, -1 auto (GLACIER_ATTN_BWD_PAIRS)
   // projection scratch and the hipBLASLt handle (created on first use)
-  DeviceBuffer lowrank_, terms_, odd_;
+  DeviceBuffer lowrank_, terms_, odd_, shadow_;
   DeviceBuffer rstd_, dyw_;  // RMSNorm backward row scales, dy copy (weight gradient)
   DeviceBuffer lm_idx_, lm_hv_, lm_logits_, lm_dl_, lm_dhv_, lm_loss_;  // LM head
   void* blas_ = nullptr;

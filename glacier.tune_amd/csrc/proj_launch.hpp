@@ -37,6 +37,7 @@ struct ProjLaunch {
   float* lowrank;  // [slot][T][r] X A_p and dY_p B_p^T
   void* terms;     // fused calls: the split terms (bf16) of the adapters, then of s L
   int* odd;        // fused calls: marks of values without a split (SplitCall)
+  void* shadow;    // outputs in the memory of x, dY or a W: written here, then copied
 };
 
 // ---- bf16 tensors: base products, low-rank delta, bias and conversion in ----
@@ -77,6 +78,7 @@ struct ProjScratchNeed {
   long lowrank;  // floats
   long terms;    // bf16
   long odd;      // ints
+  long shadow;   // bytes
 };
 ProjScratchNeed proj_scratch_need(const ProjLaunch& a, bool backward);
 

@@ -565,6 +565,29 @@ hipError_t launch_lowrank(const ProjLaunch& a, SplitCall& c, hipStream_t st) {
   return hipGetLastError();
 }
 
+// Whether output p of the call (forward: y_p; backward: dX, p 0) shares memory
+// with what its GEMM launch reads while it writes: x or every dY, and the W.
+bool in_place(const ProjLaunch& a, bool backward, int p) {
+  const size_t esz = a.io_bf16 ? 2 : 4;
+  const uintptr_t out = reinterpret_cast<uintptr_t>(backward ? a.dx : a.p[p].y);
+  const size_t out_bytes = (size_t)a.T * (backward ? a.in : a.p[p].out) * esz;
+  auto shares = [&](const void* q, size_t n) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(q);
+    return at < out + out_bytes && out < at + n * esz;
+  };
+  bool any = !backward && shares(a.x, (size_t)a.T * a.in);
+  for (int i = 0; i < a.n_proj; ++i)
+    any = any || shares(a.p[i].w, (size_t)a.p[i].out * a.in) ||
+          (backward && shares(a.p[i].dy, (size_t)a.T * a.p[i].out));
+  return any;
+}
+// Bytes of output p in ProjLaunch::shadow: none unless in_place.
+size_t shadow_bytes(const ProjLaunch& a, bool backward, int p) {
+  if (!in_place(a, backward, p)) return 0;
+  const size_t n = (size_t)a.T * (backward ? a.in : a.p[p].out) * (a.io_bf16 ? 2 : 4);
+  return (n + 15) / 16 * 16;
+}
+
 // A call: the low-rank products (and split terms), then (backward) the
 // adapters' gradients, then one GEMM launch for everything else.
 hipError_t run_call(const ProjLaunch& a, bool backward, hipStream_t st) {
@@ -572,7 +595,16 @@ hipError_t run_call(const ProjLaunch& a, bool backward, hipStream_t st) {
   const RowsPlan plan = rows_plan(a, backward);
   const int P = term_pitch(a.rank);
   GemmCall g{};
-  g.dx = a.dx;
+  // the outputs, or where the launch writes them instead
+  const int n_out = backward ? 1 : a.n_proj;
+  void* to[kMaxProj];
+  size_t shadowed[kMaxProj], at = 0;
+  for (int p = 0; p < n_out; ++p) {
+    shadowed[p] = shadow_bytes(a, backward, p);
+    to[p] = shadowed[p] > 0 ? static_cast<char*>(a.shadow) + at : backward ? a.dx : a.p[p].y;
+    at += shadowed[p];
+  }
+  g.dx = backward ? to[0] : nullptr;
   g.T = a.T;
   g.K = a.in;
   g.rank = a.rank;
@@ -586,7 +618,7 @@ hipError_t run_call(const ProjLaunch& a, bool backward, hipStream_t st) {
   c.odd = a.odd;
   for (int p = 0; p < a.n_proj; ++p) {
     const ProjSpec& s = a.p[p];
-    g.j[p] = GemmJob{s.y, s.bias, nullptr, nullptr, s.scaling, s.out, 0};
+    g.j[p] = GemmJob{backward ? nullptr : to[p], s.bias, nullptr, nullptr, s.scaling, s.out, 0};
     g.seg[p] = GemmSeg{s.w, backward ? s.dy : a.x, backward ? s.out : a.in};
     const int slot_l = backward ? plan.slot_dl[p] : plan.slot_l[p];
     if (slot_l < 0) continue;
@@ -619,13 +651,20 @@ hipError_t run_call(const ProjLaunch& a, bool backward, hipStream_t st) {
     g.n_odd = kTermBlocks + c.n * c.slabs;
   }
   if (backward) GL_CHECK(run_cols_any(a, plan, st));
-  return whole ? launch_gemm(g, backward, st) : launch_gemm_split(g, backward, a.io_bf16, st);
+  GL_CHECK(whole ? launch_gemm(g, backward, st) : launch_gemm_split(g, backward, a.io_bf16, st));
+  for (int p = 0; p < n_out; ++p)
+    if (shadowed[p] > 0)
+      GL_CHECK(hipMemcpyAsync(backward ? a.dx : a.p[p].y, to[p],
+                              (size_t)a.T * (backward ? a.in : a.p[p].out) * (a.io_bf16 ? 2 : 4),
+                              hipMemcpyDeviceToDevice, st));
+  return hipSuccess;
 }
 
 }  // namespace
 
 ProjScratchNeed proj_scratch_need(const ProjLaunch& a, bool backward) {
   ProjScratchNeed need{};
+  for (int p = 0; p < (backward ? 1 : a.n_proj); ++p) need.shadow += shadow_bytes(a, backward, p);
   const RowsPlan plan = rows_plan(a, backward);
   if (plan.n == 0) return need;
   need.lowrank = (long)plan.n * a.T * a.rank;

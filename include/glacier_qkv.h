@@ -68,7 +68,8 @@ int glacier_proj_forward(glacier_attn_ctx *ctx, const glacier_proj_desc *desc,
 /* Backward of the same projections: dx [T][in] is overwritten with the sum
  * over p of the base and adapter gradients (what the reference's three
  * LoraAdapter.Backward calls accumulate into a zeroed dXInput); grad_a and
- * grad_b are accumulated, like the reference's Grad tensors. */
+ * grad_b are accumulated, like the reference's Grad tensors.  dx may share
+ * memory with x or a dy (it is then written beside them and copied). */
 int glacier_proj_backward(glacier_attn_ctx *ctx, const glacier_proj_desc *desc,
                           const void *x, const glacier_lora_proj *proj, int n_proj,
                           void *dx);

@@ -221,3 +221,21 @@ def test_small_values_keep_their_bits(engines, dtype, where, T, n_in, outs, rank
         err = float(((got.double() - want) * scale).norm() / (want * scale).norm())
         print(f"  {err:.2e} of {within:.2e}", flush=True)
         assert err <= within
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [1024, 1028])  # both GEMMs in bf16
+def test_outputs_in_the_place_of_inputs(engines, dtype, n):
+    """dx in a dY's memory, and y in x's (out == in), are what they are beside
+    them: every workgroup reads its operands before anything replaces them."""
+    print(f"[in place] {dtype} n={n}", flush=True)
+    T, rank = 300, 8
+    x, projs = _problem(T, n, (n, 8, n), rank, dtype=dtype)
+    eng = engines[dtype]
+    dx = eng.proj_backward(x, projs, rank).clone()
+    ys = [y.clone() for y in eng.proj_forward(x, projs, rank)]
+    place = projs[2]["dy"]
+    assert torch.equal(eng.proj_backward(x, projs, rank, dx=place), dx)
+    x_in, projs[0]["y"] = x, x
+    for got, want in zip(eng.proj_forward(x_in, projs, rank), ys):
+        assert torch.equal(got, want)
