@@ -659,7 +659,7 @@ class GpuAttentionEngine:
         if not (x.is_cuda and x.is_contiguous() and x.dim() == 2):
             raise TypeError("x must be a contiguous [rows, n] GPU tensor")
         rows, n = x.shape
-        return NormDesc(rows, n, self._io_of(x), eps)
+        return NormDesc(rows, n, self._io_of(x), float(eps))
 
     @staticmethod
     def _like(t, ref, name):

@@ -325,3 +325,21 @@ def test_python_front_end_checks_device_tensors_before_the_abi():
     raises(lambda: ga.check_norm_args(x, torch.zeros(31)), "weight must have shape")
     raises(lambda: ga.check_norm_args(x, torch.zeros(32), torch.zeros(32, dtype=torch.bfloat16)),
            "d_weight must be torch.float32")
+
+
+def test_rmsnorm_eps_is_converted_like_a_float():
+    """eps as a configuration file gives it (YAML reads 1e-6 as text)."""
+    torch = pytest.importorskip("torch")
+
+    class Rows:  # a device tensor's face
+        is_cuda, shape, dtype = True, (3, 8), torch.float32
+
+        def is_contiguous(self):
+            return True
+
+        def dim(self):
+            return 2
+
+    for eps in ("1e-6", 1e-6, np.float32(1e-6)):
+        desc = ga.GpuAttentionEngine._norm_desc(ga.GpuAttentionEngine, Rows(), eps)
+        assert (desc.rows, desc.n, desc.eps) == (3, 8, np.float32(1e-6))
