@@ -271,11 +271,12 @@ struct PadJob {
   const void* src;
   void* dst;
   long rows;
+  int first;  // its first workgroup (set by the launch)
 };
 struct PadCall {  // the tensors of one direction
   PadJob j[5];
   int n;
-  void add(const void* src, void* dst, long rows) { j[n++] = PadJob{src, dst, rows}; }
+  void add(const void* src, void* dst, long rows) { j[n++] = PadJob{src, dst, rows, 0}; }
 };
 hipError_t launch_pad_rows(bool io_bf16, const PadCall& a, int d, int dp, hipStream_t st);
 hipError_t launch_unpad_rows(bool io_bf16, const PadCall& a, int d, int dp, hipStream_t st);

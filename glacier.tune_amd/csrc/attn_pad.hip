@@ -37,50 +37,81 @@ __device__ inline int pad_target(int s, int d, int dp) {
   return h;  // an odd d's last element
 }
 
-// Every tensor of one direction of a call in one launch (blockIdx.y: the
-// tensor), V consecutive elements of a row per thread: whole 16-byte pieces
-// where half a row is a whole number of them and the arrays are aligned (then a
-// piece lies in one half, and is copied or zeroed as one), else one element.
-// A workgroup takes 256 / (pieces per row) rows, so no index is divided by
-// more than a row's pieces.  Bound by the launch: a step at head size 80, 16
-// heads, 600 tokens made 14 launches of 3.9 us, one per tensor and element by
-// element; these are 4 of about 4.
-template <typename T, int V, bool PAD>
-__global__ __launch_bounds__(256) void pad_rows_kernel(const PadCall a, int d, int dp) {
-  const PadJob& job = a.j[blockIdx.y];
-  const int width = PAD ? dp : d, pieces = width / V, per_block = 256 / pieces;
-  const int sub = (int)threadIdx.x / pieces, j = V * ((int)threadIdx.x - sub * pieces);
-  const long r = (long)blockIdx.x * per_block + sub;
-  if (sub >= per_block || r >= job.rows) return;
-  const T* src = static_cast<const T*>(job.src) + r * (PAD ? d : dp);
-  T* dst = static_cast<T*>(job.dst) + r * width + j;
-  const int from = PAD ? pad_source(j, d, dp) : pad_target(j, d, dp);
-  if constexpr (V == 1) {
-    *dst = from >= 0 ? src[from] : static_cast<T>(0.0f);
-  } else {
-    i32x4 x{0, 0, 0, 0};
-    if (from >= 0) x = *reinterpret_cast<const i32x4*>(src + from);
-    *reinterpret_cast<i32x4*>(dst) = x;
+// Every tensor of one direction of a call in one launch, in pieces of V
+// consecutive elements: the most, up to 16 bytes, that half a row is a whole
+// number of and the arrays are aligned to (a piece then lies in one half of its
+// row, and is copied or zeroed as one).  A workgroup takes per_block whole rows, up
+// to 256 N pieces, N of each thread in flight at once.
+template <typename T, int V, int N, bool PAD>
+__global__ __launch_bounds__(256) void pad_rows_kernel(const PadCall a, int d, int dp, int per_block,
+                                                      unsigned inv) {
+  typedef T Piece __attribute__((ext_vector_type(V)));
+  int z = 0;
+  while (z + 1 < a.n && (int)blockIdx.x >= a.j[z + 1].first) ++z;
+  const PadJob& job = a.j[z];
+  const int width = PAD ? dp : d, pieces = width / V;
+  const long r0 = (long)((int)blockIdx.x - job.first) * per_block;
+  const int rows = static_cast<int>(min((long)per_block, job.rows - r0));
+  const T* src = static_cast<const T*>(job.src) + r0 * (PAD ? d : dp);
+  T* dst = static_cast<T*>(job.dst) + r0 * width;
+  Piece x[N];
+  int to[N];
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    const int i = (int)threadIdx.x + 256 * n;
+    // i / pieces: inv is 2^20 / pieces rounded up, i below 2^10, pieces at most 2^8
+    const int r = static_cast<int>(((unsigned)i * inv) >> 20), j = V * (i - r * pieces);
+    const int from = PAD ? pad_source(j, d, dp) : pad_target(j, d, dp);
+    to[n] = r < rows ? r * width + j : -1;
+    x[n] = *reinterpret_cast<const Piece*>(src + min(r, rows - 1) * (PAD ? d : dp) + max(from, 0));
+    if (from < 0) x[n] = Piece(static_cast<T>(0.0f));
   }
+#pragma unroll
+  for (int n = 0; n < N; ++n)
+    if (to[n] >= 0) *reinterpret_cast<Piece*>(dst + to[n]) = x[n];
 }
 
 template <typename T, bool PAD>
-hipError_t launch_pad(const PadCall& a, int d, int dp, hipStream_t st) {
-  constexpr int W = 16 / sizeof(T);
-  bool wide = (d / 2) % W == 0 && d % 2 == 0;
-  long rows = 0;
-  for (int i = 0; i < a.n; ++i) {
-    rows = rows > a.j[i].rows ? rows : a.j[i].rows;
-    wide = wide && (reinterpret_cast<uintptr_t>(a.j[i].src) & 15) == 0 &&
-           (reinterpret_cast<uintptr_t>(a.j[i].dst) & 15) == 0;
-  }
-  if (rows == 0) return hipSuccess;
-  const int per_block = 256 / ((PAD ? dp : d) / (wide ? W : 1));
-  const dim3 grid(static_cast<unsigned>((rows + per_block - 1) / per_block), a.n);
-  if (wide)
-    hipLaunchKernelGGL((pad_rows_kernel<T, W, PAD>), grid, dim3(256), 0, st, a, d, dp);
-  else
-    hipLaunchKernelGGL((pad_rows_kernel<T, 1, PAD>), grid, dim3(256), 0, st, a, d, dp);
+hipError_t launch_pad(PadCall a, int d, int dp, hipStream_t st) {
+  int v = 16 / sizeof(T);
+  auto whole = [&](int n) {
+    if (d % 2 != 0 || (d / 2) % n != 0) return n == 1;
+    for (int i = 0; i < a.n; ++i)
+      if (reinterpret_cast<uintptr_t>(a.j[i].src) % (n * sizeof(T)) != 0 ||
+          reinterpret_cast<uintptr_t>(a.j[i].dst) % (n * sizeof(T)) != 0)
+        return n == 1;
+    return true;
+  };
+  while (!whole(v)) v /= 2;
+  const int pieces = (PAD ? dp : d) / v;
+  const unsigned inv = ((1u << 20) + pieces - 1) / pieces;
+  int per_block = 0;
+  long blocks = 0;
+  auto split = [&](int n) {
+    per_block = 256 * n / pieces;
+    blocks = 0;
+    for (int i = 0; i < a.n; ++i) {
+      a.j[i].first = static_cast<int>(blocks);
+      blocks += (a.j[i].rows + per_block - 1) / per_block;
+    }
+  };
+  // Bound by the launch on short calls, by the pieces on long ones.  Forward that
+  // saves, then backward, bf16: 1500 tokens, 40/8 heads of 200: 168 + 534 us, where
+  // one element a thread took 265 + 694 and a launch per tensor 223 + 647.  Four
+  // pieces a thread once they give every CU two workgroups, one before (64
+  // tokens, 14/2 heads of 80: 14.5 + 16.8 us, 15.4 + 17.6 with four).
+  split(4);
+  const bool four = blocks >= 512;
+  if (!four) split(1);
+  if (blocks == 0) return hipSuccess;
+  auto pick = [&](auto nc) {
+    constexpr int N = decltype(nc)::value;
+    if constexpr (sizeof(T) == 2)
+      if (v == 8) return pad_rows_kernel<T, 8, N, PAD>;
+    return v == 4 ? pad_rows_kernel<T, 4, N, PAD> : v == 2 ? pad_rows_kernel<T, 2, N, PAD> : pad_rows_kernel<T, 1, N, PAD>;
+  };
+  auto fn = four ? pick(std::integral_constant<int, 4>{}) : pick(std::integral_constant<int, 1>{});
+  hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, st, a, d, dp, per_block, inv);
   return hipGetLastError();
 }
 

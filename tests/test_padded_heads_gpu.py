@@ -1,6 +1,6 @@
-"""Head sizes that run on padded rows (attn_pad.hip): rows copied in 16-byte
-pieces (half a row is a whole number of them and every array is 16-byte
-aligned) against the same rows copied element by element (one array starts one
+"""Head sizes that run on padded rows (attn_pad.hip): rows copied in pieces of
+up to 16 bytes (half a row is a whole number of them and every array is aligned
+to them) against the same rows copied element by element (one array starts one
 element off).  Both make the same padded rows, so every output is the same to
 the last bit; the oracle covers the element-wise copy at the other sizes.
 """
@@ -51,3 +51,11 @@ def test_pieces_match_elements(engine, lengths, hq, hkv, d, dtype):
                           dk=one_off(k))
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+# halves of whole 8- and 4-byte pieces only, and the longest rows of each; more
+# rows than one workgroup's, with a remainder
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("d", [4, 20, 100, 200, 248, 252])
+def test_narrower_pieces_match_elements(engine, d, dtype):
+    test_pieces_match_elements(engine, (130, 71), 6, 2, d, dtype)
