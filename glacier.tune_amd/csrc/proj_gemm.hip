@@ -651,7 +651,16 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
 
   const int fw = f0 + 32 * FB * wf, tw = t0 + 32 * TB * wt;
   const float* bias = NN || wk != 0 ? nullptr : a.j[z].bias;
-  f32x16 acc[FB][TB];
+  // fp32 tensors: the five small products of a step sum apart from the large
+  // one, whose sum then rounds once a step; bf16 results round far above that
+  constexpr bool kApart = sizeof(IO) == 4;
+  f32x16 acc[FB][TB], small[FB][TB];
+#pragma unroll
+  for (int fb = 0; fb < FB; ++fb)
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) small[fb][tb][e] = 0.0f;
   auto clear = [&] {
 #pragma unroll
     for (int fb = 0; fb < FB; ++fb)
@@ -686,9 +695,7 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
     }
   }
   bf16x8 fa[KS][FB][3], fbk[KS][TB][3];
-  auto fragments = [&](const unsigned char* base) {
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
+  auto fragments = [&](const unsigned char* base, int s) {
 #pragma unroll
       for (int p = 0; p < 3; ++p) {
 #pragma unroll
@@ -708,18 +715,18 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
           fbk[s][tb][p] = *reinterpret_cast<const bf16x8*>(base + ob[s] + kPlaneB * p + 2048 * tb);
       }
   };
-  auto products = [&] {
+  auto products = [&](int s) {
     // the small products first
     constexpr int kPa[6] = {2, 0, 1, 1, 0, 0}, kPb[6] = {0, 2, 1, 0, 1, 0};
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
 #pragma unroll
       for (int q = 0; q < 6; ++q)
 #pragma unroll
         for (int fb = 0; fb < FB; ++fb)
 #pragma unroll
-          for (int tb = 0; tb < TB; ++tb)
-            acc[fb][tb] = mma32(fa[s][fb][kPa[q]], fbk[s][tb][kPb[q]], acc[fb][tb]);
+          for (int tb = 0; tb < TB; ++tb) {
+            f32x16& sum = kApart && q < 5 ? small[fb][tb] : acc[fb][tb];
+            sum = mma32(fa[s][fb][kPa[q]], fbk[s][tb][kPb[q]], sum);
+          }
   };
   // Stage n in buffer n % 2: its fragments are read, the next stage's pieces
   // split and written to the other buffer (every wave is past its reads of it)
@@ -727,10 +734,15 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
   // the next stage's rows visible.
   int n = 0;
   auto turn = [&](auto&& next) {
-    fragments(lds + (n & 1) * kBuf);
+    const unsigned char* base = lds + (n & 1) * kBuf;
+    fragments(base, 0);
     ++n;
     next(lds + (n & 1) * kBuf);
-    products();
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      if (s > 0) fragments(base, s);
+      products(s);
+    }
     lgkm<0>();
     wg_barrier();
   };
@@ -758,6 +770,7 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
     load(PF, ring[0]);
   }
   settle(acc);
+  if constexpr (kApart) settle(small);
   for (int st0 = 0; st0 < nst; st0 += PF) {
     static_for<PF>([&](auto jc) {
       // stages past the end hold zeros (no valid element), and add nothing
@@ -768,6 +781,13 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
       });
     });
     settle(acc);
+    if constexpr (kApart) settle(small);
+  }
+  if constexpr (kApart) {
+#pragma unroll
+    for (int fb = 0; fb < FB; ++fb)
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb) acc[fb][tb] += small[fb][tb];
   }
   if (__syncthreads_or(mark.bad())) {
     // the same sums on fp32 MFMAs: lane l supplies A[row l % 32][k + l / 32]

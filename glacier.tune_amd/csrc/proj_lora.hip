@@ -154,18 +154,22 @@ constexpr int kTermBlocks = 64;
 constexpr int split_waves(int nt, int rb) { return rb == 1 && nt % 2 == 1 ? 16 : 8; }
 
 #if defined(__HIP_DEVICE_COMPILE__)
-// The k range [kb, ke) of one wave of lowrank_split_kernel, added into acc.
+// The k range [kb, ke) of one wave of lowrank_split_kernel, added into acc and,
+// the products of lower terms, into small (so that acc rounds once a step).
 // Steps of 32: lane (i, q) holds U[row i][k0 + 8q .. +7] and V[k0 + 8q ..
 // +7][16 jt + i].  Lengths are multiples of 4 (of 8 with WIDE), so each half
 // of a lane's 8 is all in or all out; out of range V is zeroed, U clamped
 // (and, where a step goes the fp32 way, zeroed as well).
 template <typename IO, bool WIDE, int NT, int RB, bool VT>
 __device__ inline void split_accumulate(const IO* const (&u)[RB], const float* __restrict__ v0, int K,
-                                        int rank, int kb, int ke, f32x4 (&acc)[RB][NT]) {
+                                        int rank, int kb, int ke, f32x4 (&acc)[RB][NT],
+                                        f32x4 (&small)[RB][NT]) {
   const int lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
   constexpr bool kF32 = sizeof(IO) == 4;
   constexpr int W = NT * RB * (kF32 ? 2 : 1);
-  constexpr int CH = W <= 2 ? 4 : W <= 8 ? 2 : 1;  // steps whose loads are issued together
+  // steps whose loads are issued together (fp32 at one tile: four would spill
+  // beside the 16 waves)
+  constexpr int CH = W <= 2 && !kF32 ? 4 : W <= 8 ? 2 : 1;
   for (int k0 = kb; k0 < ke; k0 += 32 * CH) {
     typename Raw4<IO>::T ur[CH][RB][2];
     float vr[CH][NT][8];
@@ -232,15 +236,15 @@ __device__ inline void split_accumulate(const IO* const (&u)[RB], const float* _
 #pragma unroll
           for (int b = 0; b < RB; ++b) {
             if constexpr (kF32) {
-              acc[b][jt] = Mfma<bf16>::mma(us[b].l, v.h, acc[b][jt]);
-              acc[b][jt] = Mfma<bf16>::mma(us[b].h, v.l, acc[b][jt]);
-              acc[b][jt] = Mfma<bf16>::mma(us[b].m, v.m, acc[b][jt]);
-              acc[b][jt] = Mfma<bf16>::mma(us[b].m, v.h, acc[b][jt]);
-              acc[b][jt] = Mfma<bf16>::mma(us[b].h, v.m, acc[b][jt]);
+              small[b][jt] = Mfma<bf16>::mma(us[b].l, v.h, small[b][jt]);
+              small[b][jt] = Mfma<bf16>::mma(us[b].h, v.l, small[b][jt]);
+              small[b][jt] = Mfma<bf16>::mma(us[b].m, v.m, small[b][jt]);
+              small[b][jt] = Mfma<bf16>::mma(us[b].m, v.h, small[b][jt]);
+              small[b][jt] = Mfma<bf16>::mma(us[b].h, v.m, small[b][jt]);
               acc[b][jt] = Mfma<bf16>::mma(us[b].h, v.h, acc[b][jt]);
             } else {
-              acc[b][jt] = Mfma<bf16>::mma(ub[b], v.l, acc[b][jt]);
-              acc[b][jt] = Mfma<bf16>::mma(ub[b], v.m, acc[b][jt]);
+              small[b][jt] = Mfma<bf16>::mma(ub[b], v.l, small[b][jt]);
+              small[b][jt] = Mfma<bf16>::mma(ub[b], v.m, small[b][jt]);
               acc[b][jt] = Mfma<bf16>::mma(ub[b], v.h, acc[b][jt]);
             }
           }
@@ -318,15 +322,15 @@ __global__ __launch_bounds__(64 * split_waves(NT, RB)) void lowrank_split_kernel
     u[b] = static_cast<const IO*>(job.u) + (long)min(t0 + 16 * b + i, T - 1) * K;
   int kb, ke;
   share(K, W, wave, 32, kb, ke);
-  f32x4 acc[RB][NT];
+  f32x4 acc[RB][NT], small[RB][NT];
 #pragma unroll
   for (int b = 0; b < RB; ++b)
 #pragma unroll
-    for (int jt = 0; jt < NT; ++jt) acc[b][jt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int jt = 0; jt < NT; ++jt) acc[b][jt] = small[b][jt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   if (job.vt)
-    split_accumulate<IO, WIDE, NT, RB, true>(u, job.v, K, rank, kb, ke, acc);
+    split_accumulate<IO, WIDE, NT, RB, true>(u, job.v, K, rank, kb, ke, acc, small);
   else
-    split_accumulate<IO, WIDE, NT, RB, false>(u, job.v, K, rank, kb, ke, acc);
+    split_accumulate<IO, WIDE, NT, RB, false>(u, job.v, K, rank, kb, ke, acc, small);
   // D of (b, jt): lane (i, q), register c holds row 16 b + 4q + c, column 16 jt + i
 #pragma unroll
   for (int b = 0; b < RB; ++b)
@@ -334,7 +338,7 @@ __global__ __launch_bounds__(64 * split_waves(NT, RB)) void lowrank_split_kernel
     for (int jt = 0; jt < NT; ++jt)
 #pragma unroll
       for (int c = 0; c < 4; ++c)
-        red[(wave * 16 * RB + 16 * b + 4 * q + c) * kRow + 16 * jt + i] = acc[b][jt][c];
+        red[(wave * 16 * RB + 16 * b + 4 * q + c) * kRow + 16 * jt + i] = acc[b][jt][c] + small[b][jt][c];
   __syncthreads();
   for (int idx = threadIdx.x; idx < 16 * RB * 16 * NT; idx += 64 * W) {
     const int r = idx / (16 * NT), j = idx % (16 * NT), t = t0 + r;

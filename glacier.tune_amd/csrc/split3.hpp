@@ -8,9 +8,11 @@
 // keep subnormals); the three smallest (a.m b.l, a.l b.m, a.l b.l) are left
 // out: at most (2^-24 + 2^-34) |a b| together, an fp32 rounding.  A
 // bf16 MFMA does 16 times the products of an fp32 MFMA per cycle: six of them
-// take 6/16 of its time.  Measured against 64-bit products over the projections'
-// ranges (K 896-4096), fp32 results: 3.3e-7 to 7.5e-7 relative, where fp32
-// MFMAs left 5.3e-7 to 1.1e-6 (fewer roundings: 16 products to a sum step).
+// take 6/16 of its time.  The five small products have a sum of their own, so
+// that the large one's rounds once for 16 products.  Against 64-bit products over
+// the projections' ranges (K 896-4096, T 60-540), fp32 results are 1.5e-7 to
+// 3.9e-7 off in the 2-norm, where fp32 MFMAs left 3.3e-7 to 9.5e-7 (and all six in
+// one sum 3.6e-7 to 9.7e-7).
 // An x that is not that sum (not finite, rounding to infinity, or with bits
 // below 2^-133) has no split: SplitMarks tell, and the caller takes fp32
 // products for those operands.

@@ -239,3 +239,33 @@ def test_outputs_in_the_place_of_inputs(engines, dtype, n):
     x_in, projs[0]["y"] = x, x
     for got, want in zip(eng.proj_forward(x_in, projs, rank), ys):
         assert torch.equal(got, want)
+
+
+# how far fp32 MFMAs and a reduction split over workgroups were from float64 at
+# these sizes (2-norm), and a tenth for the draw
+@pytest.mark.parametrize("dtype,T,n_in,outs,rank,y_gate,dx_gate,grad_gate", [
+    (torch.float32, 152, 3584, (3584, 512, 512), 32, 8.0e-7, 9.1e-7, 2.1e-7),
+    (torch.float32, 538, 896, (896, 128, 128), 64, 3.7e-7, 4.7e-7, 2.3e-7),
+    (torch.bfloat16, 19, 4096, (4096, 1024, 1024), 64, None, None, 1.7e-7)])
+def test_split_sums_are_as_exact_as_fp32_ones(engines, dtype, T, n_in, outs, rank, y_gate, dx_gate,
+                                              grad_gate):
+    """Splitting an fp32 operand adds sums, and each rounds: the small products
+    have a sum of their own, so that the result is no further from float64."""
+    print(f"[split sums] {dtype} T={T} in={n_in} outs={outs} rank={rank}", flush=True)
+    x, projs = _problem(T, n_in, outs, rank, dtype=dtype)
+    for p in projs:
+        p["bias"] *= 0.0
+    ys, dx = engines[dtype].proj_forward(x, projs, rank), engines[dtype].proj_backward(x, projs, rank)
+    want, want_dx = _reference(x, projs)
+    err = lambda got, ref: float((got.double() - ref).norm() / ref.norm())  # noqa: E731
+    if y_gate is not None:
+        assert err(ys[0], want[0][0]) <= y_gate
+        assert err(dx, want_dx[0]) <= dx_gate
+    xd = x.double()
+    for p in projs:
+        if "a" not in p:
+            continue
+        dl, low = p["dy"].double() @ p["b"].double().t(), xd @ p["a"].double()
+        for name, ref in (("grad_a", 2.0 * xd.t() @ dl), ("grad_b", 2.0 * low.t() @ p["dy"].double())):
+            print(f"  {name} {err(p[name], ref):.2e} of {grad_gate:.1e}", flush=True)
+            assert err(p[name], ref) <= grad_gate
