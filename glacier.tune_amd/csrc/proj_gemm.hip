@@ -435,27 +435,34 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_kernel(const GemmCall a) 
 
 // ---------------------------------------------------------------------------
 // Every other call (fp32 tensors, and bf16 tensors of other widths or
-// alignments): the same sums, with each operand element split in three bf16
-// terms (split3.hpp) on its way from global memory to LDS, and six
-// v_mfma_f32_32x32x16_bf16 per product of fragments.  The low-rank product is
-// again a stretch of the reduction, the adapters' ranks one after another, its
-// operands taken as they are (fp32, B and A read down their columns); it goes
-// first, while the base products' first stages are on their way.
+// alignments): the same sums, operands through registers.  Each fp32 element is
+// split in three bf16 terms (split3.hpp) on its way from global memory to LDS, and
+// a product of fragments is six v_mfma_f32_32x32x16_bf16; bf16 elements are one
+// term, and one product.  The low-rank product is again a stretch of the
+// reduction, the adapters' ranks one after another, its operands split as they
+// are (fp32, B and A read down their columns); it goes first, while the base
+// products' first stages are on their way.
 //
 // 8 waves: WF x WT waves of FB x TB blocks of 32 x 32, times WK groups that
 // share a stage's two k-steps.  Stages of 32 reduction elements go global ->
 // registers (PF stages ahead) -> three LDS planes of bf16 rows (layout as above:
-// 64-byte rows, backward A 64-feature sub-tiles), two buffers, one barrier a
-// stage.  Loads are unconditional at clamped addresses; elements past the
-// reduction are zeroed in A, rows past an edge reach no stored result.
-// A tile that meets an element without a split is done over on fp32 MFMAs, straight from global memory.
+// 64-byte rows, backward A 64-feature sub-tiles; one plane for one term), two
+// buffers, one barrier a stage.  Loads are unconditional at clamped addresses;
+// elements past the reduction are zeroed in A (in one term in both), rows past
+// an edge reach no stored result.  A tile that meets an element without a split
+// is done over on fp32 MFMAs, straight from global memory.
 //
-// What bounds it: at one small tile per CU the chain of a stage (split, LDS,
+// What bounds it: fp32 at one small tile per CU the chain of a stage (split, LDS,
 // six dependent products: 0.75 us); once the chip is full the six products
 // (6/16 of the fp32 MFMA's time) and the split's 11 vector instructions for each
 // 2 elements beside them.  201 x 896 -> 896/128/128: forward 24 us in one
 // launch (three of 35, and two low-rank passes, before), backward 31 us (46
-// and two).
+// and two).  bf16, the chain of a stage (0.25 us): 512 x 3584 -> 3584/512/12, whole
+// calls, 61 + 81 us (177 + 219 split in three terms, 198 + 72 with q on a DMA
+// GEMM of its own); a 3584 x 3584 W off 16 bytes, 63 + 82 (177 + 230; 58 + 71).
+// 16-byte loads take 5-10% less than two of 8 bytes; planes of 96 reduction
+// elements in place of the terms took as long (a third of the barriers, but
+// 40 more VGPRs: one 64 x 64 workgroup a CU).
 // ---------------------------------------------------------------------------
 // Ends a run of products where control flow joins: 16 wait states, so that the
 // copies of accumulators that the compiler may place there read what the last
@@ -484,8 +491,13 @@ struct Piece {
   float x[8];
   int valid;
 };
+struct Piece16 {  // of bf16 tensors
+  bf16x8 x;
+  int valid;
+  bool late;  // the 8 loaded begin 4 before the piece
+};
 
-template <typename IO, bool NN, int FB, int TB, int WF, int WT, int WK, int PF>
+template <typename IO, bool NN, bool kTiny, int FB, int TB, int WF, int WT, int WK, int PF>
 __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCall a) {
 #if defined(__HIP_DEVICE_COMPILE__)
   static_assert(WF * WT * WK == 8 && (WK == 1 || WK == 2), "8 waves");
@@ -495,6 +507,7 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
   constexpr int kPlaneA = FT * 64, kPlaneB = TT * 64, kBuf = 3 * (kPlaneA + kPlaneB);
   static_assert((PA % kGThreads == 0 && PB % kGThreads == 0) || (NA == 0 && NB == 0 && PA + PB == kGThreads),
                 "pieces per thread");
+  constexpr bool kOne = sizeof(IO) == 2;  // base operands: bf16 already, one term
   constexpr bool kShared = NA == 0;  // half of the threads bring A, half B
   constexpr int LA = kShared ? 1 : NA, LB = kShared ? 0 : NB;
   __shared__ __align__(1024) unsigned char lds[2 * kBuf];
@@ -532,27 +545,38 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
   // reduction row, 8 features) and B (row t, 8 reduction elements).
   int sg = seg0 - 1, kend = 0, kbase = 0, kcur = 0;
   const IO *ca = nullptr, *cb = nullptr;
-  auto load_a = [&](int idx, int k0, Piece& p) {
+  using Base = std::conditional_t<kOne, Piece16, Piece>;
+  // elements k .. k + 7 of a row of len (a multiple of 4), in bounds
+  auto eight = [&](const IO* row, int k, int len, Base& p) {
+    if constexpr (kOne && kTiny) {
+      p.late = false;
+      __builtin_memcpy(&p.x, row + min(k, len - 4), 8);
+      __builtin_memcpy(reinterpret_cast<char*>(&p.x) + 8, row + min(k + 4, len - 4), 8);
+    } else if constexpr (kOne) {
+      // one load, 4 early where the row ends inside it
+      const int at = min(k, len - 8);
+      p.late = k > at;
+      __builtin_memcpy(&p.x, row + at, 16);
+    } else {
+      load4_any(row + min(k, len - 4), p.x, 0);
+      load4_any(row + min(k + 4, len - 4), p.x, 4);
+    }
+  };
+  auto load_a = [&](int idx, int k0, Base& p) {
     if constexpr (NN) {
       const int k = k0 + (idx >> 3) % 32, f = f0 + 64 * (idx >> 8) + 8 * (idx & 7);
       p.valid = k < kcur ? 8 : 0;
-      const IO* row = ca + (long)min(k, kcur - 1) * K;
-      load4_any(row + min(f, K - 4), p.x, 0);
-      load4_any(row + min(f + 4, K - 4), p.x, 4);
+      eight(ca + (long)min(k, kcur - 1) * K, f, K, p);
     } else {
       const int f = min(f0 + (idx >> 2), nf - 1), k = k0 + 8 * (idx & 3);
       p.valid = kcur - k;
-      const IO* row = ca + (long)f * kcur;
-      load4_any(row + min(k, kcur - 4), p.x, 0);
-      load4_any(row + min(k + 4, kcur - 4), p.x, 4);
+      eight(ca + (long)f * kcur, k, kcur, p);
     }
   };
-  auto load_b = [&](int idx, int k0, Piece& p) {
+  auto load_b = [&](int idx, int k0, Base& p) {
     const int t = min(t0 + (idx >> 2), T - 1), k = k0 + 8 * (idx & 3);
-    p.valid = 8;
-    const IO* row = cb + (long)t * kcur;
-    load4_any(row + min(k, kcur - 4), p.x, 0);
-    load4_any(row + min(k + 4, kcur - 4), p.x, 4);
+    p.valid = kOne ? kcur - k : 8;  // one term: nothing marks a non-finite value that A's zeros meet
+    eight(cb + (long)t * kcur, k, kcur, p);
   };
   // the same of the low-rank stretch, its elements kk0 ..
   auto low_a = [&](int idx, int kk0, Piece& p) {
@@ -579,7 +603,10 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
   struct Pieces {
     Piece a[LA], b[LB > 0 ? LB : 1];
   };
-  auto load = [&](int st, Pieces& p) {
+  struct BasePieces {
+    Base a[LA], b[LB > 0 ? LB : 1];
+  };
+  auto load = [&](int st, BasePieces& p) {
     while (st >= kend && sg + 1 < seg1) {
       ++sg;
       kbase = kend;
@@ -615,15 +642,8 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
     }
   };
   SplitMarks mark;
-  // piece idx of operand `b` (0: A, 1: B) into the three planes of a buffer
-  auto put = [&](unsigned char* base, int idx, bool b, Piece& q) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      tie_v(q.x[e]);  // the load stays unconditional
-      q.x[e] = e < q.valid ? q.x[e] : 0.0f;
-    }
-    Split3 s;
-    s.set(q.x, mark);
+  // piece idx of operand `b` (0: A, 1: B) into the planes of a buffer
+  auto put = [&](unsigned char* base, int idx, bool b, auto& q) {
     int off;
     if (NN && !b) {
       const int r = (idx >> 3) % 32;
@@ -633,12 +653,25 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
       off = 64 * r + 16 * ((idx & 3) ^ lds_sw<32>(r));
     }
     unsigned char* p = base + (b ? 3 * kPlaneA : 0) + off;
-    const int plane = b ? kPlaneB : kPlaneA;
-    *reinterpret_cast<bf16x8*>(p) = s.h;
-    *reinterpret_cast<bf16x8*>(p + plane) = s.m;
-    *reinterpret_cast<bf16x8*>(p + 2 * plane) = s.l;
+    if constexpr (std::is_same_v<std::decay_t<decltype(q)>, Piece16>) {
+      tie_v(q.x);  // the load stays unconditional
+      const bf16x4 zero{}, lo{q.x[0], q.x[1], q.x[2], q.x[3]}, hi{q.x[4], q.x[5], q.x[6], q.x[7]};
+      *reinterpret_cast<bf16x8*>(p) = join8(q.valid <= 0 ? zero : q.late ? hi : lo, q.valid <= 4 ? zero : hi);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        tie_v(q.x[e]);
+        q.x[e] = e < q.valid ? q.x[e] : 0.0f;
+      }
+      Split3 s;
+      s.set(q.x, mark);
+      const int plane = b ? kPlaneB : kPlaneA;
+      *reinterpret_cast<bf16x8*>(p) = s.h;
+      *reinterpret_cast<bf16x8*>(p + plane) = s.m;
+      *reinterpret_cast<bf16x8*>(p + 2 * plane) = s.l;
+    }
   };
-  auto put_all = [&](unsigned char* base, Pieces& p) {
+  auto put_all = [&](unsigned char* base, auto& p) {
     if constexpr (kShared) {
       put(base, w < PA / 64 ? tid : tid - PA, w >= PA / 64, p.a[0]);
     } else {
@@ -695,58 +728,61 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
     }
   }
   bf16x8 fa[KS][FB][3], fbk[KS][TB][3];
-  auto fragments = [&](const unsigned char* base, int s) {
+  // k-step s of a stage in one term or three
+  auto fragments = [&](const unsigned char* base, int s, auto terms) {
 #pragma unroll
-      for (int p = 0; p < 3; ++p) {
+    for (int p = 0; p < decltype(terms)::value; ++p) {
 #pragma unroll
-        for (int fb = 0; fb < FB; ++fb) {
-          if constexpr (NN) {
-            auto tr = [&](int j) {
-              return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((bf16x4 GLACIER_LDS*)const_cast<unsigned char*>(
-                  base + oa[2 * fb + j] + kPlaneA * p + 2048 * s));
-            };
-            fa[s][fb][p] = join8(tr(0), tr(1));
-          } else {
-            fa[s][fb][p] = *reinterpret_cast<const bf16x8*>(base + oa[s] + kPlaneA * p + 2048 * fb);
-          }
+      for (int fb = 0; fb < FB; ++fb) {
+        if constexpr (NN) {
+          auto tr = [&](int j) {
+            return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((bf16x4 GLACIER_LDS*)const_cast<unsigned char*>(
+                base + oa[2 * fb + j] + kPlaneA * p + 2048 * s));
+          };
+          fa[s][fb][p] = join8(tr(0), tr(1));
+        } else {
+          fa[s][fb][p] = *reinterpret_cast<const bf16x8*>(base + oa[s] + kPlaneA * p + 2048 * fb);
         }
-#pragma unroll
-        for (int tb = 0; tb < TB; ++tb)
-          fbk[s][tb][p] = *reinterpret_cast<const bf16x8*>(base + ob[s] + kPlaneB * p + 2048 * tb);
       }
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb)
+        fbk[s][tb][p] = *reinterpret_cast<const bf16x8*>(base + ob[s] + kPlaneB * p + 2048 * tb);
+    }
   };
-  auto products = [&](int s) {
+  auto products = [&](int s, auto terms) {
     // the small products first
     constexpr int kPa[6] = {2, 0, 1, 1, 0, 0}, kPb[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
-      for (int q = 0; q < 6; ++q)
+    for (int q = decltype(terms)::value == 1 ? 5 : 0; q < 6; ++q)
 #pragma unroll
-        for (int fb = 0; fb < FB; ++fb)
+      for (int fb = 0; fb < FB; ++fb)
 #pragma unroll
-          for (int tb = 0; tb < TB; ++tb) {
-            f32x16& sum = kApart && q < 5 ? small[fb][tb] : acc[fb][tb];
-            sum = mma32(fa[s][fb][kPa[q]], fbk[s][tb][kPb[q]], sum);
-          }
+        for (int tb = 0; tb < TB; ++tb) {
+          f32x16& sum = kApart && q < 5 ? small[fb][tb] : acc[fb][tb];
+          sum = mma32(fa[s][fb][kPa[q]], fbk[s][tb][kPb[q]], sum);
+        }
   };
   // Stage n in buffer n % 2: its fragments are read, the next stage's pieces
   // split and written to the other buffer (every wave is past its reads of it)
   // behind those reads, then come the products, then the barrier that makes
   // the next stage's rows visible.
   int n = 0;
-  auto turn = [&](auto&& next) {
+  auto turn = [&](auto terms, auto&& next) {
     const unsigned char* base = lds + (n & 1) * kBuf;
-    fragments(base, 0);
+    fragments(base, 0, terms);
     ++n;
     next(lds + (n & 1) * kBuf);
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-      if (s > 0) fragments(base, s);
-      products(s);
+      if (s > 0) fragments(base, s, terms);
+      products(s, terms);
     }
     lgkm<0>();
     wg_barrier();
   };
-  Pieces ring[PF];
+  constexpr std::integral_constant<int, 3> kThree{};
+  constexpr std::integral_constant<int, kOne ? 1 : 3> kBase{};
+  BasePieces ring[PF];
   {
     Pieces low;
     if (low_st > 0) load_low(0, low);
@@ -757,11 +793,11 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
       lgkm<0>();
       wg_barrier();
       for (int st = 1; st < low_st; ++st)
-        turn([&](unsigned char* base) {
+        turn(kThree, [&](unsigned char* base) {
           put_all(base, low);
           if (st + 1 < low_st) load_low(st + 1, low);
         });
-      turn([&](unsigned char* base) { put_all(base, ring[0]); });
+      turn(kThree, [&](unsigned char* base) { put_all(base, ring[0]); });
     } else {
       put_all(lds, ring[0]);
       lgkm<0>();
@@ -775,7 +811,7 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
     static_for<PF>([&](auto jc) {
       // stages past the end hold zeros (no valid element), and add nothing
       constexpr int J = (decltype(jc)::value + 1) % PF;
-      turn([&](unsigned char* base) {
+      turn(kBase, [&](unsigned char* base) {
         put_all(base, ring[J]);
         load(st0 + decltype(jc)::value + 1 + PF, ring[J]);
       });
@@ -880,8 +916,6 @@ const GemmShape kShapes[] = {
 };
 #undef GL_GEMM
 
-constexpr int kBigSplitTiles = 128;
-
 int tiles_of(const GemmCall& a, bool nn, const GemmShape& s) {
   int ftiles = 0;
   if (nn)
@@ -929,8 +963,14 @@ namespace {
 
 template <typename IO, bool NN>
 hipError_t launch_split(GemmCall a, hipStream_t st) {
-  // 128 x 128 tiles once they fill most of the CUs (their waves do twice the
-  // products per LDS byte), else 64 x 64
+  // 128 x 128 tiles (one workgroup a CU) once they are more than the 64 x 64 ones
+  // that fit the chip at once: half of its CUs, as fp32 tensors have one of those
+  // on a CU of twice the time, bf16 tensors two.  Time at 128 x 128 over time at
+  // 64 x 64, forward and backward: fp32 32-64 tiles 1.50-1.76, 72-112 0.92-1.02,
+  // 128 0.95, 144-192 0.71, over that 0.72-0.87 (264: 1.06); bf16 up to 116 tiles
+  // 1.05-1.42, 128 1.08-1.14, 132-256 0.82-0.84 (1.07 at 132 with 1000 inputs),
+  // over that 0.69-1.05.
+  constexpr int kBigTiles = sizeof(IO) == 2 ? 129 : 128;
   auto tiles = [&](int ft) {
     a.ftiles = 0;
     for (int z = 0; z < (NN ? 1 : a.n); ++z) {
@@ -939,14 +979,19 @@ hipError_t launch_split(GemmCall a, hipStream_t st) {
     }
     return a.ftiles * ((a.T + ft - 1) / ft);
   };
+  // bf16 rows of 4 elements: no 8 to load at once
+  bool tiny = a.K < 8;
+  for (int z = 0; z < a.n; ++z) tiny = tiny || a.j[z].n < 8;
+  tiny = tiny && sizeof(IO) == 2;
   int n = tiles(128);
-  const bool big = n >= kBigSplitTiles;
+  const bool big = n >= kBigTiles && !tiny;
   if (!big) n = tiles(64);
   if (n == 0) return hipSuccess;
-  if (big)
-    hipLaunchKernelGGL((proj_gemm_split_kernel<IO, NN, 2, 1, 2, 4, 1, 2>), dim3(n), dim3(kGThreads), 0, st, a);
-  else
-    hipLaunchKernelGGL((proj_gemm_split_kernel<IO, NN, 1, 1, 2, 2, 2, 4>), dim3(n), dim3(kGThreads), 0, st, a);
+  auto fn = big ? proj_gemm_split_kernel<IO, NN, false, 2, 1, 2, 4, 1, 2>
+                : proj_gemm_split_kernel<IO, NN, false, 1, 1, 2, 2, 2, 4>;
+  if constexpr (sizeof(IO) == 2)
+    if (tiny) fn = proj_gemm_split_kernel<IO, NN, true, 1, 1, 2, 2, 2, 4>;
+  hipLaunchKernelGGL(fn, dim3(n), dim3(kGThreads), 0, st, a);
   return hipGetLastError();
 }
 

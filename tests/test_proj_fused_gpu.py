@@ -269,3 +269,32 @@ def test_split_sums_are_as_exact_as_fp32_ones(engines, dtype, T, n_in, outs, ran
         for name, ref in (("grad_a", 2.0 * xd.t() @ dl), ("grad_b", 2.0 * low.t() @ p["dy"].double())):
             print(f"  {name} {err(p[name], ref):.2e} of {grad_gate:.1e}", flush=True)
             assert err(p[name], ref) <= grad_gate
+
+
+# one term for bf16 operands of the general GEMM: rows of 4, rows that end 4
+# before a 16-byte piece, one row, the larger tiles in both directions
+@pytest.mark.parametrize("T,n_in,outs,rank", [
+    (1, 4, (4,), 1), (70, 12, (4, 36), 3), (33, 4, (12,), 2), (1, 12, (12, 8), 2),
+    (65, 268, (132, 8), 16), (1025, 2052, (2052,), 16)])
+def test_odd_bf16_widths_match_float64(engine, T, n_in, outs, rank):
+    print(f"[odd widths] T={T} in={n_in} outs={outs} rank={rank}", flush=True)
+    _run_and_check(engine, *_problem(T, n_in, outs, rank), rank)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_non_finite_row_ends_stay_in_their_rows(engine, value):
+    """Loads past a row's end repeat its last elements: where those are not
+    finite, the zeros of the other operand have to meet zeros."""
+    T, n_in, outs, rank = 70, 100, (36, 72), 3
+    x, projs = _problem(T, n_in, outs, rank)
+    x[5, n_in - 1] = value
+    projs[0]["dy"][6, outs[0] - 1] = value
+    projs[1]["w"][7, n_in - 2] = value
+    ys, dx = engine.proj_forward(x, projs, rank), engine.proj_backward(x, projs, rank)
+    want, want_dx = _reference(x, projs)
+    for got, (ref, terms) in zip([*ys, dx], [*want, want_dx]):
+        ref = ref.float().to(got.dtype)
+        assert torch.equal(torch.isnan(got), torch.isnan(ref))
+        assert torch.equal(torch.isinf(got), torch.isinf(ref))
+        ok = torch.isfinite(ref)
+        _check(got[ok], ref[ok], terms[ok], n_in, "finite")
