@@ -127,7 +127,8 @@ struct SplitCall {
   TermJob v[kMaxProj];
   int n, nv, across;
   int slabs;   // row slabs of a job
-  int* odd;    // [kTermBlocks], then [n][slabs]: a value without split terms among what that workgroup wrote
+  int groups;  // rank groups of a slab
+  int* odd;    // [kTermBlocks], then [groups][n][slabs]: a value without split terms among what that workgroup wrote
 };
 
 // The six entries of a terms row for x: side 0 the adapters', side 1 (s L).
@@ -149,20 +150,24 @@ __device__ inline bool put_terms(float x, int side, Put&& put) {
   return (left & 0xffffu) != 0 || (left & 0x7f800000u) == 0x7f800000u;
 }
 
+// Workgroups for the adapters' terms: 32 took up to 21% longer a call (16 tokens,
+// 3584 -> 3584/512/512 at rank 64), 128 from 3% less to 5% more.
 constexpr int kTermBlocks = 64;
-// Waves of a lowrank_split workgroup
-constexpr int split_waves(int nt, int rb) { return rb == 1 && nt % 2 == 1 ? 16 : 8; }
+// Waves of a lowrank_split workgroup.  16 where a workgroup has one tile: its
+// registers let all run at once, and with 8 a forward of 3584 inputs took 2-5%
+// longer (a backward of 896 inputs 6% less).
+constexpr int split_waves(int nt, int rb) { return rb == 1 && nt == 1 ? 16 : 8; }
 
 #if defined(__HIP_DEVICE_COMPILE__)
 // The k range [kb, ke) of one wave of lowrank_split_kernel, added into acc and,
 // the products of lower terms, into small (so that acc rounds once a step).
 // Steps of 32: lane (i, q) holds U[row i][k0 + 8q .. +7] and V[k0 + 8q ..
-// +7][16 jt + i].  Lengths are multiples of 4 (of 8 with WIDE), so each half
+// +7][j0 + 16 jt + i].  Lengths are multiples of 4 (of 8 with WIDE), so each half
 // of a lane's 8 is all in or all out; out of range V is zeroed, U clamped
 // (and, where a step goes the fp32 way, zeroed as well).
 template <typename IO, bool WIDE, int NT, int RB, bool VT>
 __device__ inline void split_accumulate(const IO* const (&u)[RB], const float* __restrict__ v0, int K,
-                                        int rank, int kb, int ke, f32x4 (&acc)[RB][NT],
+                                        int rank, int j0, int kb, int ke, f32x4 (&acc)[RB][NT],
                                         f32x4 (&small)[RB][NT]) {
   const int lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
   constexpr bool kF32 = sizeof(IO) == 4;
@@ -183,7 +188,7 @@ __device__ inline void split_accumulate(const IO* const (&u)[RB], const float* _
         for (int h = 0; h < 2; ++h) ur[s][b][h] = ld_raw4(u[b] + kc[h]);
 #pragma unroll
       for (int jt = 0; jt < NT; ++jt) {
-        const int jc = min(16 * jt + i, rank - 1);
+        const int jc = min(j0 + 16 * jt + i, rank - 1);
 #pragma unroll
         for (int e = 0; e < 8; e += VT ? 4 : 1) {
           const int kk = kc[e / 4] + e % 4;
@@ -264,7 +269,7 @@ __global__ __launch_bounds__(64 * split_waves(NT, RB)) void lowrank_split_kernel
   __shared__ float red[W * 16 * RB * kRow];
   const int P = term_pitch(rank);
   bool odd = false;
-  const int rows_blocks = a.n * a.slabs;
+  const int rows_blocks = a.groups * a.n * a.slabs;
   if ((int)blockIdx.x >= rows_blocks) {
     // the adapters' terms: four ranks of one feature a thread, its loads
     // together (tied, so that none sinks under the bounds tests below),
@@ -310,7 +315,8 @@ __global__ __launch_bounds__(64 * split_waves(NT, RB)) void lowrank_split_kernel
     if (threadIdx.x == 0) a.odd[(int)blockIdx.x - rows_blocks] = odd;
     return;
   }
-  const int z = (int)blockIdx.x / a.slabs, slab = (int)blockIdx.x % a.slabs;
+  const int slab = (int)blockIdx.x % a.slabs, z = (int)blockIdx.x / a.slabs % a.n;
+  const int j0 = 16 * NT * ((int)blockIdx.x / (a.slabs * a.n));  // the workgroup's ranks from j0
   const SplitJob& job = a.j[z];
   const int K = job.K;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -328,10 +334,10 @@ __global__ __launch_bounds__(64 * split_waves(NT, RB)) void lowrank_split_kernel
 #pragma unroll
     for (int jt = 0; jt < NT; ++jt) acc[b][jt] = small[b][jt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   if (job.vt)
-    split_accumulate<IO, WIDE, NT, RB, true>(u, job.v, K, rank, kb, ke, acc, small);
+    split_accumulate<IO, WIDE, NT, RB, true>(u, job.v, K, rank, j0, kb, ke, acc, small);
   else
-    split_accumulate<IO, WIDE, NT, RB, false>(u, job.v, K, rank, kb, ke, acc, small);
-  // D of (b, jt): lane (i, q), register c holds row 16 b + 4q + c, column 16 jt + i
+    split_accumulate<IO, WIDE, NT, RB, false>(u, job.v, K, rank, j0, kb, ke, acc, small);
+  // D of (b, jt): lane (i, q), register c holds row 16 b + 4q + c, column j0 + 16 jt + i
 #pragma unroll
   for (int b = 0; b < RB; ++b)
 #pragma unroll
@@ -341,11 +347,11 @@ __global__ __launch_bounds__(64 * split_waves(NT, RB)) void lowrank_split_kernel
         red[(wave * 16 * RB + 16 * b + 4 * q + c) * kRow + 16 * jt + i] = acc[b][jt][c] + small[b][jt][c];
   __syncthreads();
   for (int idx = threadIdx.x; idx < 16 * RB * 16 * NT; idx += 64 * W) {
-    const int r = idx / (16 * NT), j = idx % (16 * NT), t = t0 + r;
+    const int r = idx / (16 * NT), jl = idx % (16 * NT), j = j0 + jl, t = t0 + r;
     if (t >= T || j >= rank) continue;
     float sum = 0.0f;
 #pragma unroll
-    for (int w = 0; w < W; ++w) sum += red[(w * 16 * RB + r) * kRow + j];
+    for (int w = 0; w < W; ++w) sum += red[(w * 16 * RB + r) * kRow + jl];
     job.l[(long)t * rank + j] = sum;
     if (job.terms == nullptr) continue;
     bf16* row = static_cast<bf16*>(job.terms) + (long)t * P;
@@ -482,12 +488,27 @@ float* slot(const ProjLaunch& a, int z) { return a.lowrank + (long)z * a.T * a.r
 
 // Row blocks (of 16) per lowrank_split workgroup: V is read once per
 // workgroup, U once per job, so taller slabs save V's reads while the
-// launch still fills the CUs.
+// launch still fills half of the CUs.  Two blocks only from 256 slabs on took up to
+// 1.55 times as long a call where they start at 128 (2100 tokens), never at rank
+// 64 1.05-1.16 times; without four blocks bf16 forwards at rank 16 and 32 took
+// 1.03-1.15 times from 3000 tokens on.
 template <typename IO, bool WIDE>
 int split_row_blocks(int T, int jobs, int nt) {
   if (sizeof(IO) == 2 && WIDE && nt <= 2 && (T + 63) / 64 * jobs >= 128) return 4;
   if ((T + 31) / 32 * jobs >= 128) return 2;
   return 1;
+}
+
+// Rank tiles (of 16) per workgroup of a launch of `slabs` single-block slabs: as
+// few as leave one workgroup a CU.  A workgroup reads its V columns whole, so a
+// tile of its own costs only U again, and splits K over 16 waves.  Calls at rank
+// 64, all four tiles in one workgroup before: 16 x 3584 -> 3584 bf16 47.3 + 56.5 ->
+// 30.4 + 39.6 us, 512 tokens 54.7 + 77.3 -> 39.0 + 62.8.  Two or four workgroups a
+// CU allowed: up to 1.21 and 1.30 times as long.
+int rank_tiles(int slabs, int tiles) {
+  for (int nt : {1, 2})
+    if (slabs * ((tiles + nt - 1) / nt) <= 256) return nt;
+  return 4;
 }
 
 // Calls whose tensors the DMA of proj_gemm takes as they are: bf16, whole
@@ -545,15 +566,17 @@ hipError_t run_cols_any(const ProjLaunch& a, const RowsPlan& plan, hipStream_t s
 
 template <typename IO, bool WIDE>
 hipError_t launch_lowrank(const ProjLaunch& a, SplitCall& c, hipStream_t st) {
-  const int nt = (a.rank + 15) / 16, rb = split_row_blocks<IO, WIDE>(a.T, c.n, nt);
+  const int tiles = (a.rank + 15) / 16, rb = split_row_blocks<IO, WIDE>(a.T, c.n, tiles);
   c.slabs = (a.T + 16 * rb - 1) / (16 * rb);
-  const dim3 grid(c.n * c.slabs + kTermBlocks), block(64 * split_waves(nt, rb));
+  const int nt = rb == 1 ? rank_tiles(c.slabs * c.n, tiles) : tiles;
+  c.groups = (tiles + nt - 1) / nt;
+  const dim3 grid(c.groups * c.n * c.slabs + kTermBlocks), block(64 * split_waves(nt, rb));
   switch (8 * rb + nt) {
 #define GL_SPLIT(RB, NT)                                                                             \
   case 8 * RB + NT:                                                                                  \
     hipLaunchKernelGGL((lowrank_split_kernel<IO, WIDE, NT, RB>), grid, block, 0, st, c, a.T, a.rank); \
     break;
-    GL_SPLIT(1, 1) GL_SPLIT(1, 2) GL_SPLIT(1, 3) GL_SPLIT(1, 4)
+    GL_SPLIT(1, 1) GL_SPLIT(1, 2) GL_SPLIT(1, 4)
     GL_SPLIT(2, 1) GL_SPLIT(2, 2) GL_SPLIT(2, 3) GL_SPLIT(2, 4)
     default:
       if constexpr (sizeof(IO) == 2 && WIDE) {
@@ -652,7 +675,7 @@ hipError_t run_call(const ProjLaunch& a, bool backward, hipStream_t st) {
     else
       GL_CHECK((launch_lowrank<bf16, false>(a, c, st)));
     g.odd = a.odd;
-    g.n_odd = kTermBlocks + c.n * c.slabs;
+    g.n_odd = kTermBlocks + c.groups * c.n * c.slabs;
   }
   if (backward) GL_CHECK(run_cols_any(a, plan, st));
   GL_CHECK(whole ? launch_gemm(g, backward, st) : launch_gemm_split(g, backward, a.io_bf16, st));
@@ -672,7 +695,7 @@ ProjScratchNeed proj_scratch_need(const ProjLaunch& a, bool backward) {
   const RowsPlan plan = rows_plan(a, backward);
   if (plan.n == 0) return need;
   need.lowrank = (long)plan.n * a.T * a.rank;
-  need.odd = kTermBlocks + (long)plan.n * ((a.T + 15) / 16);
+  need.odd = kTermBlocks + (long)plan.n * ((a.T + 15) / 16) * ((a.rank + 15) / 16);
   if (whole_pieces(a, backward))
     for (int p = 0; p < a.n_proj; ++p)
       if (a.p[p].a != nullptr)

@@ -298,3 +298,12 @@ def test_non_finite_row_ends_stay_in_their_rows(engine, value):
         assert torch.equal(torch.isinf(got), torch.isinf(ref))
         ok = torch.isfinite(ref)
         _check(got[ok], ref[ok], terms[ok], n_in, "finite")
+
+
+# rank tiles over the workgroups of lowrank_split: one, two and four to a
+# workgroup, the last one partial or absent, forward and backward apart
+@pytest.mark.parametrize("dtype,n_in", [(torch.bfloat16, 264), (torch.bfloat16, 268), (torch.float32, 264)])
+@pytest.mark.parametrize("T,rank", [(37, 17), (37, 64), (1100, 40), (1100, 64), (1900, 33)])
+def test_rank_groups_match_float64(engines, dtype, n_in, T, rank):
+    print(f"[rank groups] {dtype} T={T} in={n_in} rank={rank}", flush=True)
+    _run_and_check(engines[dtype], *_problem(T, n_in, (136,), rank, dtype=dtype), rank)
