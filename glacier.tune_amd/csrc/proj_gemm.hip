@@ -883,10 +883,6 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_split_kernel(const GemmCa
 #endif
 }
 
-}  // namespace
-
-namespace {
-
 // Tile shapes (features x tokens), the times a stage of theirs was measured
 // to take, and their instances.  us per launch, forward / backward (rank 16):
 //   T, in -> outs                    256x256  128x128/2  128x128  128x64  64x64
@@ -956,10 +952,6 @@ hipError_t launch_gemm_shape(GemmCall a, bool nn, int shape, hipStream_t st) {
   hipLaunchKernelGGL(nn ? s.nn : s.nt, dim3(a.ftiles * ttiles), dim3(kGThreads), 0, st, a);
   return hipGetLastError();
 }
-
-}  // namespace
-
-namespace {
 
 template <typename IO, bool NN>
 hipError_t launch_split(GemmCall a, hipStream_t st) {

@@ -128,7 +128,8 @@ struct SplitCall {
   int n, nv, across;
   int slabs;   // row slabs of a job
   int groups;  // rank groups of a slab
-  int* odd;    // [kTermBlocks], then [groups][n][slabs]: a value without split terms among what that workgroup wrote
+  int* odd;    // [kTermBlocks], then [groups][n][slabs]: a value without split
+               // terms among what that workgroup wrote; null: no terms are written
 };
 
 // The six entries of a terms row for x: side 0 the adapters', side 1 (s L).
@@ -359,6 +360,7 @@ __global__ __launch_bounds__(64 * split_waves(NT, RB)) void lowrank_split_kernel
     if (j == 0)
       for (int e = 6 * rank; e < P; ++e) row[e] = (bf16)0.0f;
   }
+  if (a.odd == nullptr) return;
   odd = __syncthreads_or(odd);
   if (threadIdx.x == 0) a.odd[kTermBlocks + (int)blockIdx.x] = odd;
 #endif
@@ -460,7 +462,7 @@ __global__ __launch_bounds__(kLrThreads) void lowrank_cols_kernel(ColsJobs jobs,
 // where their results go (slot z of ProjLaunch::lowrank, [T][r] each).
 struct RowsPlan {
   RowsJobs jobs{};
-  int n = 0, kmax = 0;
+  int n = 0;
   int slot_l[kMaxProj], slot_dl[kMaxProj];  // -1: not computed
 };
 
@@ -473,12 +475,10 @@ RowsPlan rows_plan(const ProjLaunch& a, bool backward) {
     if (backward) {
       plan.slot_dl[p] = plan.n;
       plan.jobs.j[plan.n++] = RowsJob{s.dy, s.b, s.out, 1};
-      plan.kmax = std::max(plan.kmax, s.out);
     }
     if (!backward || s.grad_b != nullptr) {
       plan.slot_l[p] = plan.n;
       plan.jobs.j[plan.n++] = RowsJob{a.x, s.a, a.in, 0};
-      plan.kmax = std::max(plan.kmax, a.in);
     }
   }
   return plan;
@@ -511,15 +511,15 @@ int rank_tiles(int slabs, int tiles) {
   return 4;
 }
 
-// Calls whose tensors the DMA of proj_gemm takes as they are: bf16, whole
-// 16-byte pieces in every row, 16-byte aligned tensors.
-// every row of x and dY in whole 16-byte pieces
+// Every row of bf16 x and dY in whole 16-byte pieces.
 bool eights(const ProjLaunch& a) {
   bool ok = a.in % 8 == 0;
   for (int p = 0; p < a.n_proj; ++p) ok = ok && a.p[p].out % 8 == 0;
   return ok;
 }
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+// Calls whose tensors the DMA of proj_gemm takes as they are: bf16, whole
+// 16-byte pieces in every row, 16-byte aligned tensors.
 bool whole_pieces(const ProjLaunch& a, bool backward) {
   if (!a.io_bf16 || !eights(a) || !aligned16(a.x) || (backward && !aligned16(a.dx))) return false;
   for (int p = 0; p < a.n_proj; ++p)
@@ -570,7 +570,7 @@ hipError_t launch_lowrank(const ProjLaunch& a, SplitCall& c, hipStream_t st) {
   c.slabs = (a.T + 16 * rb - 1) / (16 * rb);
   const int nt = rb == 1 ? rank_tiles(c.slabs * c.n, tiles) : tiles;
   c.groups = (tiles + nt - 1) / nt;
-  const dim3 grid(c.groups * c.n * c.slabs + kTermBlocks), block(64 * split_waves(nt, rb));
+  const dim3 grid(c.groups * c.n * c.slabs + (c.nv > 0 ? kTermBlocks : 0)), block(64 * split_waves(nt, rb));
   switch (8 * rb + nt) {
 #define GL_SPLIT(RB, NT)                                                                             \
   case 8 * RB + NT:                                                                                  \
@@ -642,7 +642,7 @@ hipError_t run_call(const ProjLaunch& a, bool backward, hipStream_t st) {
     if (a.p[p].a != nullptr) lt += (long)P * (backward ? a.in : a.p[p].out);
   SplitCall c{};
   c.across = backward;
-  c.odd = a.odd;
+  c.odd = whole ? a.odd : nullptr;
   for (int p = 0; p < a.n_proj; ++p) {
     const ProjSpec& s = a.p[p];
     g.j[p] = GemmJob{backward ? nullptr : to[p], s.bias, nullptr, nullptr, s.scaling, s.out, 0};
@@ -674,8 +674,8 @@ hipError_t run_call(const ProjLaunch& a, bool backward, hipStream_t st) {
       GL_CHECK((launch_lowrank<bf16, true>(a, c, st)));
     else
       GL_CHECK((launch_lowrank<bf16, false>(a, c, st)));
-    g.odd = a.odd;
-    g.n_odd = kTermBlocks + c.groups * c.n * c.slabs;
+    g.odd = c.odd;
+    g.n_odd = whole ? kTermBlocks + c.groups * c.n * c.slabs : 0;
   }
   if (backward) GL_CHECK(run_cols_any(a, plan, st));
   GL_CHECK(whole ? launch_gemm(g, backward, st) : launch_gemm_split(g, backward, a.io_bf16, st));
@@ -695,11 +695,11 @@ ProjScratchNeed proj_scratch_need(const ProjLaunch& a, bool backward) {
   const RowsPlan plan = rows_plan(a, backward);
   if (plan.n == 0) return need;
   need.lowrank = (long)plan.n * a.T * a.rank;
+  if (!whole_pieces(a, backward)) return need;
   need.odd = kTermBlocks + (long)plan.n * ((a.T + 15) / 16) * ((a.rank + 15) / 16);
-  if (whole_pieces(a, backward))
-    for (int p = 0; p < a.n_proj; ++p)
-      if (a.p[p].a != nullptr)
-        need.terms += (long)term_pitch(a.rank) * (a.T + (backward ? a.in : a.p[p].out));
+  for (int p = 0; p < a.n_proj; ++p)
+    if (a.p[p].a != nullptr)
+      need.terms += (long)term_pitch(a.rank) * (a.T + (backward ? a.in : a.p[p].out));
   return need;
 }
 
