@@ -467,7 +467,9 @@ __global__ __launch_bounds__(kGThreads) void proj_gemm_kernel(const GemmCall a) 
 // Ends a run of products where control flow joins: 16 wait states, so that the
 // copies of accumulators that the compiler may place there read what the last
 // MFMA wrote.  (It leaves too few of its own before copies in a loop's header:
-// one instance lost its sums that way.)
+// built without this, the bf16 backward 64 x 64 instance copied one 5 wait states
+// behind a product that takes 12, and lost its sums.  The loops without it have no
+// such copies as built; tests/test_mfma_waits.py looks.)
 template <int FB, int TB>
 __device__ inline void settle(f32x16 (&acc)[FB][TB]) {
 #pragma unroll
