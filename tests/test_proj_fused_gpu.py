@@ -86,7 +86,9 @@ SHAPES = [  # T, in, outs, rank
     (640, 2056, (1032, 1032), 8),
     (1290, 520, (2056, 136), 33),
     (2051, 1024, (2048, 520, 264), 16),    # taller low-rank slabs
-    (4099, 256, (4104,), 12),              # the largest tiles, ragged in both directions
+    (4099, 256, (4104,), 12),              # 128 x 128 tiles, two to a CU, ragged in both directions
+    (2051, 4088, (4088,), 24),             # 256 x 256 tiles in both directions, ragged in both
+    (2051, 2040, (1032, 8), 40),           # 128 x 128 tiles two to a CU backward
 ]
 
 
@@ -95,8 +97,9 @@ OTHER_SHAPES = [  # the split-operand GEMM
     (torch.float32, 37, 100, (36, 72), 3),
     (torch.float32, 65, 1000, (1000, 200, 200), 20),
     (torch.float32, 130, 264, (516, 4), 64),
-    (torch.float32, 512, 3584, (3584, 512, 512), 16),  # the larger tiles
-    (torch.float32, 1025, 520, (2052,), 8),
+    (torch.float32, 512, 3584, (3584, 512, 512), 16),  # the larger tiles forward
+    (torch.float32, 1025, 520, (2052,), 8),            # the larger tiles, ragged: forward
+    (torch.float32, 1025, 2052, (520,), 8),            # and backward
     (torch.bfloat16, 37, 100, (36, 72), 3),            # rows of half 16-byte pieces
     (torch.bfloat16, 700, 1004, (3004, 12), 17),
 ]
@@ -273,9 +276,12 @@ def test_split_sums_are_as_exact_as_fp32_ones(engines, dtype, T, n_in, outs, ran
 
 # one term for bf16 operands of the general GEMM: rows of 4, rows that end 4
 # before a 16-byte piece, one row, the larger tiles in both directions
-@pytest.mark.parametrize("T,n_in,outs,rank", [
+ODD_WIDTHS = [  # T, in, outs, rank
     (1, 4, (4,), 1), (70, 12, (4, 36), 3), (33, 4, (12,), 2), (1, 12, (12, 8), 2),
-    (65, 268, (132, 8), 16), (1025, 2052, (2052,), 16)])
+    (65, 268, (132, 8), 16), (1025, 2052, (2052,), 16)]
+
+
+@pytest.mark.parametrize("T,n_in,outs,rank", ODD_WIDTHS)
 def test_odd_bf16_widths_match_float64(engine, T, n_in, outs, rank):
     print(f"[odd widths] T={T} in={n_in} outs={outs} rank={rank}", flush=True)
     _run_and_check(engine, *_problem(T, n_in, outs, rank), rank)
@@ -300,10 +306,40 @@ def test_non_finite_row_ends_stay_in_their_rows(engine, value):
         _check(got[ok], ref[ok], terms[ok], n_in, "finite")
 
 
-# rank tiles over the workgroups of lowrank_split: one, two and four to a
-# workgroup, the last one partial or absent, forward and backward apart
-@pytest.mark.parametrize("dtype,n_in", [(torch.bfloat16, 264), (torch.bfloat16, 268), (torch.float32, 264)])
-@pytest.mark.parametrize("T,rank", [(37, 17), (37, 64), (1100, 40), (1100, 64), (1900, 33)])
-def test_rank_groups_match_float64(engines, dtype, n_in, T, rank):
-    print(f"[rank groups] {dtype} T={T} in={n_in} rank={rank}", flush=True)
-    _run_and_check(engines[dtype], *_problem(T, n_in, (136,), rank, dtype=dtype), rank)
+# lowrank_split: rank tiles over its workgroups (one, two and four to a workgroup,
+# the last one partial or absent), then slabs of two and of four row blocks
+RANKS = [  # T, outs, rank
+    (37, (136,), 17), (37, (136,), 64), (1100, (136,), 40), (1100, (136,), 64), (1900, (136,), 33),
+    (1401, (136, 8, 72), 8), (1401, (136, 8, 72), 20), (1401, (136, 8, 72), 40), (1401, (136, 8, 72), 64),
+    (2107, (136, 8, 72), 16), (2107, (136, 8, 72), 20)]
+RANK_WIDTHS = [(torch.bfloat16, 264), (torch.bfloat16, 268), (torch.float32, 264)]
+
+
+@pytest.mark.parametrize("dtype,n_in", RANK_WIDTHS)
+@pytest.mark.parametrize("T,outs,rank", RANKS)
+def test_low_rank_shapes_match_float64(engines, dtype, n_in, T, outs, rank):
+    print(f"[low rank] {dtype} T={T} in={n_in} outs={outs} rank={rank}", flush=True)
+    _run_and_check(engines[dtype], *_problem(T, n_in, outs, rank, dtype=dtype), rank)
+
+
+@pytest.mark.parametrize("dtype,T,n_in,outs,where", [
+    (torch.bfloat16, 2051, 4088, (4088,), "b"), (torch.bfloat16, 2051, 2040, (1032,), "a"),
+    (torch.float32, 1025, 520, (2052,), "x"), (torch.float32, 1025, 2052, (520,), "dy")])
+def test_non_finite_values_in_large_tiles(engines, dtype, T, n_in, outs, where):
+    """As in the smallest tiles: the low-rank product of the whole call, or the
+    tile that holds the value, on fp32 products."""
+    print(f"[large non-finite] {dtype} T={T} in={n_in} outs={outs} {where}", flush=True)
+    rank = 8
+    x, projs = _problem(T, n_in, outs, rank, dtype=dtype)
+    p = projs[0]
+    place = {"x": x, "dy": p["dy"], "a": p["a"], "b": p["b"]}[where]
+    place[place.shape[0] - 2, place.shape[1] - 3] = float("inf")
+    ys, dx = engines[dtype].proj_forward(x, projs, rank), engines[dtype].proj_backward(x, projs, rank)
+    want, want_dx = _reference(x, projs)
+    for got, (ref, terms) in zip([*ys, dx], [*want, want_dx]):
+        ref32 = ref.float().to(dtype)
+        assert torch.equal(torch.isnan(got), torch.isnan(ref32))
+        assert torch.equal(torch.isinf(got), torch.isinf(ref32))
+        ok = torch.isfinite(ref32) & torch.isfinite(terms)
+        if ok.any():
+            _check(got[ok], ref[ok], terms[ok], max(n_in, outs[0]), where)
