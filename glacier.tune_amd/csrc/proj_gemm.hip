@@ -925,7 +925,8 @@ int tiles_of(const GemmCall& a, bool nn, const GemmShape& s) {
 
 // The shape with the least estimated time: rounds of the CUs times the time
 // of a stage, which grows with the share of the chip at work (the clock falls
-// under load).
+// under load).  One pair of times serves both directions: the order of the
+// shapes is what they have to tell, and the table's rows bear it out in both.
 int gemm_shape(const GemmCall& a, bool nn) {
   int best = 0;
   float best_t = 0.0f;

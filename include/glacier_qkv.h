@@ -55,7 +55,10 @@ typedef struct glacier_proj_desc {
   int32_t total_tokens;  /* T (may be 0) */
   int32_t in_features;   /* a multiple of 4 */
   int32_t rank;          /* 1..GLACIER_PROJ_MAX_RANK when any adapter is given */
-  int32_t precision;     /* GLACIER_ATTN_PREC_*: FP32 (fp32 GEMMs) or BF16 */
+  int32_t precision;     /* GLACIER_ATTN_PREC_*: FP32 (fp32 operands and sums; the
+                            products no further from exact ones than fp32
+                            products, small and non-finite values included)
+                            or BF16 */
   int32_t io_dtype;      /* GLACIER_ATTN_IO_*: F32, or BF16 with PREC_BF16 (bf16
                             GEMM operands, fp32 accumulation and adapters) */
 } glacier_proj_desc;
