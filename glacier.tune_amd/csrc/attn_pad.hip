@@ -46,11 +46,15 @@ template <typename T, int V, int N, bool PAD>
 __global__ __launch_bounds__(256) void pad_rows_kernel(const PadCall a, int d, int dp, int per_block,
                                                       unsigned inv) {
   typedef T Piece __attribute__((ext_vector_type(V)));
-  int z = 0;
-  while (z + 1 < a.n && (int)blockIdx.x >= a.j[z + 1].first) ++z;
+  // short calls (N 1): a tensor per row of a grid that its longest one fills;
+  // long ones: each tensor its own workgroups, one after another
+  int z = (int)blockIdx.y;
+  if constexpr (N > 1)
+    while (z + 1 < a.n && (int)blockIdx.x >= a.j[z + 1].first) ++z;
   const PadJob& job = a.j[z];
   const int width = PAD ? dp : d, pieces = width / V;
-  const long r0 = (long)((int)blockIdx.x - job.first) * per_block;
+  const long r0 = (long)((int)blockIdx.x - (N > 1 ? job.first : 0)) * per_block;
+  if (N == 1 && r0 >= job.rows) return;
   const int rows = static_cast<int>(min((long)per_block, job.rows - r0));
   const T* src = static_cast<const T*>(job.src) + r0 * (PAD ? d : dp);
   T* dst = static_cast<T*>(job.dst) + r0 * width;
@@ -85,25 +89,24 @@ hipError_t launch_pad(PadCall a, int d, int dp, hipStream_t st) {
   while (!whole(v)) v /= 2;
   const int pieces = (PAD ? dp : d) / v;
   const unsigned inv = ((1u << 20) + pieces - 1) / pieces;
-  int per_block = 0;
-  long blocks = 0;
-  auto split = [&](int n) {
-    per_block = 256 * n / pieces;
-    blocks = 0;
-    for (int i = 0; i < a.n; ++i) {
-      a.j[i].first = static_cast<int>(blocks);
-      blocks += (a.j[i].rows + per_block - 1) / per_block;
-    }
-  };
+  int per_block = 4 * 256 / pieces;
+  long blocks = 0, most = 0;
+  for (int i = 0; i < a.n; ++i) {
+    a.j[i].first = static_cast<int>(blocks);
+    blocks += (a.j[i].rows + per_block - 1) / per_block;
+    most = std::max(most, a.j[i].rows);
+  }
+  if (blocks == 0) return hipSuccess;
   // Bound by the launch on short calls, by the pieces on long ones.  Forward that
   // saves, then backward, bf16: 1500 tokens, 40/8 heads of 200: 168 + 534 us, where
   // one element a thread took 265 + 694 and a launch per tensor 223 + 647.  Four
   // pieces a thread once they give every CU two workgroups, one before (64
   // tokens, 14/2 heads of 80: 14.5 + 16.8 us, 15.4 + 17.6 with four).
-  split(4);
   const bool four = blocks >= 512;
-  if (!four) split(1);
-  if (blocks == 0) return hipSuccess;
+  if (!four) {
+    per_block = 256 / pieces;
+    blocks = (most + per_block - 1) / per_block;
+  }
   auto pick = [&](auto nc) {
     constexpr int N = decltype(nc)::value;
     if constexpr (sizeof(T) == 2)
@@ -111,7 +114,7 @@ hipError_t launch_pad(PadCall a, int d, int dp, hipStream_t st) {
     return v == 4 ? pad_rows_kernel<T, 4, N, PAD> : v == 2 ? pad_rows_kernel<T, 2, N, PAD> : pad_rows_kernel<T, 1, N, PAD>;
   };
   auto fn = four ? pick(std::integral_constant<int, 4>{}) : pick(std::integral_constant<int, 1>{});
-  hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, st, a, d, dp, per_block, inv);
+  hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(blocks), four ? 1 : a.n), dim3(256), 0, st, a, d, dp, per_block, inv);
   return hipGetLastError();
 }
 
